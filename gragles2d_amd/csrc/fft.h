@@ -83,13 +83,6 @@ __device__ __forceinline__ int fft_factors(int n, int* f) {
     return c;
 }
 
-// Orders the wave's LDS writes before its following reads (the line buffers are wave-private).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Forward (INV = false, w = exp(-2 pi i/n)) or inverse (unnormalised, w = exp(+2 pi i/n)) DFT of
 // the line in a, by one wave; b is the other buffer.  Returns the buffer holding the result.
 template <class T, bool INV>

@@ -7,9 +7,10 @@
 //   k_lists            comparison lists (computeSecondOrderNeighbours)
 //   k_conv_circulant   convolution of every live box (executeConvolution), one persistent
 //                      launch per bucket
-//   k_level            comparison, contour, motion check, new box, neighbours, volume and
-//                      redistancing (executeComparison .. executeRedistancing), fused, one
-//                      persistent launch per bucket
+//   k_compare, k_contour, k_alloc, k_redist
+//                      comparison, contour / motion check / new box / neighbours / volume, room for
+//                      the new boxes, redistancing (executeComparison .. executeRedistancing), one
+//                      launch per range of buckets (level_groups)
 // Each bucket's launches get the LDS its largest box needs.
 #include <hip/hip_runtime.h>
 
@@ -65,6 +66,9 @@ struct ggx_ctx {
     // arenas (field type erased)
     void* P[2] = {nullptr, nullptr};
     void* Tt = nullptr;
+    void* Cf = nullptr;            // compared fields, at the offsets of the step's input layout
+    unsigned long long* bits = nullptr;  // sign planes of the compared fields (level.h)
+    unsigned long long* gather_part = nullptr;  // running sums of the neighbour pixels compared
     uint32_t* I[2] = {nullptr, nullptr};
     int cur = 0;       // P[cur] holds phi of the current layout
     int icur = 0;      // I[icur] holds the IDLocal written by the previous step
@@ -98,7 +102,8 @@ struct ggx_ctx {
     long long updates_total = 0;
     int lds_per_cu = 163840;
     int static_conv[2] = {0, 0};   // static LDS bytes of k_conv_circulant<double/float>
-    int static_level[2] = {0, 0};  // static LDS bytes of k_level<double/float>
+    int static_contour = 0;        // static LDS bytes of k_contour (the largest of its forms)
+    int static_redist = 0;         // and of k_redist
     int static_dense[2] = {0, 0};  // static LDS bytes of k_conv_dense<double/float>
 
     // circulant kernels of every box side 1 .. kMaxBox
@@ -299,18 +304,19 @@ int raise_lds(ggx_ctx* ctx) {
     if (ctx->opt.lds_budget > 0) lim = std::min(lim, ctx->opt.lds_budget);
     // allow the dynamic-LDS kernels to use up to `lim`
     const void* fns[] = {(const void*)k_conv_circulant<double>, (const void*)k_conv_circulant<float>,
-                         (const void*)k_level<double, true, false, false>, (const void*)k_level<float, true, false, false>,
                          (const void*)k_conv_dense<double>, (const void*)k_conv_dense<float>,
                          (const void*)k_conv_fft<double, true>, (const void*)k_conv_fft<double, false>,
                          (const void*)k_conv_fft<float, true>, (const void*)k_conv_fft<float, false>,
-                         (const void*)k_level<double, false, false, false>, (const void*)k_level<float, false, false, false>,
-                         (const void*)k_level<double, true, true, false>, (const void*)k_level<float, true, true, false>,
-                         (const void*)k_level<double, false, true, false>, (const void*)k_level<float, false, true, false>,
-                         (const void*)k_level<double, true, false, true>, (const void*)k_level<float, true, false, true>,
-                         (const void*)k_level<double, false, false, true>, (const void*)k_level<float, false, false, true>,
-                         (const void*)k_level<double, true, true, true>, (const void*)k_level<float, true, true, true>,
-                         (const void*)k_level<double, false, true, true>, (const void*)k_level<float, false, true, true>,
-                         (const void*)k_conv_fft_batch<true>, (const void*)k_conv_fft_batch<false>};
+                         (const void*)k_conv_fft_batch<true>, (const void*)k_conv_fft_batch<false>,
+                         (const void*)k_contour<double, false, false, 64>, (const void*)k_contour<double, false, false, 256>,
+                         (const void*)k_contour<float, false, false, 64>, (const void*)k_contour<float, false, false, 256>,
+                         (const void*)k_contour<double, true, false, 64>, (const void*)k_contour<double, true, false, 256>,
+                         (const void*)k_contour<float, true, false, 64>, (const void*)k_contour<float, true, false, 256>,
+                         (const void*)k_contour<double, false, true, 256>, (const void*)k_contour<float, false, true, 256>,
+                         (const void*)k_contour<double, true, true, 256>, (const void*)k_contour<float, true, true, 256>,
+                         (const void*)k_redist<double, 64>, (const void*)k_redist<double, 128>, (const void*)k_redist<double, 256>,
+                         (const void*)k_redist<float, 64>, (const void*)k_redist<float, 128>, (const void*)k_redist<float, 256>};
+    constexpr int kFns = (int)(sizeof(fns) / sizeof(fns[0])), kContour0 = 10, kRedist0 = 22;
     for (const void* f : fns) {
         hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
         if (e != hipSuccess) {
@@ -320,13 +326,15 @@ int raise_lds(ggx_ctx* ctx) {
     }
     ctx->lds_max = lim;
     // static __shared__ bytes count against the same per-workgroup limit as the dynamic request
-    int* dst[] = {&ctx->static_conv[0], &ctx->static_conv[1], &ctx->static_level[0], &ctx->static_level[1],
-                  &ctx->static_dense[0], &ctx->static_dense[1], &ctx->static_fft[0][1], &ctx->static_fft[0][0],
-                  &ctx->static_fft[1][1], &ctx->static_fft[1][0]};
-    for (int k = 0; k < 10; ++k) {
+    int* dst[] = {&ctx->static_conv[0], &ctx->static_conv[1], &ctx->static_dense[0], &ctx->static_dense[1],
+                  &ctx->static_fft[0][1], &ctx->static_fft[0][0], &ctx->static_fft[1][1], &ctx->static_fft[1][0]};
+    for (int k = 0; k < kFns; ++k) {
         hipFuncAttributes fa;
         HIPCHK(hipFuncGetAttributes(&fa, fns[k]));
-        *dst[k] = (int)fa.sharedSizeBytes;
+        const int st = (int)fa.sharedSizeBytes;
+        if (k < 8) *dst[k] = st;
+        else if (k >= kRedist0) ctx->static_redist = std::max(ctx->static_redist, st);
+        else if (k >= kContour0) ctx->static_contour = std::max(ctx->static_contour, st);
     }
     {
         const void* af[] = {(const void*)k_aniso<double>, (const void*)k_aniso<float>};
@@ -346,10 +354,16 @@ void build_live(ggx_ctx* ctx) {
         if ((ctx->h_flags[g] & kPresent) && (ctx->h_flags[g] & kExists)) ctx->h_live.push_back(g);
 }
 
+// Contour points of a slot of bucket b.  A small network's buckets up to kMergeSide share one size.
+int slot_cap(const ggx_ctx* ctx, int b) { return contour_cap(ctx->edges[std::max(b, ctx->merge_bucket)]); }
+
 Buckets bucket_table(const ggx_ctx* ctx) {
     Buckets B;
     B.count = ctx->nbuckets;
-    for (int b = 0; b < kMaxBuckets; ++b) B.edge[b] = b < ctx->nbuckets ? ctx->edges[b] : 0;
+    for (int b = 0; b < kMaxBuckets; ++b) {
+        B.edge[b] = b < ctx->nbuckets ? ctx->edges[b] : 0;
+        B.cap[b] = b < ctx->nbuckets ? slot_cap(ctx, b) : 0;
+    }
     return B;
 }
 
@@ -385,24 +399,109 @@ int launch_aniso(ggx_ctx* ctx, hipStream_t st, const int* list, const int* count
     return GGX_OK;
 }
 
-// The fused level-set kernel of one bucket: compared field in LDS or in the arena, with or
-// without the anisotropic records (junctions, boundary properties).
-template <class T, bool COARSEN = false>
-void launch_level(const ggx_ctx* ctx, hipStream_t st, bool full, int grid, long long lds, const LevelArgs<T>& A) {
-    if (ctx->K.on) {
-        if (full) hipLaunchKernelGGL((k_level<T, true, true, COARSEN>), dim3(grid), dim3(256), (size_t)lds, st, A);
-        else hipLaunchKernelGGL((k_level<T, false, true, COARSEN>), dim3(grid), dim3(256), (size_t)lds, st, A);
-    } else {
-        if (full) hipLaunchKernelGGL((k_level<T, true, false, COARSEN>), dim3(grid), dim3(256), (size_t)lds, st, A);
-        else hipLaunchKernelGGL((k_level<T, false, false, COARSEN>), dim3(grid), dim3(256), (size_t)lds, st, A);
-    }
-}
-
 AnisoState aniso_state(const ggx_ctx* ctx) {
     AnisoState S;
     S.quat = ctx->quat; S.nb_e = ctx->nb_e; S.nb_m = ctx->nb_m; S.junc = ctx->junc; S.jcnt = ctx->jcnt;
     S.idl_org = ctx->idl_org;
     return S;
+}
+
+// The arguments every kernel of the level-set phase shares.
+template <class T>
+LevelArgs<T> level_args(const ggx_ctx* ctx) {
+    LevelArgs<T> A;
+    A.box = ctx->box; A.off = ctx->off; A.cmp_cnt = ctx->cmp_cnt; A.cmp = ctx->cmp;
+    A.tilde = (const T*)ctx->Tt; A.cfield = (T*)ctx->Cf; A.bits = ctx->bits; A.plane = plane_words(ctx->field_alloc);
+    A.idl_old = ctx->I[ctx->icur]; A.idl_new = ctx->I[ctx->icur ^ 1];
+    A.off_prev = ctx->off_prev; A.n_prev = ctx->nprev; A.out_field = (T*)ctx->P[ctx->cur ^ 1];
+    A.rec_s = nullptr; A.rec_win = nullptr; A.rec_area = nullptr;
+    ContourOut& O = A.O;
+    O.pts = ctx->pts; O.coff = ctx->coff; O.ccap = ctx->ccap; O.clen = ctx->clen;
+    O.volume = ctx->volume; O.perimeter = ctx->perimeter; O.energy = ctx->energy; O.meanda = ctx->meanda;
+    O.nb_cnt = ctx->nb_cnt; O.nb_id = ctx->nb_id; O.nb_len = ctx->nb_len;
+    O.box_next = ctx->box_next; O.off_next = ctx->off_next; O.flags = ctx->flags; O.err = ctx->errs;
+    O.tops = &ctx->sched->tops[0]; O.field_cap = ctx->field_cap; O.contour_cap = ctx->contour_cap;
+    A.G = grid_const(ctx); A.loop = &ctx->sched->loop_cur; A.analysis_timestep = ctx->s.analysis_timestep;
+    A.gather_part = ctx->gather_part; A.out_total = &ctx->sched->out_total;
+    A.contour_base = ctx->sched->contour_base;
+    A.K = ctx->K; A.AS = aniso_state(ctx);
+    return A;
+}
+
+// Buckets b0 .. b1 of the work lists as one launch's items.
+template <class T>
+void level_items(const ggx_ctx* ctx, LevelArgs<T>& A, int b0, int b1) {
+    A.it.lists = ctx->blists; A.it.total = ctx->sched->bucket_total; A.it.stride = ctx->nslots;
+    A.it.b0 = b0; A.it.b1 = b1;
+    A.cap = 0;
+    for (int b = 0; b < kMaxBuckets; ++b) A.it.cap[b] = b < ctx->nbuckets ? slot_cap(ctx, b) : 0;
+    for (int b = b0; b <= b1; ++b) A.cap = std::max(A.cap, A.it.cap[b]);
+    A.nb = ctx->edges[b1];
+}
+
+// The bucket ranges the level-set kernels are launched over.  Buckets up to side 64 each have a
+// launch sized for them, unless the network is small (one launch for all of them: there a launch
+// lasts as long as its slowest grain); the buckets up to 128 and those above share one each.
+std::vector<std::pair<int, int>> level_groups(const ggx_ctx* ctx) {
+    std::vector<std::pair<int, int>> R;
+    int b = 0;
+    if (ctx->merge_bucket >= 0) {
+        R.push_back({0, ctx->merge_bucket});
+        b = ctx->merge_bucket + 1;
+    }
+    while (b < ctx->nbuckets) {
+        const int lim = ctx->edges[b] <= 64 ? ctx->edges[b] : (ctx->edges[b] <= 128 ? 128 : kMaxBox);
+        int e = b;
+        while (e + 1 < ctx->nbuckets && ctx->edges[e + 1] <= lim) ++e;
+        R.push_back({b, e});
+        b = e + 1;
+    }
+    return R;
+}
+
+template <class T>
+int launch_compare(const ggx_ctx* ctx, hipStream_t st, LevelArgs<T>& A, int items, bool coarsen) {
+    A.blocks = ((A.nb + kRows - 1) / kRows) * ((A.nb + 63) / 64);
+    const long long wgs = ((long long)items * A.blocks + 3) / 4;
+    const int grid = (int)std::max<long long>(1, std::min<long long>(wgs, ctx->cu_count * 8));
+    if (coarsen) hipLaunchKernelGGL((k_compare<T, true>), dim3(grid), dim3(256), 0, st, A);
+    else hipLaunchKernelGGL((k_compare<T, false>), dim3(grid), dim3(256), 0, st, A);
+    return GGX_OK;
+}
+
+template <class T>
+int launch_contour(ggx_ctx* ctx, hipStream_t st, LevelArgs<T>& A, int items, bool coarsen) {
+    const bool wide = coarsen || A.nb > 64;
+    const long long lds = contour_layout(A.nb, A.cap, wide ? 256 : 64).total;
+    if (lds + ctx->static_contour + 256 > ctx->lds_max)
+        return fail(ctx, GGX_E_BOUNDS, "box too large for the contour kernel: side " + std::to_string(A.nb) + " needs " +
+                                           std::to_string(lds) + " of " + std::to_string(ctx->lds_max) + " LDS bytes");
+    const int grid = std::max(1, std::min(items, ctx->cu_count * 128));
+    const size_t l = (size_t)lds;
+    if (coarsen) {
+        if (ctx->K.on) hipLaunchKernelGGL((k_contour<T, true, true, 256>), dim3(grid), dim3(256), l, st, A);
+        else hipLaunchKernelGGL((k_contour<T, false, true, 256>), dim3(grid), dim3(256), l, st, A);
+    } else if (ctx->K.on) {
+        if (wide) hipLaunchKernelGGL((k_contour<T, true, false, 256>), dim3(grid), dim3(256), l, st, A);
+        else hipLaunchKernelGGL((k_contour<T, true, false, 64>), dim3(grid), dim3(64), l, st, A);
+    } else {
+        if (wide) hipLaunchKernelGGL((k_contour<T, false, false, 256>), dim3(grid), dim3(256), l, st, A);
+        else hipLaunchKernelGGL((k_contour<T, false, false, 64>), dim3(grid), dim3(64), l, st, A);
+    }
+    return GGX_OK;
+}
+
+template <class T>
+int launch_redist(const ggx_ctx* ctx, hipStream_t st, LevelArgs<T>& A, int items) {
+    const int room = ctx->lds_max - ctx->static_redist - 256;
+    A.tile = A.nb + kTileMargin;
+    if (A.tile > 256 || redist_lds<T>(A.tile) > room) A.tile = 0;
+    const size_t lds = (size_t)redist_lds<T>(A.tile);
+    const int grid = std::max(1, std::min(items, ctx->cu_count * 128));
+    if (A.tile > 128 || A.tile == 0) hipLaunchKernelGGL((k_redist<T, 256>), dim3(grid), dim3(256), lds, st, A);
+    else if (A.tile > 64) hipLaunchKernelGGL((k_redist<T, 128>), dim3(grid), dim3(128), lds, st, A);
+    else hipLaunchKernelGGL((k_redist<T, 64>), dim3(grid), dim3(64), lds, st, A);
+    return GGX_OK;
 }
 
 std::vector<hipEvent_t> take_events(ggx_ctx* ctx, int count) {
@@ -499,15 +598,10 @@ int snapshot_for_adjoint(ggx_ctx* ctx, hipStream_t st, const void* P, const uint
 template <class T>
 int launch_step(ggx_ctx* ctx, bool timed, bool record = false) {
     hipStream_t st = ctx->stream;
-    GridConst G = grid_const(ctx);
     const int NS = ctx->nslots;
     T* P = (T*)ctx->P[ctx->cur];
-    T* Pn = (T*)ctx->P[ctx->cur ^ 1];
     T* Tt = (T*)ctx->Tt;
     uint32_t* Iold = ctx->I[ctx->icur];
-    uint32_t* Inew = ctx->I[ctx->icur ^ 1];
-    const int ti = sizeof(T) == 8 ? 0 : 1;
-    const int level_max = ctx->lds_max - ctx->static_level[ti] - 256;
     const int cus = ctx->cu_count;
     Sched* S = ctx->sched;
     std::vector<hipEvent_t> ev;
@@ -562,47 +656,34 @@ int launch_step(ggx_ctx* ctx, bool timed, bool record = false) {
         }
     }
     if (timed) HIPCHK(hipEventRecord(ev[2], st));
-    // fused comparison / level set / redistancing, one persistent launch per bucket
-    ContourOut O;
-    O.pts = ctx->pts; O.coff = ctx->coff; O.ccap = ctx->ccap; O.clen = ctx->clen;
-    O.volume = ctx->volume; O.perimeter = ctx->perimeter; O.energy = ctx->energy; O.meanda = ctx->meanda;
-    O.nb_cnt = ctx->nb_cnt; O.nb_id = ctx->nb_id; O.nb_len = ctx->nb_len;
-    O.box_next = ctx->box_next; O.off_next = ctx->off_next; O.flags = ctx->flags; O.err = ctx->errs;
-    O.tops = &S->tops[0]; O.field_cap = ctx->field_cap; O.contour_cap = ctx->contour_cap;
-    // a small network: the buckets up to edges[merge] as one launch over all live grains (each
-    // takes the grains that fit its layout), every launch taking contour slots from the bump
-    // allocator (the contour arena of a small network is sized for that at load)
-    const int merge = ctx->merge_bucket;
-    for (int b = merge >= 0 ? merge : 0; b < ctx->nbuckets; ++b) {
-        int nb = ctx->edges[b];
-        LevelLayout full = level_layout<T>(nb, true), small = level_layout<T>(nb, false);
-        // FP64, isotropic: the compared field and output tile in LDS while that still leaves four
-        // workgroups per CU; below that, the layout with both in the arena and more workgroups per
-        // CU is faster (batch-100k: buckets 56-128 in the arena, k_level 12.25 -> 11.81 ms per
-        // step).  Measured slower for FP32 (10.99 -> 11.20 ms) and for the anisotropic kernel,
-        // whose four-wave register target leaves the arena layout no more workgroups.
-        const bool arena = sizeof(T) == 8 && !ctx->K.on && per_cu(ctx, full.total + ctx->static_level[ti]) < 4;
-        const bool use_full = full.total <= level_max && !arena;
-        long long lds = use_full ? full.total : small.total;
-        if (lds > level_max)
-            return fail(ctx, GGX_E_BOUNDS, "box too large for the level-set kernel: bucket " + std::to_string(nb) + " needs " + std::to_string(lds) + " of " + std::to_string(level_max) + " LDS bytes");
-        LevelArgs<T> A;
-        A.list = b == merge ? ctx->alist : ctx->blists + (size_t)b * NS;
-        A.count = b == merge ? &S->all_total : &S->bucket_total[b];
-        A.box = ctx->box; A.off = ctx->off; A.cmp_cnt = ctx->cmp_cnt; A.cmp = ctx->cmp;
-        A.tilde = Tt; A.cglobal = P; A.idl_old = Iold; A.idl_new = Inew;
-        A.off_prev = ctx->off_prev; A.n_prev = ctx->nprev; A.out_field = Pn;
-        A.rec_s = record ? (T*)ctx->rec.s : nullptr; A.rec_win = record ? ctx->rec.win : nullptr;
-        A.rec_area = record ? ctx->rec.area : nullptr;
-        A.O = O; A.G = G; A.loop = &S->loop_cur; A.analysis_timestep = ctx->s.analysis_timestep;
-        A.nb = nb; A.lds_bytes = (int)lds;
-        A.contour_base = merge >= 0 ? nullptr : S->contour_base; A.bucket = b; A.cursor = &S->cursor[b];
-        A.gather_total = &S->gather_total; A.out_total = &S->out_total;
-        A.K = ctx->K; A.AS = aniso_state(ctx);
-        int grid = cus * per_cu(ctx, lds + ctx->static_level[ti]);
-        if (!ctx->opt.persistent) grid = counts[b];
-        if (grid == 0) continue;
-        launch_level<T>(ctx, st, lds == full.total, grid, lds, A);
+    // comparison, contour, room for the new boxes, redistancing: per range of buckets
+    LevelArgs<T> A = level_args<T>(ctx);
+    A.rec_s = record ? (T*)ctx->rec.s : nullptr; A.rec_win = record ? ctx->rec.win : nullptr;
+    A.rec_area = record ? ctx->rec.area : nullptr;
+    const auto groups = level_groups(ctx);
+    int all = 0;
+    auto items = [&](const std::pair<int, int>& r) {  // grains of a launch: counted, or all the grains there are
+        if (ctx->opt.persistent) return NS - 1;
+        int c = 0;
+        for (int b = r.first; b <= r.second; ++b) c += counts[b];
+        return c;
+    };
+    for (int phase = 0; phase < 3; ++phase) {
+        for (const auto& r : groups) {
+            const int k = items(r);
+            if (k == 0) continue;
+            level_items(ctx, A, r.first, r.second);
+            int rc = GGX_OK;
+            if (phase == 0) rc = launch_compare<T>(ctx, st, A, k, false);
+            else if (phase == 1) { rc = launch_contour<T>(ctx, st, A, k, false); all += k; }
+            else rc = launch_redist<T>(ctx, st, A, k);
+            if (rc) return rc;
+        }
+        if (phase == 1) {
+            const int grid = std::max(1, std::min((std::min(all, NS - 1) + 255) / 256, cus * 8));
+            hipLaunchKernelGGL(k_alloc, dim3(grid), dim3(256), 0, st, (const int*)ctx->alist, (const int*)&S->all_total, A.O,
+                               &S->out_total);
+        }
     }
     if (timed) HIPCHK(hipEventRecord(ev[3], st));
     HIPCHK(hipGetLastError());
@@ -661,16 +742,11 @@ int finish(ggx_ctx* ctx) {
 template <class T>
 int launch_step_pergrain(ggx_ctx* ctx) {
     hipStream_t st = ctx->stream;
-    GridConst G = grid_const(ctx);
     const int NS = ctx->nslots;
     T* P = (T*)ctx->P[ctx->cur];
-    T* Pn = (T*)ctx->P[ctx->cur ^ 1];
     T* Tt = (T*)ctx->Tt;
     uint32_t* Iold = ctx->I[ctx->icur];
-    uint32_t* Inew = ctx->I[ctx->icur ^ 1];
     Sched* S = ctx->sched;
-    const int ti = sizeof(T) == 8 ? 0 : 1;
-    const int level_max = ctx->lds_max - ctx->static_level[ti] - 256;
     std::vector<hipEvent_t> ev = take_events(ctx, 5);
     // host view of the live grains and their boxes
     std::vector<int> f((size_t)NS);
@@ -705,31 +781,18 @@ int launch_step_pergrain(ggx_ctx* ctx) {
         }
     }
     HIPCHK(hipEventRecord(ev[2], st));
-    ContourOut O;
-    O.pts = ctx->pts; O.coff = ctx->coff; O.ccap = ctx->ccap; O.clen = ctx->clen;
-    O.volume = ctx->volume; O.perimeter = ctx->perimeter; O.energy = ctx->energy; O.meanda = ctx->meanda;
-    O.nb_cnt = ctx->nb_cnt; O.nb_id = ctx->nb_id; O.nb_len = ctx->nb_len;
-    O.box_next = ctx->box_next; O.off_next = ctx->off_next; O.flags = ctx->flags; O.err = ctx->errs;
-    O.tops = &S->tops[0]; O.field_cap = ctx->field_cap; O.contour_cap = ctx->contour_cap;
+    LevelArgs<T> A = level_args<T>(ctx);
+    A.contour_base = nullptr;  // contour slots from the bump allocator
     for (size_t i = 0; i < live.size(); ++i) {
-        int n = bx[live[i]].n;
-        LevelLayout full = level_layout<T>(n, true), small = level_layout<T>(n, false);
-        long long lds = full.total <= level_max ? full.total : small.total;
-        if (lds > level_max)
-            return fail(ctx, GGX_E_BOUNDS, "box too large for the level-set kernel: bucket " + std::to_string(n) + " needs " + std::to_string(lds) + " of " + std::to_string(level_max) + " LDS bytes");
-        LevelArgs<T> A;
-        A.list = ctx->pg_list + i;
-        A.count = ctx->pg_one + i;
-        A.box = ctx->box; A.off = ctx->off; A.cmp_cnt = ctx->cmp_cnt; A.cmp = ctx->cmp;
-        A.tilde = Tt; A.cglobal = P; A.idl_old = Iold; A.idl_new = Inew;
-        A.off_prev = ctx->off_prev; A.n_prev = ctx->nprev; A.out_field = Pn;
-        A.rec_s = nullptr; A.rec_win = nullptr; A.rec_area = nullptr;
-        A.O = O; A.G = G; A.loop = &S->loop_cur; A.analysis_timestep = ctx->s.analysis_timestep;
-        A.nb = n; A.lds_bytes = (int)lds;
-        A.contour_base = nullptr; A.bucket = 0; A.cursor = nullptr;
-        A.gather_total = &S->gather_total; A.out_total = &S->out_total;
-        A.K = ctx->K; A.AS = aniso_state(ctx);
-        launch_level<T>(ctx, st, lds == full.total, 1, lds, A);
+        A.it.lists = ctx->pg_list + i; A.it.total = ctx->pg_one + i; A.it.stride = 0; A.it.b0 = A.it.b1 = 0;
+        A.nb = bx[live[i]].n;
+        A.cap = A.it.cap[0] = contour_cap(A.nb);
+        int rc = launch_compare<T>(ctx, st, A, 1, false);
+        if (!rc) rc = launch_contour<T>(ctx, st, A, 1, false);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_alloc, dim3(1), dim3(256), 0, st, (const int*)(ctx->pg_list + i), (const int*)(ctx->pg_one + i),
+                           A.O, &S->out_total);
+        if ((rc = launch_redist<T>(ctx, st, A, 1))) return rc;
     }
     HIPCHK(hipEventRecord(ev[3], st));
     HIPCHK(hipGetLastError());
@@ -863,7 +926,7 @@ int coarsen(ggx_ctx* ctx, int present) {
         hs.bucket_total[b] = (int)bl[(size_t)b].size();
         hs.cursor[b] = 0;
         hs.contour_base[b] = cbase;
-        cbase += (long long)bl[(size_t)b].size() * (long long)contour_cap(ctx->edges[b]);
+        cbase += (long long)bl[(size_t)b].size() * (long long)slot_cap(ctx, b);
         if (!bl[(size_t)b].empty())
             HIPCHK(hipMemcpy(ctx->blists + (size_t)b * NS, bl[(size_t)b].data(), bl[(size_t)b].size() * sizeof(int),
                              hipMemcpyHostToDevice));
@@ -871,36 +934,18 @@ int coarsen(ggx_ctx* ctx, int present) {
     hs.tops[0] = (unsigned long long)total;  // the next step's input layout
     hs.tops[1] = 0ull;
     HIPCHK(hipMemcpy(S, &hs, sizeof(Sched), hipMemcpyHostToDevice));
-    const int ti = sizeof(T) == 8 ? 0 : 1;
-    const int level_max = ctx->lds_max - ctx->static_level[ti] - 256;
-    ContourOut O;
-    O.pts = ctx->pts; O.coff = ctx->coff; O.ccap = ctx->ccap; O.clen = ctx->clen;
-    O.volume = ctx->volume; O.perimeter = ctx->perimeter; O.energy = ctx->energy; O.meanda = ctx->meanda;
-    O.nb_cnt = ctx->nb_cnt; O.nb_id = ctx->nb_id; O.nb_len = ctx->nb_len;
-    O.box_next = ctx->box_next; O.off_next = ctx->off_next; O.flags = ctx->flags; O.err = ctx->errs;
-    O.tops = &S->tops[0]; O.field_cap = ctx->field_cap; O.contour_cap = ctx->contour_cap;
-    for (int b = 0; b < ctx->nbuckets; ++b) {
-        if (bl[(size_t)b].empty()) continue;
-        const int nbk = ctx->edges[b];
-        LevelLayout full = level_layout<T>(nbk, true), small = level_layout<T>(nbk, false);
-        long long lds = full.total <= level_max ? full.total : small.total;
-        if (lds > level_max) return fail(ctx, GGX_E_BOUNDS, "box too large for the level-set kernel");
-        LevelArgs<T> A;
-        A.list = ctx->blists + (size_t)b * NS;
-        A.count = &S->bucket_total[b];
-        A.box = ctx->box; A.off = ctx->off; A.cmp_cnt = ctx->sec_cnt; A.cmp = ctx->sec;  // the last step's lists
-        A.tilde = Tt; A.cglobal = (T*)ctx->P[ctx->cur];
-        A.idl_old = ctx->I[ctx->icur]; A.idl_new = ctx->I[ctx->icur ^ 1];
-        A.off_prev = ctx->off_prev; A.n_prev = ctx->nprev; A.out_field = (T*)ctx->P[ctx->cur ^ 1];
-        A.rec_s = nullptr; A.rec_win = nullptr; A.rec_area = nullptr;
-        A.O = O; A.G = grid_const(ctx); A.loop = &S->loop_cur; A.analysis_timestep = ctx->s.analysis_timestep;
-        A.nb = nbk; A.lds_bytes = (int)lds;
-        A.contour_base = S->contour_base; A.bucket = b; A.cursor = &S->cursor[b];
-        A.gather_total = &S->gather_total; A.out_total = &S->out_total;
-        A.K = ctx->K; A.AS = aniso_state(ctx);
-        const int grid = ctx->cu_count * per_cu(ctx, lds + ctx->static_level[ti]);
-        launch_level<T, true>(ctx, st, lds == full.total, grid, lds, A);
-    }
+    // the comparison writes IDLocal, then the contours are traced in (and may edit) the new fields
+    LevelArgs<T> A = level_args<T>(ctx);
+    A.cmp_cnt = ctx->sec_cnt; A.cmp = ctx->sec;  // the last step's lists
+    A.cfield = (T*)ctx->P[ctx->cur];
+    for (int phase = 0; phase < 2; ++phase)
+        for (const auto& r : level_groups(ctx)) {
+            int k = 0;
+            for (int b = r.first; b <= r.second; ++b) k += (int)bl[(size_t)b].size();
+            if (k == 0) continue;
+            level_items(ctx, A, r.first, r.second);
+            if ((rc = phase == 0 ? launch_compare<T>(ctx, st, A, k, true) : launch_contour<T>(ctx, st, A, k, true))) return rc;
+        }
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
     ctx->icur ^= 1;
@@ -1016,7 +1061,7 @@ extern "C" void ggx_destroy(ggx_ctx* ctx) {
     if (!ctx) return;
     (void)hipDeviceSynchronize();
     for (int k = 0; k < 2; ++k) { dfree(ctx->P[k]); dfree(ctx->I[k]); }
-    dfree(ctx->Tt); dfree(ctx->pts);
+    dfree(ctx->Tt); dfree(ctx->Cf); dfree(ctx->bits); dfree(ctx->gather_part); dfree(ctx->pts);
     dfree(ctx->box); dfree(ctx->box_next); dfree(ctx->off); dfree(ctx->off_next); dfree(ctx->off_prev);
     dfree(ctx->nprev); dfree(ctx->flags); dfree(ctx->errs); dfree(ctx->sec_cnt); dfree(ctx->sec);
     dfree(ctx->cmp_cnt); dfree(ctx->cmp); dfree(ctx->newbox); dfree(ctx->coff); dfree(ctx->ccap); dfree(ctx->clen);
@@ -1133,7 +1178,12 @@ extern "C" int ggx_load_network(ggx_ctx* ctx, const ggx_network* net) {
         HIPCHK(hipMemset(ctx->I[k], 0, (size_t)field_alloc * 4));
     }
     HIPCHK(hipMalloc(&p, (size_t)field_alloc * es)); ctx->Tt = p;
+    HIPCHK(hipMalloc(&p, (size_t)field_alloc * es)); ctx->Cf = p;
     int rc;
+    if ((rc = dalloc(ctx, ctx->bits, (size_t)(kPlanes * plane_words(field_alloc)))) ||
+        (rc = dalloc(ctx, ctx->gather_part, (size_t)kCountSlots * kCountStride)))
+        return rc;
+    HIPCHK(hipMemset(ctx->gather_part, 0, (size_t)kCountSlots * kCountStride * 8));
     if ((rc = dalloc(ctx, ctx->pts, (size_t)std::max(1LL, ctx->contour_cap)))) return rc;
     if ((rc = dalloc(ctx, ctx->box, NS)) || (rc = dalloc(ctx, ctx->box_next, NS)) || (rc = dalloc(ctx, ctx->off, NS)) ||
         (rc = dalloc(ctx, ctx->off_next, NS)) || (rc = dalloc(ctx, ctx->off_prev, NS)) || (rc = dalloc(ctx, ctx->nprev, NS)) ||
@@ -1871,12 +1921,15 @@ extern "C" int ggx_get_stats(ggx_ctx* ctx, ggx_stats* out) {
             ctx->ev_free.push_back(ev);
         }
         ctx->graph_events.clear();
+        unsigned long long part[kCountSlots * kCountStride], gathered = 0;
+        HIPCHK(hipMemcpy(part, ctx->gather_part, sizeof(part), hipMemcpyDeviceToHost));
+        for (int k = 0; k < kCountSlots; ++k) gathered += part[k * kCountStride];
         const Sched& H = *ctx->h_sched;
         ctx->st.grid_point_updates = (int64_t)H.updates_total;
         const int64_t S = ctx->esize;
         ctx->st.conv_bytes = 2 * S * (int64_t)H.updates_total;
         // comparison: own phi~ + neighbour gathers; IDLocal written on the box; phi' on the new box
-        ctx->st.algorithmic_bytes = ctx->st.conv_bytes + S * (int64_t)(H.updates_total + H.gather_total + H.out_total) +
+        ctx->st.algorithmic_bytes = ctx->st.conv_bytes + S * (int64_t)(H.updates_total + gathered + H.out_total) +
                                     4 * (int64_t)H.updates_total;
         ctx->st.live_grains = H.all_count;
         ctx->st.max_box = H.max_n;

@@ -39,6 +39,13 @@ __device__ __forceinline__ long long flat_index(int row, int col, int x0, int y0
     return ((long long)k < size) ? (long long)k : -1;
 }
 
+// Orders the wave's LDS writes before its following reads (the other waves are not waited for).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ------------------------------------------------------------------------------------------
 // Per-step scheduling, all on the device so that a step needs no host round trip.
 // Sched holds the counters of one step; k_reset clears them, k_prep deletes the grains that
@@ -70,13 +77,13 @@ struct Sched {
     unsigned long long in_top;       // field-arena elements used by the step's input layout
     unsigned long long updates_total;  // sum of n^2 over all steps (never reset)
     unsigned long long steps_total;
-    unsigned long long gather_total;   // sum over steps and grains of the neighbour pixels compared
     unsigned long long out_total;      // sum over steps and grains of the redistanced box areas
 };
 
 struct Buckets {
     int count;
     int edge[kMaxBuckets];           // bucket b holds edge[b-1] < n <= edge[b]
+    int cap[kMaxBuckets];            // contour points of a slot of bucket b
 };
 
 // Counters of a freshly loaded network: everything zero except the field-arena layout of the
@@ -117,7 +124,7 @@ __global__ void k_reset(Sched* __restrict__ S) {
 // After k_prep: the bucket sizes k_prep's atomics produced, read once with atomic loads and
 // written with plain stores for the kernels that follow (every workgroup of those reads them),
 // and each bucket's first contour slot: bucket b's grains take consecutive slots of
-// contour_cap(edge[b]) points after the lower buckets' slots (no per-grain allocation).
+// cap[b] points after the lower buckets' slots (no per-grain allocation).
 __global__ void k_tally(Sched* __restrict__ S, Buckets B) {
     const int t = threadIdx.x;
     if (t < kMaxBuckets) S->bucket_total[t] = t < B.count ? load_counter(&S->bucket_count[t]) : 0;
@@ -126,7 +133,7 @@ __global__ void k_tally(Sched* __restrict__ S, Buckets B) {
         long long base = 0;
         for (int b = 0; b < B.count; ++b) {
             S->contour_base[b] = base;
-            base += (long long)load_counter(&S->bucket_count[b]) * (long long)contour_cap(B.edge[b]);
+            base += (long long)load_counter(&S->bucket_count[b]) * (long long)B.cap[b];
         }
         S->tops[1] = (unsigned long long)base;
     }
