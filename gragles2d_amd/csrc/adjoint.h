@@ -201,10 +201,9 @@ __global__ void __launch_bounds__(256) k_adj_weight(AdjWeightArgs W) {
         }
         if (threadIdx.x < 16) s_grad[threadIdx.x] = 0.0;
         __syncthreads();
-        if (threadIdx.x == 0 && !s_bad) {
-            build_sectors(c, L, s_j, nj, s_jw, A.h, A.K.csr, A.K.isr, S);
-            if (S.err) s_bad = 1;
-        }
+        if (threadIdx.x < 64 && !s_bad) build_sectors(c, L, s_j, nj, s_jw, A.h, A.K.csr, A.K.isr, S);
+        __syncthreads();
+        if (threadIdx.x == 0 && !s_bad && S.err) s_bad = 1;
         __syncthreads();
         if (s_bad) continue;  // the forward step reported this grain (kErrAniso)
         const int ncons = S.ncons, ninterp = S.ninterp;

@@ -8,13 +8,13 @@
 //    box.cpp:1785-1823), the mobility models (LSbox::GBmobilityModel, box.cpp:1825-1865) and the
 //    projection of a point onto a contour (ExplicitGrainBoundary::projectToGrainBondary,
 //    grainBoundary.cpp:365-447);
-//  * k_aniso, the velocity corrector of LSbox::executeConvolution (box.cpp:428-510), run on the
-//    convolved fields of all grains before the comparison reads them: per grain the contour
-//    sectors of the previous contour (ExplicitGrainBoundary::buildBoundarySectors,
+//  * k_sectors and k_aniso, the velocity corrector of LSbox::executeConvolution (box.cpp:428-510),
+//    run on the convolved fields of all grains before the comparison reads them: per grain the
+//    contour sectors of the previous contour (ExplicitGrainBoundary::buildBoundarySectors,
 //    setPointsOnBoundary, grainBoundary.cpp:233-330,524-559; ContourSector, contourSector.cpp)
-//    with the junction weights (GrainJunction::getWeight, junction.cpp:23-192), then per pixel
-//    of IDLocal's window intersected with the box: out = in + (out - in) * weight where
-//    in > -delta, else -delta.
+//    with the junction weights (GrainJunction::getWeight, junction.cpp:23-192), laid out per
+//    contour segment; then per pixel of IDLocal's window intersected with the box:
+//    out = in + (out - in) * weight where in > -delta, else -delta.
 // All of it is FP64 whatever the field type, with contraction off so that every decision
 // (nearest vertex, sector bounds, floors) sees the rounding of a scalar CPU build.
 #pragma once
@@ -24,7 +24,7 @@ namespace ggx {
 
 constexpr int kJuncCap = 32;           // junctions recorded per grain (m_grainJunctions)
 constexpr int kSecCap = 2 * kJuncCap;  // interpolating sectors per grain (two per constant sector)
-constexpr int kAnisoContourLds = 3072; // contour points staged in LDS (longer contours are read in place)
+constexpr int kAnisoContourLds = 320;  // contour points staged in LDS (longer contours are read in place)
 
 struct AnisoConst {
     int on;              // 1: anisotropic network
@@ -150,48 +150,44 @@ __device__ __forceinline__ int nearest_vertex(const double2* c, int size, double
     return nearest;
 }
 
-// Contour points per box of the pruned nearest-vertex scan, and the LDS a staged contour of
-// `cap` points takes with its boxes (minx, maxx, miny, maxy per chunk).
-constexpr int kProjChunk = 16;
-__host__ __device__ constexpr long long aniso_lds_bytes(int cap) {
-    return (((long long)cap * 16 + 31) / 32) * 32 + (long long)((cap + kProjChunk - 1) / kProjChunk) * 32;
-}
-
-// nearest_vertex with the scan pruned by chunk boxes, the same vertex: a chunk is skipped when
-// the squared distance to its box exceeds the distance to an actual vertex (the first vertex of
-// the chunk whose box is nearest).  The box bound is computed with the same subtractions,
-// squares and sum as a vertex's distance, and rounding is monotone, so it never exceeds the
-// distance of a vertex in the chunk: a skipped chunk holds no vertex at the minimum.  The other
-// chunks are scanned in contour order with the strict comparison of the full scan.
-__device__ __forceinline__ int nearest_vertex_boxed(const double2* c, int size, const double4* bb, double px,
-                                                    double py) {
+// nearest_vertex for the 64 pixels of an 8 x 8 tile by one wave, the same vertex: the scan is cut to
+// the vertices that can be a pixel's nearest.  With vmin the vertex nearest to the tile's centre c,
+// a vertex v is nearer than vmin to some point of the tile only if
+//   |v - c|^2 - |vmin - c|^2 <= 7 (|vx - vminx| + |vy - vminy|)
+// (the half-plane nearer to v meets the square of half side 3.5), tested in float with a margin
+// above its rounding; the others are scanned in contour order with the strict comparison of the
+// full scan.  A contour point every 0.8 grid points leaves 20 to 25 of a contour's 110 vertices.
+// (tx, ty): the tile's first pixel; px, py: the lane's pixel.  All lanes of the wave call this.
+__device__ __forceinline__ int nearest_vertex_tile(const double2* c, int size, int tx, int ty, double px, double py) {
 #pragma clang fp contract(off)
-    const int nv = size - 1;
+    const int lane = (int)(threadIdx.x & 63), nv = size - 1;
     if (nv < 1) return -1;
-    const int nch = (nv + kProjChunk - 1) / kProjChunk;
-    auto lower = [&](const double4 b) {
-        const double dx = px < b.x ? b.x - px : (px > b.y ? px - b.y : 0.0);
-        const double dy = py < b.z ? b.z - py : (py > b.w ? py - b.w : 0.0);
-        return dx * dx + dy * dy;
-    };
-    int best = 0;
-    double best_lb = lower(bb[0]);
-    for (int i = 1; i < nch; ++i) {
-        const double lb = lower(bb[i]);
-        if (lb < best_lb) { best_lb = lb; best = i; }
+    const double cx = tx + 3.5, cy = ty + 3.5;
+    float dm = 3.0e38f, mx = 0.0f, my = 0.0f;
+    for (int k = lane; k < nv; k += 64) {
+        const double2 v = c[k];
+        const float dx = (float)(v.x - cx), dy = (float)(v.y - cy), d = dx * dx + dy * dy;
+        if (d < dm) { dm = d; mx = dx; my = dy; }
     }
-    double guess;
-    {
-        const double2 v = c[best * kProjChunk];
-        const double dx = px - v.x, dy = py - v.y;
-        guess = dx * dx + dy * dy;
-    }
+    float lo = dm;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) lo = fminf(lo, __shfl_xor(lo, d));
+    const int at = (int)__builtin_ctzll(__ballot(dm == lo));
+    mx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx), at));
+    my = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my), at));
     double minDist = 1000000.0;
     int nearest = -1;
-    for (int i = 0; i < nch; ++i) {
-        if (lower(bb[i]) > guess) continue;
-        const int hi = min(nv, (i + 1) * kProjChunk);
-        for (int k = i * kProjChunk; k < hi; k++) {
+    for (int c0 = 0; c0 < nv; c0 += 64) {
+        bool may = false;
+        if (c0 + lane < nv) {
+            const double2 v = c[c0 + lane];
+            const float dx = (float)(v.x - cx), dy = (float)(v.y - cy), d = dx * dx + dy * dy;
+            may = d - lo <= 7.0f * (fabsf(dx - mx) + fabsf(dy - my)) + (1e-5f * d + 0.01f);
+        }
+        unsigned long long todo = __ballot(may);
+        while (todo) {
+            const int k = c0 + (int)__builtin_ctzll(todo);
+            todo &= todo - 1ull;
             const double2 v = c[k];
             const double dx = px - v.x, dy = py - v.y;
             const double dist = dx * dx + dy * dy;
@@ -243,8 +239,24 @@ __device__ __forceinline__ int project_to_contour(const double2* c, int size, do
 }
 
 // ------------------------------------------------------------------------------------------
-// k_aniso: the velocity corrector, one workgroup per grain of a bucket (static items).
+// The velocity corrector.
 // ------------------------------------------------------------------------------------------
+
+// What k_sectors leaves per grain for the pixels: the weights of the constant sectors, and of the
+// interpolating sectors the length and the weight's polynomial in the relative arc length
+// (contourSector.cpp:211-271): quadratic between two constant sectors, else between two end weights.
+struct SectorRecord {
+    int ok;                       // 0: nothing to correct (or the grain reports an error)
+    int pad;
+    double cw[kJuncCap];
+    int kind[kSecCap];            // kLinear, kQuadratic, or kNoWeight where IDLocal has no value at an end
+    double len[kSecCap], a[kSecCap], b[kSecCap], c[kSecCap];
+};
+enum { kLinear = 0, kQuadratic = 1, kNoWeight = 2 };
+// Sector codes of a segment: constant sector, kInterp + interpolating sector, or a plain boundary point.
+enum { kInterp = kJuncCap, kPlain = 255 };
+static_assert(kInterp + kSecCap < kPlain, "sector codes");
+
 template <class T>
 struct AnisoArgs {
     const int* list;
@@ -268,10 +280,12 @@ struct AnisoArgs {
     AnisoConst K;
     const int* loop;
     double h, delta;
-    int ccap_lds;                 // contour points the dynamic LDS holds
+    unsigned char* seg_code;      // per contour point: the sector its segment lies in (k_sectors)
+    double* seg_arc;              // and, in an interpolating sector, the arc length from its right end
+    SectorRecord* sectors;        // per grain
 };
 
-// Sectors of one grain, built by lane 0 (ContourSector: left and right contour points, the
+// Sectors of one grain (ContourSector: left and right contour points, the
 // constant sectors' junctions, the interpolating sectors' bounding constant sectors, lengths).
 struct SectorSet {
     int ncons, ninterp, err;
@@ -379,129 +393,158 @@ __device__ bool junction_weight(const AnisoArgs<T>& A, int me, const Junc& J, do
 }
 
 // ExplicitGrainBoundary::buildBoundarySectors with setPointsOnBoundary and the interpolating
-// sector generators, on lane 0.  jw: the junction weights.  Sets S.err on a contour too short to
-// end the reference's length-bounded walks.
+// sector generators, by one wave (S in LDS): the walks along the contour, a chain of square roots
+// each, run one junction or constant sector per lane; only the merging of constant sectors, a few
+// comparisons per junction, is serial.  jw: the junction weights.  Sets S.err on a contour too short
+// to end the reference's length-bounded walks, or beyond the capacities.
 __device__ void build_sectors(const double2* c, int size, const Junc* J, int nj, const double* jw, double h,
                               double csr, double isr, SectorSet& S) {
 #pragma clang fp contract(off)
-    S.ncons = 0; S.ninterp = 0; S.err = 0;
+    const int lane = (int)(threadIdx.x & 63);
+    if (lane == 0) { S.ncons = 0; S.ninterp = 0; S.err = 0; }
+    wave_lds_sync();
     if (nj == 0) return;
-    if (size < 2) { S.err = 1; return; }
+    if (size < 2) {
+        if (lane == 0) S.err = 1;
+        wave_lds_sync();
+        return;
+    }
     const int P = size - 1;  // PERIODIC modulus (grainBoundary.cpp:27)
     auto per = [P](int x) { return (x + P) % P; };
-    const long long cap = 1LL << 24;
-    auto set_points = [&](int j, int* right, int* left) -> bool {
+    const int cap = 1 << 24;
+    bool bad = false;
+    if (lane < nj) {  // setPointsOnBoundary of junction `lane`; kept in il / ir until the merge is done
         double dist = 0;
-        int l = J[j].seg;
-        dist += scaled_len(c[per(l + 1)], c[l], 1 - J[j].lambda) * h;
+        int l = J[lane].seg, it = 0;
+        dist += scaled_len(c[per(l + 1)], c[l], 1 - J[lane].lambda) * h;
         l = per(l + 1);
-        long long it = 0;
-        while (dist < csr) {
+        while (dist < csr && !bad) {
             dist += seg_len(c[per(l + 1)], c[l]) * h;
             l = per(l + 1);
-            if (++it > cap) return false;
+            if (++it > cap) bad = true;
         }
         dist = 0;
-        int r = J[j].seg;
-        dist += scaled_len(c[per(r + 1)], c[r], J[j].lambda) * h;
+        int r = J[lane].seg;
+        dist += scaled_len(c[per(r + 1)], c[r], J[lane].lambda) * h;
         r = per(r);
-        while (dist < csr) {
+        it = 0;
+        while (dist < csr && !bad) {
             dist += seg_len(c[per(r - 1)], c[r]) * h;
             r = per(r - 1);
-            if (++it > cap) return false;
+            if (++it > cap) bad = true;
         }
-        *right = r;
-        *left = l;
-        return true;
-    };
-    int r0, l0;
-    if (!set_points(0, &r0, &l0)) { S.err = 1; return; }
-    S.cl[0] = l0; S.cr[0] = r0; S.cnj[0] = 1; S.cj[0][0] = 0;
-    S.ncons = 1;
-    int cur = 0;
-    for (int i = 1; i < nj; i++) {
-        int rr, ll;
-        if (!set_points(i, &rr, &ll)) { S.err = 1; return; }
-        if (sector_within(S.cr[cur], S.cl[cur], size, rr)) {
-            if (S.cnj[cur] >= kJuncCap) { S.err = 1; return; }
-            S.cj[cur][S.cnj[cur]++] = (unsigned char)i;
-            S.cl[cur] = ll;
-            if (i == nj - 1 && sector_within(S.cr[0], S.cl[0], size, S.cl[cur])) {
-                if (cur == 0) {
-                    S.cl[0] = -1;
-                    S.cr[0] = -1;
-                } else {
-                    const int m = S.cnj[cur];
-                    for (int q = 0; q < m; ++q) {
-                        if (S.cnj[0] >= kJuncCap) { S.err = 1; return; }
-                        S.cj[0][S.cnj[0]++] = S.cj[cur][q];
+        S.ir[lane] = r;
+        S.il[lane] = l;
+    }
+    if (__ballot(bad)) {
+        if (lane == 0) S.err = 1;
+        wave_lds_sync();
+        return;
+    }
+    wave_lds_sync();
+    if (lane == 0) {
+        int ncons = 1, cur = 0, err = 0;
+        S.cl[0] = S.il[0]; S.cr[0] = S.ir[0]; S.cnj[0] = 1; S.cj[0][0] = 0;
+        for (int i = 1; i < nj && !err; i++) {
+            const int rr = S.ir[i], ll = S.il[i];
+            if (sector_within(S.cr[cur], S.cl[cur], size, rr)) {
+                if (S.cnj[cur] >= kJuncCap) { err = 1; break; }
+                S.cj[cur][S.cnj[cur]++] = (unsigned char)i;
+                S.cl[cur] = ll;
+                if (i == nj - 1 && sector_within(S.cr[0], S.cl[0], size, S.cl[cur])) {
+                    if (cur == 0) {
+                        S.cl[0] = -1;
+                        S.cr[0] = -1;
+                    } else {
+                        const int m = S.cnj[cur];
+                        for (int q = 0; q < m; ++q) {
+                            if (S.cnj[0] >= kJuncCap) { err = 1; break; }
+                            S.cj[0][S.cnj[0]++] = S.cj[cur][q];
+                        }
+                        S.cr[0] = S.cr[cur];
                     }
-                    S.cr[0] = S.cr[cur];
                 }
-            }
-        } else if (i == nj - 1 && sector_within(S.cr[0], S.cl[0], size, ll)) {
-            if (S.cnj[0] >= kJuncCap) { S.err = 1; return; }
-            S.cr[0] = rr;
-            S.cj[0][S.cnj[0]++] = (unsigned char)i;
-        } else {
-            const int k = S.ncons++;
-            S.cl[k] = ll; S.cr[k] = rr; S.cnj[k] = 1; S.cj[k][0] = (unsigned char)i;
-            cur++;
-        }
-    }
-    const int sec_len = S.ncons;
-    if (S.ncons > 1 || S.cl[0] != S.cr[0]) {
-        for (int i = 0; i < S.ncons && S.ncons > 1; i++) {
-            const int sr = i, sl = (i + 1 + sec_len) % sec_len;
-            // generateLeftInterpolatingContour of sector sr (contourSector.cpp:108-127)
-            double dist = 0;
-            int j;
-            long long it = 0;
-            for (j = S.cl[sr]; dist <= isr; j = (j + 1 + P) % P) {
-                dist += seg_len(c[j], c[(j + 1 + P) % P]) * h;
-                if (++it > cap) { S.err = 1; return; }
-            }
-            const int nr_left = (j + 1 + P) % P, nr_right = S.cl[sr];
-            const double nr_len = dist;
-            // generateRightInterpolatingContour of sector sl (contourSector.cpp:149-169)
-            dist = 0;
-            for (j = S.cr[sl]; dist <= isr; j = (j - 1 + P) % P) {
-                dist += seg_len(c[j], c[(j - 1 + P) % P]) * h;
-                if (++it > cap) { S.err = 1; return; }
-            }
-            const int nl_left = S.cr[sl], nl_right = (j - 1 + P) % P;
-            const double nl_len = dist;
-            bool merged = false;
-            for (int q = nr_right; q != per(nr_left + 1); q = per(q + 1)) {
-                if (q == nl_left || q == nl_right) merged = true;
-                if (++it > cap) { S.err = 1; return; }
-            }
-            if (merged) {
-                // generateInterpolatingSector: this = sector sl, other = sector sr
-                if (S.ninterp >= kSecCap) { S.err = 1; return; }
-                const int k = S.ninterp++;
-                S.il[k] = S.cr[sl]; S.ils[k] = sl; S.ir[k] = S.cl[sr]; S.irs[k] = sr;
-                double d2 = 0;
-                for (int q = S.ir[k]; q != S.il[k]; q = (q + 1 + P) % P) {
-                    d2 += seg_len(c[q], c[(q - 1 + P) % P]) * h;
-                    if (++it > cap) { S.err = 1; return; }
-                }
-                S.ilen[k] = d2;
+            } else if (i == nj - 1 && sector_within(S.cr[0], S.cl[0], size, ll)) {
+                if (S.cnj[0] >= kJuncCap) { err = 1; break; }
+                S.cr[0] = rr;
+                S.cj[0][S.cnj[0]++] = (unsigned char)i;
             } else {
-                if (S.ninterp + 2 > kSecCap) { S.err = 1; return; }
-                int k = S.ninterp++;
-                S.il[k] = nr_left; S.ir[k] = nr_right; S.ils[k] = -1; S.irs[k] = sr; S.ilen[k] = nr_len;
-                k = S.ninterp++;
-                S.il[k] = nl_left; S.ir[k] = nl_right; S.ils[k] = sl; S.irs[k] = -1; S.ilen[k] = nl_len;
+                const int k = ncons++;
+                S.cl[k] = ll; S.cr[k] = rr; S.cnj[k] = 1; S.cj[k][0] = (unsigned char)i;
+                cur++;
             }
         }
+        S.ncons = ncons;
+        S.err = err;
     }
+    wave_lds_sync();
+    if (S.err) return;
+    const int ncons = S.ncons;
     // ContourSector::getWeight of a constant sector: the mean of its junctions' weights
-    for (int k = 0; k < S.ncons; ++k) {
+    if (lane < ncons) {
         double weight = 0;
-        for (int q = 0; q < S.cnj[k]; ++q) weight += jw[S.cj[k][q]];
-        S.cw[k] = weight / S.cnj[k];
+        for (int q = 0; q < S.cnj[lane]; ++q) weight += jw[S.cj[lane][q]];
+        S.cw[lane] = weight / S.cnj[lane];
     }
+    wave_lds_sync();
+    if (ncons < 2) return;
+    // between constant sector `lane` and the next one: their interpolating contours, one sector each,
+    // or one sector for both where the two contours meet
+    const int sr = lane, sl = (lane + 1 + ncons) % ncons;
+    int nr_left = 0, nr_right = 0, nl_left = 0, nl_right = 0;
+    double nr_len = 0, nl_len = 0, both_len = 0;
+    bool merged = false;
+    if (lane < ncons) {
+        // generateLeftInterpolatingContour of sector sr (contourSector.cpp:108-127)
+        double dist = 0;
+        int j, it = 0;
+        for (j = S.cl[sr]; dist <= isr && !bad; j = (j + 1 + P) % P) {
+            dist += seg_len(c[j], c[(j + 1 + P) % P]) * h;
+            if (++it > cap) bad = true;
+        }
+        nr_left = (j + 1 + P) % P;
+        nr_right = S.cl[sr];
+        nr_len = dist;
+        // generateRightInterpolatingContour of sector sl (contourSector.cpp:149-169)
+        dist = 0;
+        for (j = S.cr[sl]; dist <= isr && !bad; j = (j - 1 + P) % P) {
+            dist += seg_len(c[j], c[(j - 1 + P) % P]) * h;
+            if (++it > cap) bad = true;
+        }
+        nl_left = S.cr[sl];
+        nl_right = (j - 1 + P) % P;
+        nl_len = dist;
+        for (int q = nr_right; q != per(nr_left + 1) && !bad; q = per(q + 1)) {
+            if (q == nl_left || q == nl_right) merged = true;
+            if (++it > cap) bad = true;
+        }
+        if (merged)  // generateInterpolatingSector: this = sector sl, other = sector sr
+            for (int q = S.cl[sr]; q != S.cr[sl] && !bad; q = (q + 1 + P) % P) {
+                both_len += seg_len(c[q], c[(q - 1 + P) % P]) * h;
+                if (++it > cap) bad = true;
+            }
+    }
+    // places in the order of the constant sectors: one entry where merged, two else
+    const unsigned long long here = ncons < 64 ? (1ull << ncons) - 1ull : ~0ull, one = __ballot(merged) & here;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const int k = 2 * __popcll(here & below) - __popcll(one & below);
+    const int count = 2 * __popcll(here) - __popcll(one);
+    if (__ballot(bad) || count > kSecCap) {
+        if (lane == 0) S.err = 1;
+        wave_lds_sync();
+        return;
+    }
+    wave_lds_sync();  // il / ir served the merge until here
+    if (lane < ncons) {
+        if (merged) {
+            S.il[k] = S.cr[sl]; S.ils[k] = sl; S.ir[k] = S.cl[sr]; S.irs[k] = sr; S.ilen[k] = both_len;
+        } else {
+            S.il[k] = nr_left; S.ir[k] = nr_right; S.ils[k] = -1; S.irs[k] = sr; S.ilen[k] = nr_len;
+            S.il[k + 1] = nl_left; S.ir[k + 1] = nl_right; S.ils[k + 1] = sl; S.irs[k + 1] = -1; S.ilen[k + 1] = nl_len;
+        }
+    }
+    if (lane == 0) S.ninterp = count;
+    wave_lds_sync();
 }
 
 // LSbox::getGBEnergyTimesGBMobility(i, j) (box.cpp:544-554): IDLocal's neighbour at (i, j), its
@@ -528,151 +571,218 @@ __device__ __forceinline__ bool gb_weight_at(const AnisoArgs<T>& A, long long op
     return true;
 }
 
+// k_sectors: one wave per grain.  The sectors of the previous contour and, laid out for k_aniso,
+// the sector of every contour segment, the arc length before it and every sector's weight.  Bound
+// by the latency of the walks (square roots in a chain): a kernel of its own, so that the pixels'
+// waves do not hold their registers and LDS through it.  10000 grains: 0.13 ms.
 template <class T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_aniso(AnisoArgs<T> A) {
+__global__ void __launch_bounds__(64) k_sectors(AnisoArgs<T> A) {
 #pragma clang fp contract(off)
-    HIP_DYNAMIC_SHARED(unsigned char, smem)
-    double2* s_c = (double2*)smem;
-    double4* s_bb = (double4*)(smem + (((long long)A.ccap_lds * 16 + 31) / 32) * 32);
     __shared__ SectorSet S;
     __shared__ Junc s_j[kJuncCap];
     __shared__ double s_jw[kJuncCap];
     __shared__ int s_nid[kNbCap];
     __shared__ double s_nw[kNbCap];
-    __shared__ int s_bad;
+    __shared__ double2 s_c[kAnisoContourLds];
+    __shared__ unsigned char s_code[kAnisoContourLds];
     const int total = *A.count;
     const int loop = *A.loop;
+    const int lane = (int)threadIdx.x;
+    for (int item = blockIdx.x; item < total; item += gridDim.x) {
+        wave_lds_sync();  // the previous grain's shared state is free
+        const int g = A.list[item];
+        SectorRecord& R = A.sectors[g];
+        if (loop == 0 || !(A.flags[g] & kRegular)) {  // box.cpp:428-429
+            if (lane == 0) R.ok = 0;
+            continue;
+        }
+        const int L = A.clen[g];
+        const int nj = min(A.S.jcnt[g], kJuncCap);
+        const long long co = A.coff[g];
+        const double2* cg = A.pts + co;
+        const int nbc = A.nb_cnt[g];
+        const long long op = A.off_prev[g];
+        const int np = A.n_prev[g];
+        const int2 org = A.S.idl_org[g];
+        const bool staged = L <= kAnisoContourLds;
+        if (staged)
+            for (int k = lane; k < L; k += 64) s_c[k] = cg[k];
+        for (int k = lane; k < nbc; k += 64) {
+            s_nid[k] = A.nb_id[(size_t)g * kNbCap + k];
+            const double e = A.S.nb_e[(size_t)g * kNbCap + k], m = A.S.nb_m[(size_t)g * kNbCap + k];
+            s_nw[k] = (e * m > 0.01) ? e * m : 0.01;
+        }
+        bool bad = false;
+        if (lane < nj) {
+            s_j[lane] = A.S.junc[(size_t)g * kJuncCap + lane];
+            double w = 1.0;
+            if (!junction_weight(A, g, s_j[lane], &w)) bad = true;
+            s_jw[lane] = w;
+        }
+        wave_lds_sync();
+        // the contour in LDS when it fits; separate code, so that the walks read LDS and not through
+        // a generic pointer in the usual case
+        auto build = [&](const double2* c) -> bool {
+            build_sectors(c, L, s_j, nj, s_jw, A.h, A.K.csr, A.K.isr, S);
+            if (S.err) return false;
+            const int ncons = S.ncons, ninterp = S.ninterp, P = L - 1;
+            if (lane < ncons) R.cw[lane] = S.cw[lane];
+            if (lane < ninterp) {
+                // end weights: a constant sector's, or the boundary's at the end point
+                const int s = lane;
+                double left_w = 0, right_w = 0, bw = 0;
+                bool ok = true;
+                if (S.ils[s] >= 0) left_w = S.cw[S.ils[s]];
+                else ok = gb_weight_at(A, op, np, org.x, org.y, s_nid, s_nw, nbc, (int)c[S.il[s]].y, (int)c[S.il[s]].x, &left_w);
+                if (S.irs[s] >= 0) right_w = S.cw[S.irs[s]];
+                else ok = ok && gb_weight_at(A, op, np, org.x, org.y, s_nid, s_nw, nbc, (int)c[S.ir[s]].y, (int)c[S.ir[s]].x, &right_w);
+                const bool both = S.ils[s] >= 0 && S.irs[s] >= 0;
+                R.len[s] = S.ilen[s];
+                if (both) {
+                    const double2 sample = c[(S.ir[s] + 1) % P];
+                    ok = ok && gb_weight_at(A, op, np, org.x, org.y, s_nid, s_nw, nbc, (int)sample.y, (int)sample.x, &bw);
+                    const double two_isr = 2 * A.K.isr;
+                    const double quot = (S.ilen[s] > two_isr ? two_isr : S.ilen[s]);
+                    const double amplitude = (bw - (left_w + right_w) / 2) / (two_isr) * quot + (left_w + right_w) / 2;
+                    const double a0 = 2 * right_w, a1 = -4 * amplitude, a2 = 2 * left_w;
+                    R.a[s] = a0 + a1 + a2;
+                    R.b[s] = -(a0 * 1.5 + a1 + a2 * 0.5);
+                    R.c[s] = a0 * 0.5;
+                } else {
+                    R.a[s] = left_w;
+                    R.b[s] = right_w;
+                }
+                R.kind[s] = ok ? (both ? kQuadratic : kLinear) : kNoWeight;
+            }
+            for (int k = lane; k < P; k += 64) {
+                int code = kPlain;
+                for (int s = 0; s < ncons && code == kPlain; ++s)
+                    if (sector_within(S.cr[s], S.cl[s], L, k)) code = s;
+                for (int s = 0; s < ninterp && code == kPlain; ++s)
+                    if (sector_within(S.ir[s], S.il[s], L, k)) code = kInterp + s;
+                A.seg_code[co + k] = (unsigned char)code;
+                if (staged) s_code[k] = (unsigned char)code;
+            }
+            wave_lds_sync();
+            // arc length from an interpolating sector's right end to each of its segments, a sector per
+            // lane; a segment in two sectors keeps the first one's (the one its code names)
+            auto arcs = [&](int s, auto mine) {
+                double arc = 0;
+                int k = S.ir[s];
+                for (int it = 0; it < P; ++it) {
+                    if (mine(k)) A.seg_arc[co + k] = arc;
+                    if (k == S.il[s]) break;
+                    arc += seg_len(c[k + 1], c[k]) * A.h;
+                    k = (k + 1 + P) % P;
+                }
+            };
+            if (staged) {
+                if (lane < ninterp) arcs(lane, [&](int k) { return (int)s_code[k] == kInterp + lane; });
+            } else if (lane == 0) {
+                for (int s = ninterp - 1; s >= 0; --s) arcs(s, [](int) { return true; });
+            }
+            return true;
+        };
+        const bool ok = !__ballot(bad) && (staged ? build(s_c) : build(cg));
+        if (lane == 0) {
+            R.ok = ok ? 1 : 0;
+            if (!ok) A.err[g] = kErrAniso;
+        }
+    }
+}
+
+// k_aniso: the corrected field.  One workgroup per grain, a wave per 8 x 8 tile of pixels (the tile
+// keeps the pixels' candidate vertices few); contour, segment codes and arc lengths in LDS.  Bound
+// by the vertex scan and the two projections (FP64 VALU).  10000 grains: 0.38 ms, with k_sectors
+// 0.51 ms, where one kernel with a lane-0 sector build, chunk boxes per pixel and a walk to each
+// pixel's segment took 2.5 to 3.0 ms.
+template <class T>
+__global__ void __launch_bounds__(256) k_aniso(AnisoArgs<T> A) {
+#pragma clang fp contract(off)
+    __shared__ double2 s_c[kAnisoContourLds];
+    __shared__ double s_arc[kAnisoContourLds];
+    __shared__ unsigned char s_code[kAnisoContourLds];
+    __shared__ int s_nid[kNbCap];
+    __shared__ double s_nw[kNbCap];
+    const int total = *A.count;
+    const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6), nw = (int)(blockDim.x >> 6);
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
         __syncthreads();  // the previous grain's shared state is free
         const int g = A.list[item];
-        if (loop == 0 || !(A.flags[g] & kRegular)) continue;  // box.cpp:428-429
+        const SectorRecord& R = A.sectors[g];
+        if (!R.ok) continue;
         const int L = A.clen[g];
-        const int nj = min(A.S.jcnt[g], kJuncCap);
-        // the contour in LDS when it fits; the two paths below are separate code, so that the
-        // projection loop reads LDS (not through a generic pointer) in the usual case
-        const bool staged = L <= A.ccap_lds;
-        const double2* cg = A.pts + A.coff[g];
-        if (staged) {
-            for (int k = threadIdx.x; k < L; k += blockDim.x) s_c[k] = cg[k];
-            // boxes of the chunks of the nearest-vertex scan, from the global copy
-            const int nch = (L - 1 + kProjChunk - 1) / kProjChunk;
-            for (int i = threadIdx.x; i < nch; i += blockDim.x) {
-                const int lo = i * kProjChunk, hi = min(L - 1, lo + kProjChunk);
-                double4 bx = make_double4(cg[lo].x, cg[lo].x, cg[lo].y, cg[lo].y);
-                for (int k = lo + 1; k < hi; ++k) {
-                    const double2 v = cg[k];
-                    bx.x = fmin(bx.x, v.x); bx.y = fmax(bx.y, v.x);
-                    bx.z = fmin(bx.z, v.y); bx.w = fmax(bx.w, v.y);
-                }
-                s_bb[i] = bx;
+        const long long co = A.coff[g];
+        const bool staged = L <= kAnisoContourLds;
+        if (staged)
+            for (int k = threadIdx.x; k < L; k += blockDim.x) {
+                s_c[k] = A.pts[co + k];
+                s_arc[k] = A.seg_arc[co + k];
+                s_code[k] = A.seg_code[co + k];
             }
-        }
         const int nbc = A.nb_cnt[g];
         for (int k = threadIdx.x; k < nbc; k += blockDim.x) {
             s_nid[k] = A.nb_id[(size_t)g * kNbCap + k];
             const double e = A.S.nb_e[(size_t)g * kNbCap + k], m = A.S.nb_m[(size_t)g * kNbCap + k];
             s_nw[k] = (e * m > 0.01) ? e * m : 0.01;
         }
-        if (threadIdx.x == 0) s_bad = 0;
+        // pixels: IDLocal's window (previous step) intersected with the box (box.cpp:452-470)
+        const Box b = A.box[g];
+        const long long o = A.off[g];
+        const int np = A.n_prev[g];
+        const long long op = A.off_prev[g];
+        const int2 org = A.S.idl_org[g];
+        const int ix0 = max(org.x, b.x0), ix1 = min(org.x + np, b.x0 + b.n);
+        const int iy0 = max(org.y, b.y0), iy1 = min(org.y + np, b.y0 + b.n);
         __syncthreads();
-        auto process = [&](const double2* c, const double4* bb) {
-            for (int k = threadIdx.x; k < nj; k += blockDim.x) {
-                s_j[k] = A.S.junc[(size_t)g * kJuncCap + k];
-                double w = 1.0;
-                if (!junction_weight(A, g, s_j[k], &w)) s_bad = 1;
-                s_jw[k] = w;
-            }
-            __syncthreads();
-            if (threadIdx.x == 0 && !s_bad) {
-                build_sectors(c, L, s_j, nj, s_jw, A.h, A.K.csr, A.K.isr, S);
-                if (S.err) s_bad = 1;
-            }
-            __syncthreads();
-            if (s_bad) {
-                if (threadIdx.x == 0) A.err[g] = kErrAniso;
-                return;
-            }
-            // pixels: IDLocal's window (previous step) intersected with the box (box.cpp:452-470)
-            const Box b = A.box[g];
-            const long long o = A.off[g];
-            const int np = A.n_prev[g];
-            const long long op = A.off_prev[g];
-            const int2 org = A.S.idl_org[g];
-            const int ix0 = max(org.x, b.x0), ix1 = min(org.x + np, b.x0 + b.n);
-            const int iy0 = max(org.y, b.y0), iy1 = min(org.y + np, b.y0 + b.n);
-            const int wx = ix1 - ix0, wy = iy1 - iy0;
-            bool bad = false;
-            if (wx > 0 && wy > 0) {
-                const int ncons = S.ncons, ninterp = S.ninterp;
-                for (int p = threadIdx.x; p < wx * wy; p += blockDim.x) {
-                    const int i = iy0 + p / wx, j = ix0 + p % wx;
-                    const long long q = o + (long long)(i - b.y0) * b.n + (j - b.x0);
-                    const double val = (double)A.phi[q];
-                    if (!(val > -A.delta)) { A.tilde[q] = (T)(-A.delta); continue; }
-                    // ExplicitGrainBoundary::getWeight (grainBoundary.cpp:344-363)
-                    double lambda = 0, weight = 0;
-                    const int nearest = bb ? nearest_vertex_boxed(c, L, bb, (double)j, (double)i)
-                                           : nearest_vertex(c, L, (double)j, (double)i);
-                    const int segment = segment_at(c, L, nearest, (double)j, (double)i, &lambda);
-                    if (segment < 0) { bad = true; continue; }
-                    int found = -1;
-                    for (int s = 0; s < ncons && found < 0; ++s)
-                        if (sector_within(S.cr[s], S.cl[s], L, segment)) found = s;
-                    if (found >= 0) {
-                        weight = S.cw[found];
+        if (ix0 >= ix1 || iy0 >= iy1) continue;
+        const int tw = (ix1 - ix0 + 7) >> 3, th = (iy1 - iy0 + 7) >> 3;
+        auto process = [&](const double2* c, const unsigned char* code_of, const double* arc_of) {
+            for (int tile = wave; tile < tw * th; tile += nw) {
+                const int ty = iy0 + (tile / tw) * 8, tx = ix0 + (tile % tw) * 8;
+                const int i = ty + (lane >> 3), j = tx + (lane & 7);
+                const bool on = i < iy1 && j < ix1;
+                const long long q = o + (long long)(i - b.y0) * b.n + (j - b.x0);
+                const double val = on ? (double)A.phi[q] : -A.delta;
+                const bool act = on && val > -A.delta;
+                if (on && !act) A.tilde[q] = (T)(-A.delta);
+                if (!__ballot(act)) continue;
+                // ExplicitGrainBoundary::getWeight (grainBoundary.cpp:344-363)
+                const int nearest = nearest_vertex_tile(c, L, tx, ty, (double)j, (double)i);
+                if (!act) continue;
+                double lambda = 0, weight = 0;
+                const int segment = segment_at(c, L, nearest, (double)j, (double)i, &lambda);
+                bool ok = segment >= 0;
+                if (ok) {
+                    const int code = code_of[segment];
+                    if (code < kInterp) {
+                        weight = R.cw[code];
+                    } else if (code == kPlain) {
+                        ok = gb_weight_at(A, op, np, org.x, org.y, s_nid, s_nw, nbc, i, j, &weight);
                     } else {
-                        for (int s = 0; s < ninterp && found < 0; ++s)
-                            if (sector_within(S.ir[s], S.il[s], L, segment)) found = s;
-                        if (found < 0) {
-                            if (!gb_weight_at(A, op, np, org.x, org.y, s_nid, s_nw, nbc, i, j, &weight)) { bad = true; continue; }
-                        } else {
-                            // ContourSector::getWeight of an interpolating sector (contourSector.cpp:211-271)
-                            const int s = found, rcs = L - 1;
-                            double left_w, right_w;
-                            if (S.ils[s] >= 0) left_w = S.cw[S.ils[s]];
-                            else if (!gb_weight_at(A, op, np, org.x, org.y, s_nid, s_nw, nbc, (int)c[S.il[s]].y,
-                                                   (int)c[S.il[s]].x, &left_w)) { bad = true; continue; }
-                            if (S.irs[s] >= 0) right_w = S.cw[S.irs[s]];
-                            else if (!gb_weight_at(A, op, np, org.x, org.y, s_nid, s_nw, nbc, (int)c[S.ir[s]].y,
-                                                   (int)c[S.ir[s]].x, &right_w)) { bad = true; continue; }
-                            double interpolator = 0;
-                            int k = S.ir[s];
-                            for (; k != segment; k = (k + 1 + rcs) % rcs) interpolator += seg_len(c[k + 1], c[k]) * A.h;
-                            interpolator += scaled_len(c[(k + 1 + rcs) % rcs], c[k], lambda);
-                            interpolator /= S.ilen[s];
-                            if (interpolator < 0) interpolator = 0;
-                            if (interpolator > 1) interpolator = 1;
-                            if (S.ils[s] >= 0 && S.irs[s] >= 0) {
-                                const double2 sample = c[(S.ir[s] + 1) % rcs];
-                                double bw;
-                                if (!gb_weight_at(A, op, np, org.x, org.y, s_nid, s_nw, nbc, (int)sample.y, (int)sample.x, &bw)) {
-                                    bad = true;
-                                    continue;
-                                }
-                                const double two_isr = 2 * A.K.isr;
-                                const double quot = (S.ilen[s] > two_isr ? two_isr : S.ilen[s]);
-                                const double amplitude = (bw - (left_w + right_w) / 2) / (two_isr) * quot + (left_w + right_w) / 2;
-                                const double a0 = 2 * right_w, a1 = -4 * amplitude, a2 = 2 * left_w;
-                                const double Aq = a0 + a1 + a2;
-                                const double Bq = -(a0 * 1.5 + a1 + a2 * 0.5);
-                                const double Cq = a0 * 0.5;
-                                weight = Aq * interpolator * interpolator + Bq * interpolator + Cq;
-                            } else {
-                                weight = interpolator * left_w + (1 - interpolator) * right_w;
-                            }
-                        }
+                        // ContourSector::getWeight of an interpolating sector (contourSector.cpp:211-271)
+                        const int s = code - kInterp, rcs = L - 1, kind = R.kind[s];
+                        double t = arc_of[segment];
+                        t += scaled_len(c[(segment + 1 + rcs) % rcs], c[segment], lambda);
+                        t /= R.len[s];
+                        if (t < 0) t = 0;
+                        if (t > 1) t = 1;
+                        if (kind == kQuadratic) weight = R.a[s] * t * t + R.b[s] * t + R.c[s];
+                        else if (kind == kLinear) weight = t * R.a[s] + (1 - t) * R.b[s];
+                        else ok = false;
                     }
-                    const double radiuscorrection = 1.0;  // box.cpp:501
-                    const double t = (double)A.tilde[q];
-                    A.tilde[q] = (T)(val + (t - val) * weight * radiuscorrection);
                 }
+                if (!ok) {
+                    A.err[g] = kErrAniso;
+                    continue;
+                }
+                const double radiuscorrection = 1.0;  // box.cpp:501
+                const double t = (double)A.tilde[q];
+                A.tilde[q] = (T)(val + (t - val) * weight * radiuscorrection);
             }
-            if (bad) s_bad = 1;
-            __syncthreads();
-            if (threadIdx.x == 0 && s_bad) A.err[g] = kErrAniso;
         };
-        if (staged) process(s_c, s_bb);
-        else process(cg, nullptr);
+        if (staged) process(s_c, s_code, s_arc);
+        else process(A.pts + co, A.seg_code + co, A.seg_arc + co);
     }
 }
 

@@ -123,7 +123,9 @@ struct ggx_ctx {
     Junc* junc = nullptr;
     int* jcnt = nullptr;
     int2* idl_org = nullptr;
-    int static_aniso[2] = {0, 0};  // static LDS bytes of k_aniso<double/float>
+    unsigned char* seg_code = nullptr;  // k_sectors' output for k_aniso, per contour point ...
+    double* seg_arc = nullptr;
+    SectorRecord* sectors = nullptr;    // ... and per grain
     // grid coarsening: grainhdl::ngrains (the grain count at the last coarsening) and the number of
     // coarsenings so far
     int ngrains = 0;
@@ -336,14 +338,6 @@ int raise_lds(ggx_ctx* ctx) {
         else if (k >= kRedist0) ctx->static_redist = std::max(ctx->static_redist, st);
         else if (k >= kContour0) ctx->static_contour = std::max(ctx->static_contour, st);
     }
-    {
-        const void* af[] = {(const void*)k_aniso<double>, (const void*)k_aniso<float>};
-        for (int k = 0; k < 2; ++k) {
-            hipFuncAttributes fa;
-            HIPCHK(hipFuncGetAttributes(&fa, af[k]));
-            ctx->static_aniso[k] = (int)fa.sharedSizeBytes;
-        }
-    }
     return GGX_OK;
 }
 
@@ -372,12 +366,11 @@ int per_cu(const ggx_ctx* ctx, long long lds) {
     return (int)std::max<long long>(1, std::min<long long>(8, k));
 }
 
-// The velocity corrector of anisotropic networks on the convolved fields of one bucket's grains
-// (static items, one workgroup per grain), with the previous step's contours staged in LDS.
+// The velocity corrector of anisotropic networks on the convolved fields of a list's grains (items:
+// how many at most), before any comparison reads them.
 template <class T>
-int launch_aniso(ggx_ctx* ctx, hipStream_t st, const int* list, const int* count, int nb, int grid, const T* P, T* Tt,
-                 const uint32_t* Iold) {
-    const int ti = sizeof(T) == 8 ? 0 : 1;
+void launch_aniso(ggx_ctx* ctx, hipStream_t st, const int* list, const int* count, int items, const T* P, T* Tt,
+                  const uint32_t* Iold) {
     AnisoArgs<T> A;
     A.list = list; A.count = count; A.box = ctx->box; A.off = ctx->off;
     A.phi = P; A.tilde = Tt; A.idl = Iold; A.off_prev = ctx->off_prev; A.n_prev = ctx->nprev;
@@ -389,14 +382,10 @@ int launch_aniso(ggx_ctx* ctx, hipStream_t st, const int* list, const int* count
     A.loop = &ctx->sched->loop_cur;
     A.h = ctx->d.h;
     A.delta = ctx->d.delta;
-    const long long budget = ctx->lds_max - ctx->static_aniso[ti] - 256;
-    int cap = std::min(contour_cap(nb + 16), kAnisoContourLds);
-    while (cap > 0 && aniso_lds_bytes(cap) > budget) cap -= kProjChunk;
-    A.ccap_lds = std::max(0, cap);
-    const long long lds = A.ccap_lds > 0 ? aniso_lds_bytes(A.ccap_lds) : 0;
-    if (grid <= 0) grid = ctx->cu_count * per_cu(ctx, lds + ctx->static_aniso[ti]);
-    hipLaunchKernelGGL(k_aniso<T>, dim3(grid), dim3(256), (size_t)lds, st, A);
-    return GGX_OK;
+    A.seg_code = ctx->seg_code; A.seg_arc = ctx->seg_arc; A.sectors = ctx->sectors;
+    const int grid = std::max(1, std::min(items, ctx->cu_count * 64));
+    hipLaunchKernelGGL(k_sectors<T>, dim3(grid), dim3(64), 0, st, A);
+    hipLaunchKernelGGL(k_aniso<T>, dim3(grid), dim3(256), 0, st, A);
 }
 
 AnisoState aniso_state(const ggx_ctx* ctx) {
@@ -638,23 +627,9 @@ int launch_step(ggx_ctx* ctx, bool timed, bool record = false) {
         if (rc) return rc;
         HIPCHK(hipMemsetAsync(ctx->rec.area, 0, (size_t)ctx->nslots * 4, st));
     }
-    // anisotropic networks: the velocity corrector of every grain before any comparison reads
-    // the convolved fields
-    if (ctx->K.on && ctx->opt.persistent && NS - 1 <= kSmallNetwork) {
-        // a small network: one launch over all live grains (a launch costs about its slowest
-        // grain's lane-0 sector build, so one launch instead of one per bucket)
-        int rc = launch_aniso<T>(ctx, st, ctx->alist, &S->all_total, ctx->edges[ctx->nbuckets - 1], 0,
-                                 (const T*)P, Tt, Iold);
-        if (rc) return rc;
-    } else if (ctx->K.on) {
-        for (int b = 0; b < ctx->nbuckets; ++b) {
-            int grid = ctx->opt.persistent ? 0 : counts[b];
-            if (!ctx->opt.persistent && grid == 0) continue;
-            int rc = launch_aniso<T>(ctx, st, ctx->blists + (size_t)b * NS, &S->bucket_total[b], ctx->edges[b], grid,
-                                     (const T*)P, Tt, Iold);
-            if (rc) return rc;
-        }
-    }
+    if (ctx->K.on)
+        launch_aniso<T>(ctx, st, ctx->alist, &S->all_total, ctx->opt.persistent ? NS - 1 : std::max(1, ctx->h_sched->all_count),
+                        (const T*)P, Tt, Iold);
     if (timed) HIPCHK(hipEventRecord(ev[2], st));
     // comparison, contour, room for the new boxes, redistancing: per range of buckets
     LevelArgs<T> A = level_args<T>(ctx);
@@ -776,8 +751,7 @@ int launch_step_pergrain(ggx_ctx* ctx) {
     }
     if (ctx->K.on) {
         for (size_t i = 0; i < live.size(); ++i) {
-            int rc = launch_aniso<T>(ctx, st, ctx->pg_list + i, ctx->pg_one + i, bx[live[i]].n, 1, (const T*)P, Tt, Iold);
-            if (rc) return rc;
+            launch_aniso<T>(ctx, st, ctx->pg_list + i, ctx->pg_one + i, 1, (const T*)P, Tt, Iold);
         }
     }
     HIPCHK(hipEventRecord(ev[2], st));
@@ -1067,7 +1041,7 @@ extern "C" void ggx_destroy(ggx_ctx* ctx) {
     dfree(ctx->cmp_cnt); dfree(ctx->cmp); dfree(ctx->newbox); dfree(ctx->coff); dfree(ctx->ccap); dfree(ctx->clen);
     dfree(ctx->volume); dfree(ctx->perimeter); dfree(ctx->energy); dfree(ctx->meanda); dfree(ctx->nb_cnt);
     dfree(ctx->nb_id); dfree(ctx->nb_len);
-    dfree(ctx->quat); dfree(ctx->nb_e); dfree(ctx->nb_m); dfree(ctx->junc); dfree(ctx->jcnt); dfree(ctx->idl_org); dfree(ctx->sched); dfree(ctx->live); dfree(ctx->perm); dfree(ctx->kern_off); dfree(ctx->kern);
+    dfree(ctx->quat); dfree(ctx->nb_e); dfree(ctx->nb_m); dfree(ctx->junc); dfree(ctx->jcnt); dfree(ctx->idl_org); dfree(ctx->seg_code); dfree(ctx->seg_arc); dfree(ctx->sectors); dfree(ctx->sched); dfree(ctx->live); dfree(ctx->perm); dfree(ctx->kern_off); dfree(ctx->kern);
     dfree(ctx->tw); dfree(ctx->fft_work);
     dfree(ctx->blists); dfree(ctx->alist); dfree(ctx->pg_list); dfree(ctx->pg_one);
     {
@@ -1289,7 +1263,9 @@ extern "C" int ggx_load_network(ggx_ctx* ctx, const ggx_network* net) {
         // mobility 0 (grainBoundary.h:68)
         if ((rc = dalloc(ctx, ctx->quat, NS)) || (rc = dalloc(ctx, ctx->nb_e, (size_t)NS * kNbCap)) ||
             (rc = dalloc(ctx, ctx->nb_m, (size_t)NS * kNbCap)) || (rc = dalloc(ctx, ctx->junc, (size_t)NS * kJuncCap)) ||
-            (rc = dalloc(ctx, ctx->jcnt, NS)) || (rc = dalloc(ctx, ctx->idl_org, NS)))
+            (rc = dalloc(ctx, ctx->jcnt, NS)) || (rc = dalloc(ctx, ctx->idl_org, NS)) ||
+            (rc = dalloc(ctx, ctx->seg_code, (size_t)std::max(1LL, ctx->contour_cap))) ||
+            (rc = dalloc(ctx, ctx->seg_arc, (size_t)std::max(1LL, ctx->contour_cap))) || (rc = dalloc(ctx, ctx->sectors, NS)))
             return rc;
         std::vector<double4> hq((size_t)NS);
         std::vector<int2> horg((size_t)NS);
@@ -1666,7 +1642,8 @@ extern "C" int ggx_step_adjoint(ggx_ctx* ctx, const double* d_area, const double
     A.idl = R.idl; A.off_prev = R.off_prev; A.n_prev = R.nprev; A.flags = R.flags; A.err = nullptr; A.nslots = NS;
     A.pts = R.pts; A.coff = R.coff; A.clen = R.clen; A.nb_cnt = R.nb_cnt; A.nb_id = R.nb_id;
     A.S.quat = ctx->quat; A.S.nb_e = R.nb_e; A.S.nb_m = R.nb_m; A.S.junc = R.junc; A.S.jcnt = R.jcnt;
-    A.S.idl_org = R.idl_org; A.K = ctx->K; A.loop = nullptr; A.h = ctx->d.h; A.delta = ctx->d.delta; A.ccap_lds = 0;
+    A.S.idl_org = R.idl_org; A.K = ctx->K; A.loop = nullptr; A.h = ctx->d.h; A.delta = ctx->d.delta;
+    A.seg_code = nullptr; A.seg_arc = nullptr; A.sectors = nullptr;
     W.tilde0 = R.tilde0; W.lam_u = R.lam_u; W.grad = R.grad; W.loop = R.loop;
     hipLaunchKernelGGL(k_adj_weight, dim3(grid), dim3(256), 0, st, W);
     HIPCHK(hipGetLastError());

@@ -193,6 +193,9 @@ inline double __shfl_xor(double v, int mask) {
     return __longlong_as_double((long long)emu::wave_exchange((unsigned long long)__double_as_longlong(v),
                                                              (emu::g_cur % 64) ^ mask, false));
 }
+inline int __float_as_int(float f) { int r; std::memcpy(&r, &f, 4); return r; }
+inline float __int_as_float(int v) { float r; std::memcpy(&r, &v, 4); return r; }
+inline float __shfl_xor(float v, int mask) { return (float)__shfl_xor((double)v, mask); }
 
 #define threadIdx (emu::g_tid)
 #define blockIdx (emu::g_bid)
