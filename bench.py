@@ -201,7 +201,7 @@ def phase_split(G, N, s, net, prec, w, a):
         kern, byts, ms = "k_level", level_b, phases["level_ms"]
     else:
         fft = a.conv == "fft" or s.convolution_mode != 2
-        kern, byts, ms = ("k_conv_fft" if fft else "k_conv_dense"), conv_b, phases["convolution_ms"]
+        kern, byts, ms = ("k_conv_fft" if fft else "k_conv_tiles"), conv_b, phases["convolution_ms"]
     achieved = byts / (ms * 1e-3)
     precision = "fp64" if prec == N.PREC_FP64 else "fp32"
     if aniso:

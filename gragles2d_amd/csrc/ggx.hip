@@ -5,13 +5,13 @@
 //   k_reset / k_prep   deletion of grains that vanished in the previous step, survivor count,
 //                      filing of live grains into box-size buckets, allocator reset
 //   k_lists            comparison lists (computeSecondOrderNeighbours)
-//   k_conv_circulant   convolution of every live box (executeConvolution), one persistent
-//                      launch per bucket
+//   k_conv_tiles / k_conv_strip / k_conv_fft
+//                      convolution of every live box (executeConvolution)
 //   k_compare, k_contour, k_alloc, k_redist
 //                      comparison, contour / motion check / new box / neighbours / volume, room for
 //                      the new boxes, redistancing (executeComparison .. executeRedistancing), one
 //                      launch per range of buckets (level_groups)
-// Each bucket's launches get the LDS its largest box needs.
+// A launch gets the LDS the largest box of its buckets needs.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -101,10 +101,8 @@ struct ggx_ctx {
     int *pg_list = nullptr, *pg_one = nullptr;  // per-grain baseline: one-grain work lists
     long long updates_total = 0;
     int lds_per_cu = 163840;
-    int static_conv[2] = {0, 0};   // static LDS bytes of k_conv_circulant<double/float>
     int static_contour = 0;        // static LDS bytes of k_contour (the largest of its forms)
     int static_redist = 0;         // and of k_redist
-    int static_dense[2] = {0, 0};  // static LDS bytes of k_conv_dense<double/float>
 
     // circulant kernels of every box side 1 .. kMaxBox
     long long* kern_off = nullptr;
@@ -305,8 +303,7 @@ int raise_lds(ggx_ctx* ctx) {
     if (smp > lim) lim = smp;
     if (ctx->opt.lds_budget > 0) lim = std::min(lim, ctx->opt.lds_budget);
     // allow the dynamic-LDS kernels to use up to `lim`
-    const void* fns[] = {(const void*)k_conv_circulant<double>, (const void*)k_conv_circulant<float>,
-                         (const void*)k_conv_dense<double>, (const void*)k_conv_dense<float>,
+    const void* fns[] = {(const void*)k_conv_strip<double, 2>, (const void*)k_conv_strip<float, 2>,
                          (const void*)k_conv_fft<double, true>, (const void*)k_conv_fft<double, false>,
                          (const void*)k_conv_fft<float, true>, (const void*)k_conv_fft<float, false>,
                          (const void*)k_conv_fft_batch<true>, (const void*)k_conv_fft_batch<false>,
@@ -317,8 +314,12 @@ int raise_lds(ggx_ctx* ctx) {
                          (const void*)k_contour<double, false, true, 256>, (const void*)k_contour<float, false, true, 256>,
                          (const void*)k_contour<double, true, true, 256>, (const void*)k_contour<float, true, true, 256>,
                          (const void*)k_redist<double, 64>, (const void*)k_redist<double, 128>, (const void*)k_redist<double, 256>,
-                         (const void*)k_redist<float, 64>, (const void*)k_redist<float, 128>, (const void*)k_redist<float, 256>};
-    constexpr int kFns = (int)(sizeof(fns) / sizeof(fns[0])), kContour0 = 10, kRedist0 = 22;
+                         (const void*)k_redist<float, 64>, (const void*)k_redist<float, 128>, (const void*)k_redist<float, 256>,
+                         (const void*)k_conv_strip<double, 4>, (const void*)k_conv_strip<double, 8>,
+                         (const void*)k_conv_strip<float, 4>, (const void*)k_conv_strip<float, 8>,
+                         (const void*)k_conv_tiles<double, 2>, (const void*)k_conv_tiles<double, 3>, (const void*)k_conv_tiles<double, 4>,
+                         (const void*)k_conv_tiles<float, 2>, (const void*)k_conv_tiles<float, 3>, (const void*)k_conv_tiles<float, 4>};
+    constexpr int kFns = (int)(sizeof(fns) / sizeof(fns[0])), kContour0 = 8, kRedist0 = 20, kRedist1 = 26;
     for (const void* f : fns) {
         hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
         if (e != hipSuccess) {
@@ -328,15 +329,14 @@ int raise_lds(ggx_ctx* ctx) {
     }
     ctx->lds_max = lim;
     // static __shared__ bytes count against the same per-workgroup limit as the dynamic request
-    int* dst[] = {&ctx->static_conv[0], &ctx->static_conv[1], &ctx->static_dense[0], &ctx->static_dense[1],
-                  &ctx->static_fft[0][1], &ctx->static_fft[0][0], &ctx->static_fft[1][1], &ctx->static_fft[1][0]};
+    int* dst[] = {&ctx->static_fft[0][1], &ctx->static_fft[0][0], &ctx->static_fft[1][1], &ctx->static_fft[1][0]};
     for (int k = 0; k < kFns; ++k) {
         hipFuncAttributes fa;
         HIPCHK(hipFuncGetAttributes(&fa, fns[k]));
         const int st = (int)fa.sharedSizeBytes;
-        if (k < 8) *dst[k] = st;
-        else if (k >= kRedist0) ctx->static_redist = std::max(ctx->static_redist, st);
-        else if (k >= kContour0) ctx->static_contour = std::max(ctx->static_contour, st);
+        if (k >= 2 && k < 6) *dst[k - 2] = st;
+        else if (k >= kRedist0 && k < kRedist1) ctx->static_redist = std::max(ctx->static_redist, st);
+        else if (k >= kContour0 && k < kRedist0) ctx->static_contour = std::max(ctx->static_contour, st);
     }
     return GGX_OK;
 }
@@ -418,12 +418,26 @@ LevelArgs<T> level_args(const ggx_ctx* ctx) {
 }
 
 // Buckets b0 .. b1 of the work lists as one launch's items.
+Items bucket_items(const ggx_ctx* ctx, int b0, int b1) {
+    Items it;
+    it.lists = ctx->blists; it.total = ctx->sched->bucket_total; it.stride = ctx->nslots;
+    it.b0 = b0; it.b1 = b1;
+    for (int b = 0; b < kMaxBuckets; ++b) it.cap[b] = b < ctx->nbuckets ? slot_cap(ctx, b) : 0;
+    return it;
+}
+
+Items single_item(const int* list, const int* one, int n) {  // a one-grain work list, box side n
+    Items it;
+    it.lists = list; it.total = one; it.stride = 0;
+    it.b0 = it.b1 = 0;
+    for (int b = 0; b < kMaxBuckets; ++b) it.cap[b] = b == 0 ? contour_cap(n) : 0;
+    return it;
+}
+
 template <class T>
 void level_items(const ggx_ctx* ctx, LevelArgs<T>& A, int b0, int b1) {
-    A.it.lists = ctx->blists; A.it.total = ctx->sched->bucket_total; A.it.stride = ctx->nslots;
-    A.it.b0 = b0; A.it.b1 = b1;
+    A.it = bucket_items(ctx, b0, b1);
     A.cap = 0;
-    for (int b = 0; b < kMaxBuckets; ++b) A.it.cap[b] = b < ctx->nbuckets ? slot_cap(ctx, b) : 0;
     for (int b = b0; b <= b1; ++b) A.cap = std::max(A.cap, A.it.cap[b]);
     A.nb = ctx->edges[b1];
 }
@@ -556,29 +570,33 @@ int launch_conv_fft(ggx_ctx* ctx, hipStream_t st, const int* list, const int* co
     return GGX_OK;
 }
 
-// Convolution of the grains of one work list whose boxes have side <= nb: the FFT engine where
-// fft_for() picks it; else the register-blocked circulant when both of its tiles fit in LDS,
-// else the strip circulant.
+// The circulant convolution of a launch's items, boxes up to side nb: the register tiles of 2, 3 or 4
+// times 16 columns, the LDS strip above 64.
 template <class T>
-int launch_conv(ggx_ctx* ctx, hipStream_t st, const int* list, const int* count, int nb, int grid,
-                const T* src, T* dst) {
-    if (fft_for(ctx, nb)) return launch_conv_fft<T>(ctx, st, list, count, nb, grid, src, dst);
-    const int ti = sizeof(T) == 8 ? 0 : 1;
-    const long long dense = dense_lds<T>(nb);
-    if (dense + ctx->static_dense[ti] + 256 <= ctx->lds_max) {
-        if (grid <= 0) grid = ctx->cu_count * per_cu(ctx, dense + ctx->static_dense[ti]);
-        hipLaunchKernelGGL(k_conv_dense<T>, dim3(grid), dim3(256), (size_t)dense, st, list, count, ctx->box,
-                           ctx->off, src, dst, ctx->kern_off, (const T*)ctx->kern);
+int launch_conv(ggx_ctx* ctx, hipStream_t st, const Items& it, int nb, int items, const T* src, T* dst) {
+    const int nt = (nb + 15) / 16;
+    const T* kern = (const T*)ctx->kern;
+    if (nb <= 64) {
+        const int tiles = std::max(2, nt);
+        const size_t lds = (size_t)conv_tiles_lds<T>(tiles);
+        const dim3 grid(std::max(1, std::min(items, ctx->cu_count * 64))), block(64 * tiles);
+        if (tiles == 2)
+            hipLaunchKernelGGL((k_conv_tiles<T, 2>), grid, block, lds, st, it, ctx->box, ctx->off, src, dst, ctx->kern_off, kern);
+        else if (tiles == 3)
+            hipLaunchKernelGGL((k_conv_tiles<T, 3>), grid, block, lds, st, it, ctx->box, ctx->off, src, dst, ctx->kern_off, kern);
+        else
+            hipLaunchKernelGGL((k_conv_tiles<T, 4>), grid, block, lds, st, it, ctx->box, ctx->off, src, dst, ctx->kern_off, kern);
         return GGX_OK;
     }
-    const int conv_max = ctx->lds_max - ctx->static_conv[ti] - 256;
-    long long kkn = (2LL * nb + 4 + 1) & ~1LL;
-    long long need = (kkn + 2LL * nb * nb) * (long long)sizeof(T);
-    long long lds = std::min<long long>(need, conv_max);
-    if ((kkn + 4LL * nb) * (long long)sizeof(T) > lds) return fail(ctx, GGX_E_BOUNDS, "box too large for LDS strips");
-    if (grid <= 0) grid = ctx->cu_count * per_cu(ctx, lds + ctx->static_conv[ti]);
-    hipLaunchKernelGGL(k_conv_circulant<T>, dim3(grid), dim3(256), (size_t)lds, st, list, count, ctx->box,
-                       ctx->off, src, dst, ctx->kern_off, (const T*)ctx->kern, nb, (int)lds);
+    const long long lds = conv_strip_lds<T>(nb);
+    if (lds + 256 > ctx->lds_max) return fail(ctx, GGX_E_BOUNDS, "box too large for LDS strips");
+    const dim3 grid((unsigned)std::max<long long>(1, std::min<long long>((long long)items * nt, ctx->cu_count * 64))), block(256);
+    if (nb <= 128)
+        hipLaunchKernelGGL((k_conv_strip<T, 2>), grid, block, (size_t)lds, st, it, nt, ctx->box, ctx->off, src, dst, ctx->kern_off, kern);
+    else if (nb <= 256)
+        hipLaunchKernelGGL((k_conv_strip<T, 4>), grid, block, (size_t)lds, st, it, nt, ctx->box, ctx->off, src, dst, ctx->kern_off, kern);
+    else
+        hipLaunchKernelGGL((k_conv_strip<T, 8>), grid, block, (size_t)lds, st, it, nt, ctx->box, ctx->off, src, dst, ctx->kern_off, kern);
     return GGX_OK;
 }
 
@@ -612,13 +630,30 @@ int launch_step(ggx_ctx* ctx, bool timed, bool record = false) {
         HIPCHK(hipStreamSynchronize(st));
         for (int b = 0; b < ctx->nbuckets; ++b) counts[b] = ctx->h_sched->bucket_count[b];
     }
-    // convolution, one launch per bucket
-    for (int b = 0; b < ctx->nbuckets; ++b) {
-        int grid = ctx->opt.persistent ? 0 : counts[b];
-        if (!ctx->opt.persistent && grid == 0) continue;
-        int rc = launch_conv<T>(ctx, st, ctx->blists + (size_t)b * NS, &S->bucket_total[b],
-                                ctx->edges[b], grid, (const T*)P, Tt);
+    // convolution, per range of buckets of one engine and tile count
+    for (int b = 0; b < ctx->nbuckets;) {
+        const bool fft = fft_for(ctx, ctx->edges[b]);
+        int e = b;
+        if (!fft) {
+            auto tiles = [&](int k) {  // what a launch is sized for
+                const int side = ctx->edges[k];
+                return side <= 64 ? (ctx->merge_bucket >= 0 ? 4 : std::max(2, (side + 15) / 16)) : (side <= 128 ? 8 : side <= 256 ? 16 : 32);
+            };
+            while (e + 1 < ctx->nbuckets && !fft_for(ctx, ctx->edges[e + 1]) && tiles(e + 1) == tiles(b)) ++e;
+        }
+        int items = NS - 1;
+        if (!ctx->opt.persistent) {
+            items = 0;
+            for (int k = b; k <= e; ++k) items += counts[k];
+        }
+        int rc = GGX_OK;
+        if (fft && (ctx->opt.persistent || items > 0))
+            rc = launch_conv_fft<T>(ctx, st, ctx->blists + (size_t)b * NS, &S->bucket_total[b], ctx->edges[b],
+                                    ctx->opt.persistent ? 0 : items, (const T*)P, Tt);
+        else if (!fft && items > 0)
+            rc = launch_conv<T>(ctx, st, bucket_items(ctx, b, e), ctx->edges[e], items, (const T*)P, Tt);
         if (rc) return rc;
+        b = e + 1;
     }
     // a recorded step keeps the convolved fields before the corrector and the corrector's inputs
     if (record) {
@@ -745,8 +780,9 @@ int launch_step_pergrain(ggx_ctx* ctx) {
                            ctx->box, ctx->flags, ctx->sec_cnt, ctx->sec, ctx->cmp_cnt, ctx->cmp, ctx->errs);
     HIPCHK(hipEventRecord(ev[1], st));
     for (size_t i = 0; i < live.size(); ++i) {
-        int rc = launch_conv<T>(ctx, st, ctx->pg_list + i, ctx->pg_one + i, bx[live[i]].n, 1,
-                                (const T*)P, Tt);
+        const int n = bx[live[i]].n;
+        int rc = fft_for(ctx, n) ? launch_conv_fft<T>(ctx, st, ctx->pg_list + i, ctx->pg_one + i, n, 1, (const T*)P, Tt)
+                                 : launch_conv<T>(ctx, st, single_item(ctx->pg_list + i, ctx->pg_one + i, n), n, 1, (const T*)P, Tt);
         if (rc) return rc;
     }
     if (ctx->K.on) {
@@ -758,9 +794,9 @@ int launch_step_pergrain(ggx_ctx* ctx) {
     LevelArgs<T> A = level_args<T>(ctx);
     A.contour_base = nullptr;  // contour slots from the bump allocator
     for (size_t i = 0; i < live.size(); ++i) {
-        A.it.lists = ctx->pg_list + i; A.it.total = ctx->pg_one + i; A.it.stride = 0; A.it.b0 = A.it.b1 = 0;
         A.nb = bx[live[i]].n;
-        A.cap = A.it.cap[0] = contour_cap(A.nb);
+        A.cap = contour_cap(A.nb);
+        A.it = single_item(ctx->pg_list + i, ctx->pg_one + i, A.nb);
         int rc = launch_compare<T>(ctx, st, A, 1, false);
         if (!rc) rc = launch_contour<T>(ctx, st, A, 1, false);
         if (rc) return rc;

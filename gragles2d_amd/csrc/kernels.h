@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "ggx_internal.h"
 
 namespace ggx {
@@ -196,6 +198,43 @@ __global__ void __launch_bounds__(256) k_prep(int nslots, int* __restrict__ flag
     }
 }
 
+// A wave-uniform read of data no lane of this kernel writes (lists, boxes, offsets): through the
+// scalar cache into scalar registers, so that the chain list -> box -> field costs a scalar load's
+// latency per link and no lane waits for a broadcast.
+template <class X>
+__device__ __forceinline__ X sload(const X* p) {
+    return *(const __attribute__((address_space(4))) X*)p;
+}
+__device__ __forceinline__ Box sload_box(const Box* p) { return Box{sload(&p->x0), sload(&p->y0), sload(&p->n), 0}; }
+
+// Work items of a launch: the grains of buckets b0 .. b1, bucket after bucket.
+struct Items {
+    const int* lists;        // work list of bucket b at lists + b * stride
+    const int* total;        // grains per bucket (device)
+    int stride, b0, b1;
+    int cap[kMaxBuckets];    // contour points a grain of each bucket has room for
+};
+
+__device__ __forceinline__ int items_total(const Items& it) {
+    int n = 0;
+    for (int b = it.b0; b <= it.b1; ++b) n += sload(it.total + b);
+    return n;
+}
+
+// Grain of item `item`, with its bucket and its position in the bucket's list.
+__device__ __forceinline__ int item_grain(const Items& it, int item, int* bucket, int* pos) {
+    int b = it.b0;
+    while (b < it.b1) {
+        const int t = sload(it.total + b);
+        if (item < t) break;
+        item -= t;
+        ++b;
+    }
+    *bucket = b;
+    *pos = item;
+    return sload(it.lists + (size_t)b * it.stride + item);
+}
+
 // Work-list items.  Kernels whose per-item work is uniform (the convolutions: boxes of one bucket)
 // take them statically, workgroup i taking items i, i + grid, ...: a shared cursor costs one
 // same-address atomic per item, and those serialise across the chip at about 12 ns each.
@@ -376,268 +415,327 @@ __global__ void __launch_bounds__(256) k_lists(const int* __restrict__ alist, co
 
 // ------------------------------------------------------------------------------------------
 // Circulant tables: the table of box side n holds K_n[(t - kKPad) mod n] for
-// t in [0, 2n + 2 kKPad), so that every index a register block needs is in range without a
-// modulo.
+// t in [0, 2n + 2 kKPad), so that every index a tile needs is in range without a modulo (a step's
+// padding reaches three taps beyond the box).
 constexpr int kKPad = 8;
 __host__ __device__ inline long long ktab_len(int n) { return 2LL * n + 2 * kKPad; }
 
 // Convolution as an exact dense circulant (LSbox::convolutionGeneratorFFTW, box.cpp:622-695,
 // Gaussian mode).  The Gaussian symbol G(i,j) = g(i) g(j) is separable and even, so
 // IDFT(G . DFT(phi)) = K_n phi K_n with the symmetric circulant
-// K_n[m] = sum_k g(k) cos(2 pi k m / n), computed on the host per box size with all n taps
+// K_n[m] = sum_k g(k) cos(2 pi k m / n) computed on the host per box size with all n taps
 // (the symbol is cut at Nyquist, so K_n has a slowly decaying tail and cannot be banded).
-// Rows first, then columns.  Each lane produces a 4-wide run of outputs so that one LDS read
-// of the input feeds four FMAs.  kk holds K_n twice (length 2n) so no modulo is needed.
+//
+// Two contractions, so they run on the matrix cores: 16 x 16 x 4 products, whose sums are the
+// ascending chain of fused multiply-adds a scalar loop over the taps makes, bit for bit (FP64 and
+// FP32).  Rows first, B = phi K for all n rows of 16 columns, then columns, D = K B.  An FP64
+// product's result lies in the registers as the next product's operand does (row lane / 16 + 4 r of
+// the tile in register r, operand row lane / 16 of step r), so B need not leave them; an FP32 one
+// holds rows 4 (lane / 16) + r and is turned through LDS.  The operands come from LDS, where the
+// field lies zero-padded to whole tiles at a pitch that spreads a product's 16 rows over all banks
+// (read from global memory instead, a product's 16 row pieces take as long as the product), and the
+// coefficients of a step are 19 consecutive table entries.  Both kernels ask for two waves per SIMD or
+// more: within 256 registers the compiler keeps the accumulators in vector registers, else it moves
+// them to and from accumulation registers around every product (three times the time).
+//
+// On the 100k-grain network in FP64 (4 n flops and 16 bytes per point: floor 0.6 ms, the products at
+// the 77 TFLOP/s the matrix cores reach) this takes 1.2 ms per step, where register-blocked VALU
+// products with both tiles in LDS took 1.85 ms (five output blocks on four waves, 40 of 64 lanes
+// active).  The boxes of 130 to 190 points among 200 fine grains, whose tiles did not fit LDS before,
+// go from 1.7 to 0.05 ms.  What is left is the latency of reading and writing each box.
 // ------------------------------------------------------------------------------------------
-template <class T, int S>
-__device__ __forceinline__ void circ_run(const T* __restrict__ line, int stride, int n, int x0,
-                                         const T* __restrict__ kk, T* acc) {
-    // acc[s] = sum_j line[j] * K[(x0 + s - j) mod n],  kk[t] = K[t mod n] for t in [0, 2n)
-#pragma unroll
-    for (int s = 0; s < S; ++s) acc[s] = T(0);
-    for (int j = 0; j < n; ++j) {
-        T v = line[j * stride];
-        const T* kr = kk + (x0 - j + n);
-#pragma unroll
-        for (int s = 0; s < S; ++s) acc[s] += kr[s] * v;
+template <class T> struct Mma;
+template <> struct Mma<double> {
+    typedef double V __attribute__((vector_size(32)));
+    static __device__ __forceinline__ V run(double a, double b, V c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
+    static __device__ __forceinline__ int row(int q, int r) { return q + 4 * r; }  // of register r, lanes 16 q ..
+};
+template <> struct Mma<float> {
+    typedef float V __attribute__((vector_size(16)));
+    static __device__ __forceinline__ V run(float a, float b, V c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int q, int r) { return 4 * q + r; }
+};
+
+// Smallest pitch >= w at which lanes (row lane % 16, column lane / 16) meet every LDS bank once:
+// 2 mod 4 doubles, 4 mod 8 floats.
+template <class T>
+__host__ __device__ inline int tile_pitch(int w) {
+    constexpr int m = sizeof(T) == 8 ? 4 : 8;
+    return w + (m / 2 - w % m + m) % m;
 }
 
 template <class T>
-__device__ __forceinline__ void conv_one(int n, const T* __restrict__ s, T* __restrict__ d, T* kk, T* A, long long avail) {
-    constexpr int S = 4;
-    const long long nn = (long long)n * n;
-    const int runs = (n + S - 1) / S;  // output runs per line
-    if (2 * nn <= avail) {
-        T* B = A + nn;
-        for (long long p = threadIdx.x; p < nn; p += blockDim.x) A[p] = s[p];
-        __syncthreads();
-        for (int it = threadIdx.x; it < n * runs; it += blockDim.x) {
-            int y = it / runs, x0 = (it - y * runs) * S;
-            T acc[S];
-            circ_run<T, S>(A + (long long)y * n, 1, n, x0, kk, acc);
-#pragma unroll
-            for (int q = 0; q < S; ++q)
-                if (x0 + q < n) B[(long long)y * n + x0 + q] = acc[q];
-        }
-        __syncthreads();
-        for (int it = threadIdx.x; it < n * runs; it += blockDim.x) {
-            int x = it / runs, y0 = (it - x * runs) * S;
-            T acc[S];
-            circ_run<T, S>(B + x, n, n, y0, kk, acc);
-#pragma unroll
-            for (int q = 0; q < S; ++q)
-                if (y0 + q < n) d[(long long)(y0 + q) * n + x] = acc[q];
-        }
-        return;
-    }
-    // strip mode: rows in strips of H rows, then columns in strips of H columns
-    int H = (int)(avail / (2LL * n));
-    if (H < 1) H = 1;  // the host guarantees room for two lines
-    for (int y0 = 0; y0 < n; y0 += H) {
-        int hh = min(H, n - y0);
-        T* B = A + (long long)hh * n;
-        for (long long p = threadIdx.x; p < (long long)hh * n; p += blockDim.x) A[p] = s[(long long)y0 * n + p];
-        __syncthreads();
-        for (int it = threadIdx.x; it < hh * runs; it += blockDim.x) {
-            int y = it / runs, x0 = (it - y * runs) * S;
-            T acc[S];
-            circ_run<T, S>(A + (long long)y * n, 1, n, x0, kk, acc);
-#pragma unroll
-            for (int q = 0; q < S; ++q)
-                if (x0 + q < n) B[(long long)y * n + x0 + q] = acc[q];
-        }
-        __syncthreads();
-        for (long long p = threadIdx.x; p < (long long)hh * n; p += blockDim.x) d[(long long)y0 * n + p] = B[p];
-        __syncthreads();
-    }
-    __threadfence();
-    __syncthreads();
-    for (int xs = 0; xs < n; xs += H) {
-        int ww = min(H, n - xs);
-        T* B = A + (long long)ww * n;
-        for (long long p = threadIdx.x; p < (long long)ww * n; p += blockDim.x) {
-            int y = (int)(p / ww), x = (int)(p - (long long)y * ww);
-            A[(long long)x * n + y] = d[(long long)y * n + xs + x];
-        }
-        __syncthreads();
-        for (int it = threadIdx.x; it < ww * runs; it += blockDim.x) {
-            int x = it / runs, y0 = (it - x * runs) * S;
-            T acc[S];
-            circ_run<T, S>(A + (long long)x * n, 1, n, y0, kk, acc);
-#pragma unroll
-            for (int q = 0; q < S; ++q)
-                if (y0 + q < n) B[(long long)x * n + y0 + q] = acc[q];
-        }
-        __syncthreads();
-        for (long long p = threadIdx.x; p < (long long)ww * n; p += blockDim.x) {
-            int y = (int)(p / ww), x = (int)(p - (long long)y * ww);
-            d[(long long)y * n + xs + x] = B[(long long)x * n + y];
-        }
-        __syncthreads();
-    }
+__host__ __device__ inline long long conv_tiles_lds(int tiles) {
+    const int side = 16 * tiles;
+    // an FP32 wave turns its tiles through 16 x 17 floats
+    return ((long long)side * tile_pitch<T>(side) + ktab_len(side) + (sizeof(T) == 4 ? tiles * 16 * 17 : 0)) * (long long)sizeof(T);
 }
 
-// Persistent: every workgroup pulls grains of its bucket until the list is exhausted.
-template <class T>
-__global__ void __launch_bounds__(256) k_conv_circulant(const int* __restrict__ list, const int* __restrict__ count,
-                                                        const Box* __restrict__ box,
+// Boxes up to side 16 NT: a workgroup of NT waves per box, a wave per 16 columns, B in registers.  All
+// NT row tiles are multiplied, those beyond the box as zeros: a test per product costs more.
+template <class T, int NT>
+__global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT == 2 ? 5 : NT == 3 ? 4 : 3))) k_conv_tiles(Items it, const Box* __restrict__ box,
                                                         const long long* __restrict__ off, const T* __restrict__ src,
                                                         T* __restrict__ dst, const long long* __restrict__ kern_off,
-                                                        const T* __restrict__ kern, int nb, int lds_bytes) {
-    constexpr int S = 4;
+                                                        const T* __restrict__ kern) {
+    using V = typename Mma<T>::V;
     HIP_DYNAMIC_SHARED(unsigned char, smem)
-    const int kkn = (2 * nb + S + 1) & ~1;  // kk region sized for the bucket's largest box
-    T* kk = (T*)smem;
-    T* A = kk + kkn;
-    const long long avail = (long long)lds_bytes / (long long)sizeof(T) - kkn;
-    const int total = *count;  // written by k_tally (or the host) before this kernel
+    const int tid = (int)threadIdx.x, lane = tid & 63, j = lane & 15, q = lane >> 4;
+    const int xt = __builtin_amdgcn_readfirstlane(tid >> 6);
+    T* field = (T*)smem;
+    const int total = items_total(it);
+    // The next box is read while this one's products run: wave xt carries rows xt, xt + NT, .. (lane =
+    // column), thread tid the table's entry tid; its list entry was read one box earlier still.
+    T carry[16], coef;
+    int next_n = 0, next_g = 0;
+    long long next_o = 0;
+    auto grain_of = [&](int i) {
+        int bucket, pos;
+        return i < total ? item_grain(it, i, &bucket, &pos) : 0;
+    };
+    auto fetch = [&](int g) {
+        next_n = sload(&box[g].n);
+        next_o = sload(off + g);
+        const T* s = src + next_o;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int y = xt + NT * u;
+            carry[u] = y < next_n && lane < next_n ? s[y * next_n + lane] : T(0);
+        }
+        const T* kg = kern + sload(kern_off + next_n);
+        coef = tid < (int)ktab_len(next_n) ? kg[tid] : T(0);
+    };
+    if ((int)blockIdx.x < total) fetch(grain_of((int)blockIdx.x));
+    next_g = grain_of((int)blockIdx.x + (int)gridDim.x);
     for (int item = (int)blockIdx.x; item < total; item += (int)gridDim.x) {
+        const int n = next_n;
+        const long long o = next_o;
+        const int nt = (n + 15) >> 4, pairs = (n + 7) >> 3, pitch = tile_pitch<T>(8 * pairs);
+        T* table = field + 16 * NT * pitch;
         __syncthreads();  // the previous box's LDS is free
-        int g = list[item];
-        int n = box[g].n;
-        long long o = off[g];
-        const T* kg = kern + kern_off[n];
-        for (int t = threadIdx.x; t < 2 * n + S; t += blockDim.x) kk[t] = kg[kKPad + t % n];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int y = xt + NT * u;
+            if (lane < 8 * pairs) field[y * pitch + lane] = carry[u];
+        }
+        if (tid < (int)ktab_len(n)) table[tid] = coef;
         __syncthreads();
-        conv_one<T>(n, src + o, dst + o, kk, A, avail);
+        if (item + (int)gridDim.x < total) {
+            fetch(next_g);
+            next_g = grain_of(item + 2 * (int)gridDim.x);
+        }
+        if (xt >= nt) continue;
+        const T* kt = table + n + kKPad;         // K_n[m] at m, -n - kKPad <= m < n + kKPad
+        const int x = min(16 * xt + j, n - 1);  // columns beyond the box repeat the last one
+        V acc[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][r] = T(0);
+        // rows: B[y][x] = sum_k phi[y][k] K[x - k], two steps at a time
+        for (int p = 0; p < pairs; ++p) {
+            T v[2][NT], kb[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int k = 8 * p + 4 * u + q;
+                kb[u] = kt[x - k];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) v[u][t] = field[(16 * t + j) * pitch + k];
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[t] = Mma<T>::run(v[u][t], kb[u], acc[t]);
+        }
+        if constexpr (sizeof(T) == 4) {  // register r of lanes 16 q ..: row 4 q + r -> row q + 4 r
+            T* turn = table + ktab_len(n) + xt * 16 * 17;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) turn[(4 * q + r) * 17 + j] = acc[t][r];
+                wave_lds_sync();
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[t][r] = turn[(q + 4 * r) * 17 + j];
+                wave_lds_sync();
+            }
+        }
+        // columns: D[y][x] = sum_i K[y - i] B[i][x]; the rows of B beyond the box are zero, and the rows
+        // of D beyond it (clamped coefficients) are not stored
+        V out[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[t][r] = T(0);
+#pragma unroll
+        for (int p = 0; p < 2 * NT; ++p) {
+            if (p < pairs) {
+                T k[2][NT];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) k[u][t] = kt[min(16 * t + j, n - 1) - (8 * p + 4 * u + q)];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) out[t] = Mma<T>::run(k[u][t], acc[p >> 1][2 * (p & 1) + u], out[t]);
+            }
+        }
+        T* d = dst + o;
+        if (16 * xt + j < n) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int y = 16 * t + Mma<T>::row(q, r);
+                    if (y < n) d[y * n + 16 * xt + j] = out[t][r];
+                }
+        }
     }
 }
 
-// ------------------------------------------------------------------------------------------
-// The same circulant convolution, register-blocked for boxes whose two tiles fit in LDS.
-// Row pass: lane = row y, each task a block of 8 outputs x0..x0+7 of the wave's rows,
-//   B[y][x] = sum_j A[y][j] K[x - j];
-// column pass: lane = column x, each task a block of 8 outputs y0..y0+7,
-//   D[y][x] = sum_i B[i][x] K[y - i].
-// The circulant coefficients of a block depend only on the task, so they are wave-uniform and
-// come through the scalar cache into SGPRs; LDS only feeds the field values (one 8-byte read per
-// 8 FMAs).  The tiles are zero-padded to n8 = 8 ceil(n/8) rows and columns and their pitch
-// (n8 + 2 doubles, n8 + 4 floats) keeps the per-lane 16-byte row reads free of bank conflicts.
-// ------------------------------------------------------------------------------------------
-template <class T>
-__host__ __device__ inline int dense_pitch(int n8) { return n8 + (sizeof(T) == 8 ? 2 : 4); }
+// Larger boxes, up to side 64 TU: four waves share 16 columns, each takes every fourth 16-row tile;
+// B in LDS, the field through LDS 16 columns at a time (the next 16 on their way meanwhile).
+constexpr int kStripCols = 16;
 
 template <class T>
-__host__ __device__ inline long long dense_lds(int nb) {
-    const int n8 = (nb + 7) & ~7;
-    return 2LL * n8 * dense_pitch<T>(n8) * (long long)sizeof(T);
+__host__ __device__ inline long long conv_strip_lds(int nb) {
+    const int rows = (nb + 15) & ~15;
+    return ((long long)rows * 16 + (long long)rows * tile_pitch<T>(kStripCols) + ktab_len(nb)) * (long long)sizeof(T);
 }
 
-template <class T>
-using ctab_ptr = const __attribute__((address_space(4))) T*;
-
-template <class T>
-__device__ __forceinline__ void load8(const T* p, T* a) {
-    if constexpr (sizeof(T) == 8) {
-        const double2* q = reinterpret_cast<const double2*>(p);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) { double2 v = q[k]; a[2 * k] = v.x; a[2 * k + 1] = v.y; }
-    } else {
-        const float4* q = reinterpret_cast<const float4*>(p);
-#pragma unroll
-        for (int k = 0; k < 2; ++k) { float4 v = q[k]; a[4 * k] = v.x; a[4 * k + 1] = v.y; a[4 * k + 2] = v.z; a[4 * k + 3] = v.w; }
+// Calls f with the tile count as a constant: 1 .. N.
+template <int N, class F>
+__device__ __forceinline__ void by_tiles(int count, F f) {
+    if constexpr (N > 0) {
+        if (count == N) f(std::integral_constant<int, N>());
+        else by_tiles<N - 1>(count, f);
     }
 }
 
-template <class T>
-__device__ __forceinline__ void store8(T* p, const T* a) {
-    if constexpr (sizeof(T) == 8) {
-        double2* q = reinterpret_cast<double2*>(p);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) q[k] = make_double2(a[2 * k], a[2 * k + 1]);
-    } else {
-        float4* q = reinterpret_cast<float4*>(p);
-#pragma unroll
-        for (int k = 0; k < 2; ++k) q[k] = make_float4(a[4 * k], a[4 * k + 1], a[4 * k + 2], a[4 * k + 3]);
-    }
-}
-
-// acc[q] += sum_u v[u] * W[q - u + 7], W = 15 consecutive (wave-uniform) table entries
-template <class T>
-__device__ __forceinline__ void block8(T* acc, const T* v, ctab_ptr<T> w) {
-    T W[15];
-#pragma unroll
-    for (int t = 0; t < 15; ++t) W[t] = w[t];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-        for (int q = 0; q < 8; ++q) acc[q] += v[u] * W[q - u + 7];
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) k_conv_dense(const int* __restrict__ list, const int* __restrict__ count,
-                                                    const Box* __restrict__ box,
+template <class T, int TU>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_conv_strip(Items it, int blocks, const Box* __restrict__ box,
                                                     const long long* __restrict__ off, const T* __restrict__ src,
                                                     T* __restrict__ dst, const long long* __restrict__ kern_off,
                                                     const T* __restrict__ kern) {
+    using V = typename Mma<T>::V;
     HIP_DYNAMIC_SHARED(unsigned char, smem)
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int nwaves = (int)(blockDim.x >> 6);
-    const int total = __builtin_amdgcn_readfirstlane(*count);  // written by k_tally (or the host)
-    for (int item = (int)blockIdx.x; item < total; item += (int)gridDim.x) {
-        __syncthreads();  // the previous box's LDS is free
-        const int g = list[item];
-        const int n = box[g].n;
-        const long long o = off[g];
-        const int n8 = (n + 7) & ~7;
-        const int pa = dense_pitch<T>(n8);
-        T* A = (T*)smem;
-        T* B = A + (long long)n8 * pa;
-        const ctab_ptr<T> kt = (ctab_ptr<T>)(kern + kern_off[n]);
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, q = lane >> 4;
+    constexpr int kU = TU >= 8 ? 1 : 2;  // steps whose operands are read together
+    const int pitch = tile_pitch<T>(kStripCols);
+    const int total = items_total(it);
+    int item = (int)(blockIdx.x / (unsigned)blocks), xt = (int)(blockIdx.x % (unsigned)blocks);
+    const int item_step = (int)(gridDim.x / (unsigned)blocks), xt_step = (int)(gridDim.x % (unsigned)blocks);
+    for (; item < total; item += item_step, xt += xt_step) {
+        if (xt >= blocks) {
+            xt -= blocks;
+            if (++item >= total) break;
+        }
+        int bucket, pos;
+        const int g = item_grain(it, item, &bucket, &pos);
+        const int n = sload(&box[g].n);
+        const int nt = (n + 15) >> 4;
+        if (xt >= nt) continue;
+        const long long o = sload(off + g);
         const T* s = src + o;
-        // A = phi, zero-padded to n8 x n8
-        for (int p = threadIdx.x; p < n8 * n8; p += blockDim.x) {
-            const int y = p / n8, x = p - y * n8;
-            A[y * pa + x] = (y < n && x < n) ? s[y * n + x] : T(0);
-        }
-        __syncthreads();
-        // row pass
-        const int xb = n8 >> 3, rg = (n8 + 63) >> 6;
-        for (int task = wave; task < rg * xb; task += nwaves) {
-            const int r64 = task / xb, bx = task - r64 * xb;
-            const int y = r64 * 64 + lane, x0 = bx * 8;
-            T acc[8];
+        T* strip = (T*)smem;                      // B: row i, 16 columns
+        T* chunk = strip + 16 * nt * 16;          // the field's columns k0 .. k0 + 15, all rows
+        T* table = chunk + 16 * nt * pitch;
+        const T* kg = kern + sload(kern_off + n);
+        const T* kt = table + n + kKPad;
+        const int x = min(16 * xt + j, n - 1), low = -n - kKPad;  // the table's first tap: for the zeros beyond the box
+        // thread tid carries column tid % 16 of rows tid / 16 + 16 u
+        const int cx = tid & 15, cy = tid >> 4;
+        T carry[4 * TU];
+        auto fetch = [&](int k0) {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) acc[q] = T(0);
-            const T* arow = A + (long long)y * pa;
-            const bool on = y < n8;
-            for (int j0 = 0; j0 < n8; j0 += 8) {
-                T v[8];
-                if (on) load8(arow + j0, v);
-                else {
+            for (int u = 0; u < 4 * TU; ++u) {
+                const int y = cy + 16 * u;
+                carry[u] = u < nt && y < n && k0 + cx < n ? s[y * n + k0 + cx] : T(0);
+            }
+        };
+        fetch(0);
+        __syncthreads();  // the previous strip is free
+        for (int t = tid; t < (int)ktab_len(n); t += 256) table[t] = kg[t];
+        V acc[TU];
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) v[u] = T(0);
+        for (int u = 0; u < TU; ++u)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[u][r] = T(0);
+        // the products of this wave's U tiles (the count fixed at compile time: a test per product costs
+        // more than the product)
+        const int mine = (nt - wave + 3) >> 2;
+        auto rows_of = [&](auto tiles, int k0) {
+            constexpr int U = decltype(tiles)::value;
+#pragma unroll
+            for (int p0 = 0; p0 < 4; p0 += kU) {
+                T v[kU][U], kb[kU];
+#pragma unroll
+                for (int p = 0; p < kU; ++p) {
+                    const int k = 4 * (p0 + p) + q;
+                    kb[p] = kt[max(x - (k0 + k), low)];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) v[p][u] = chunk[(16 * (wave + 4 * u) + j) * pitch + k];
                 }
-                block8(acc, v, kt + (x0 - j0 + n + kKPad - 7));
+#pragma unroll
+                for (int p = 0; p < kU; ++p)
+#pragma unroll
+                    for (int u = 0; u < U; ++u) acc[u] = Mma<T>::run(v[p][u], kb[p], acc[u]);
             }
-            if (on) store8(B + (long long)y * pa + x0, acc);
+        };
+        auto columns_of = [&](auto tiles) {
+            constexpr int U = decltype(tiles)::value;
+            for (int p0 = 0; p0 < 4 * nt; p0 += kU) {
+                T v[kU], k[kU][U];
+#pragma unroll
+                for (int p = 0; p < kU; ++p) {
+                    const int i = 4 * (p0 + p) + q;
+                    v[p] = strip[i * 16 + j];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) k[p][u] = kt[max(min(16 * (wave + 4 * u) + j, n - 1) - i, low)];
+                }
+#pragma unroll
+                for (int p = 0; p < kU; ++p)
+#pragma unroll
+                    for (int u = 0; u < U; ++u) acc[u] = Mma<T>::run(k[p][u], v[p], acc[u]);
+            }
+        };
+        auto rows = [&](int k0) { by_tiles<TU>(mine, [&](auto tiles) { rows_of(tiles, k0); }); };
+        auto columns = [&]() { by_tiles<TU>(mine, [&](auto tiles) { columns_of(tiles); }); };
+        for (int k0 = 0; k0 < n; k0 += kStripCols) {
+#pragma unroll
+            for (int u = 0; u < 4 * TU; ++u)
+                if (u < nt) chunk[(cy + 16 * u) * pitch + cx] = carry[u];
+            __syncthreads();
+            if (k0 + kStripCols < n) fetch(k0 + kStripCols);
+            rows(k0);
+            __syncthreads();
         }
+#pragma unroll
+        for (int u = 0; u < TU; ++u)
+            if (wave + 4 * u < nt) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    strip[(16 * (wave + 4 * u) + Mma<T>::row(q, r)) * 16 + j] = acc[u][r];
+                    acc[u][r] = T(0);
+                }
+            }
         __syncthreads();
-        // column pass
-        const int yb = n8 >> 3, cg = (n + 63) >> 6;
+        columns();
         T* d = dst + o;
-        for (int task = wave; task < cg * yb; task += nwaves) {
-            const int c64 = task / yb, by = task - c64 * yb;
-            const int x = c64 * 64 + lane, y0 = by * 8;
-            const bool on = x < n;
-            T acc[8];
+        if (16 * xt + j < n) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r) acc[r] = T(0);
-            for (int i0 = 0; i0 < n8; i0 += 8) {
-                T v[8];
+            for (int u = 0; u < TU; ++u)
 #pragma unroll
-                for (int u = 0; u < 8; ++u) v[u] = on ? B[(long long)(i0 + u) * pa + x] : T(0);
-                block8(acc, v, kt + (y0 - i0 + n + kKPad - 7));
-            }
-            if (on) {
-#pragma unroll
-                for (int r = 0; r < 8; ++r)
-                    if (y0 + r < n) d[(long long)(y0 + r) * n + x] = acc[r];
-            }
+                for (int r = 0; r < 4; ++r) {
+                    const int y = 16 * (wave + 4 * u) + Mma<T>::row(q, r);
+                    if (y < n) d[y * n + 16 * xt + j] = acc[u][r];
+                }
         }
-        __syncthreads();
     }
 }
 

@@ -25,29 +25,6 @@
 
 namespace ggx {
 
-// Work items of a launch: the grains of buckets b0 .. b1, bucket after bucket.
-struct Items {
-    const int* lists;        // work list of bucket b at lists + b * stride
-    const int* total;        // grains per bucket (device)
-    int stride, b0, b1;
-    int cap[kMaxBuckets];    // contour points a grain of each bucket has room for
-};
-
-__device__ __forceinline__ int items_total(const Items& it) {
-    int n = 0;
-    for (int b = it.b0; b <= it.b1; ++b) n += it.total[b];
-    return n;
-}
-
-// Grain of item `item`, with its bucket and its position in the bucket's list.
-__device__ __forceinline__ int item_grain(const Items& it, int item, int* bucket, int* pos) {
-    int b = it.b0;
-    while (b < it.b1 && item >= it.total[b]) { item -= it.total[b]; ++b; }
-    *bucket = b;
-    *pos = item;
-    return it.lists[(size_t)b * it.stride + item];
-}
-
 // Sign planes of the compared fields, 64-bit words in the grain's field slot (offset / 8 words,
 // which n rows of ceil(n / 64) words always fit): per row and per column the bits C >= 0 and C > 0.
 // Row bits beyond the box are zero; column bits beyond it are undefined.
@@ -256,16 +233,16 @@ __global__ void __launch_bounds__(256) k_compare(LevelArgs<T> A) {
             if (++item >= total) break;
         }
         int bucket, pos;
-        const int g = __builtin_amdgcn_readfirstlane(item_grain(A.it, item, &bucket, &pos));
-        const Box b = A.box[g];
+        const int g = item_grain(A.it, item, &bucket, &pos);
+        const Box b = sload_box(A.box + g);
         const int n = b.n, W = (n + 63) >> 6, rb = (n + kRows - 1) / kRows;
         if (blk >= rb * W) continue;
         const int xc = blk / rb, rblk = blk - xc * rb;
         const int r0 = rblk * kRows, rows = min(kRows, n - r0), x = xc * 64 + lane;
         const bool on = x < n;
-        const long long o = A.off[g];
-        const bool cmp_on = COARSEN ? ((A.O.flags[g] & kExists) != 0) : true;
-        const int cnt = cmp_on ? A.cmp_cnt[g] : 0;
+        const long long o = sload(A.off + g);
+        const bool cmp_on = COARSEN ? ((sload(A.O.flags + g) & kExists) != 0) : true;
+        const int cnt = cmp_on ? sload(A.cmp_cnt + g) : 0;
         T own[kRows], mx[kRows];
         int id[kRows];
 #pragma unroll
@@ -334,8 +311,9 @@ __global__ void __launch_bounds__(256) k_compare(LevelArgs<T> A) {
         // per pixel: the wall as grain 0, IDLocal, the set comparison, the sign bits
         const bool bnd = at_wall(b, G) && cmp_on;
         const double band = 0.7 * G.delta;
-        const long long np = (long long)A.n_prev[g] * A.n_prev[g];
-        const long long op = A.off_prev[g];
+        const int nprev = sload(A.n_prev + g);
+        const long long np = (long long)nprev * nprev;
+        const long long op = sload(A.off_prev + g);
         unsigned long long row_ge = 0, row_gt = 0;  // of the block's row `lane`
         unsigned col_ge = 0, col_gt = 0;            // of the lane's column, bit = row
 #pragma unroll
@@ -499,9 +477,9 @@ __global__ void __launch_bounds__(NT) k_contour(LevelArgs<T> A) {
         int bucket, pos;
         const int g = item_grain(A.it, item, &bucket, &pos);
         const int ccap = A.it.cap[bucket];
-        const Box b = A.box[g];
+        const Box b = sload_box(A.box + g);
         const int n = b.n, W = (n + 63) >> 6;
-        const long long o = A.off[g];
+        const long long o = sload(A.off + g);
         const long long nn = (long long)n * n;
         unsigned long long* bits = A.bits + (o >> 3);
         T* C = A.cfield + o;
@@ -1470,12 +1448,12 @@ __global__ void __launch_bounds__(NT) k_redist(LevelArgs<T> A) {
         __syncthreads();  // the previous grain's tile is free
         int bucket, pos;
         const int g = item_grain(A.it, item, &bucket, &pos);
-        if (!(A.O.flags[g] & kExists)) continue;  // vanished, or no room for its field
-        const Box b = A.box[g], bo = A.O.box_next[g];
+        if (!(sload(A.O.flags + g) & kExists)) continue;  // vanished, or no room for its field
+        const Box b = sload_box(A.box + g), bo = sload_box(A.O.box_next + g);
         const int n = b.n, no = bo.n, W = (n + 63) >> 6, words = 2 * W;
-        const long long o = A.off[g];
+        const long long o = sload(A.off + g);
         const T* C = A.cfield + o;
-        T* gout = A.out_field + A.O.off_next[g];
+        T* gout = A.out_field + sload(A.O.off_next + g);
         const unsigned long long* bits = A.bits + (o >> 3);
         const int ixmin = max(b.x0, bo.x0), ixmax = min(b.x0 + n, bo.x0 + no);
         const int iymin = max(b.y0, bo.y0), iymax = min(b.y0 + n, bo.y0 + no);

@@ -196,6 +196,36 @@ inline double __shfl_xor(double v, int mask) {
 inline int __float_as_int(float f) { int r; std::memcpy(&r, &f, 4); return r; }
 inline float __int_as_float(int v) { float r; std::memcpy(&r, &v, 4); return r; }
 inline float __shfl_xor(float v, int mask) { return (float)__shfl_xor((double)v, mask); }
+// Matrix products of a wave: 16 x 16 results, four fused multiply-adds in ascending order each.
+// Operands a: row lane % 16, term lane / 16; b: column lane % 16, term lane / 16.
+namespace emu {
+// Two buffers in turn: a lane fills a buffer again only after every lane has met the barrier of the
+// product between, so one barrier per product is enough.
+inline double g_ma[2][16][64], g_mb[2][16][64];
+inline unsigned g_mturn[16][64];
+template <class V, class X, class Row>
+inline V mfma(X a, X b, V c, Row row) {
+    const unsigned w = (unsigned)g_cur / 64u, l = (unsigned)g_cur % 64u, t = g_mturn[w][l]++ & 1u;
+    g_ma[t][w][l] = a;
+    g_mb[t][w][l] = b;
+    wave_sync();
+    for (int r = 0; r < 4; ++r) {
+        X s = c[r];
+        for (int k = 0; k < 4; ++k)
+            s = std::fma((X)g_ma[t][w][row((int)(l / 16), r) + 16 * k], (X)g_mb[t][w][l % 16 + 16 * k], s);
+        c[r] = s;
+    }
+    return c;
+}
+typedef double v4d __attribute__((vector_size(32)));
+typedef float v4f __attribute__((vector_size(16)));
+}  // namespace emu
+inline emu::v4d __builtin_amdgcn_mfma_f64_16x16x4f64(double a, double b, emu::v4d c, int, int, int) {
+    return emu::mfma(a, b, c, [](int q, int r) { return q + 4 * r; });
+}
+inline emu::v4f __builtin_amdgcn_mfma_f32_16x16x4f32(float a, float b, emu::v4f c, int, int, int) {
+    return emu::mfma(a, b, c, [](int q, int r) { return 4 * q + r; });
+}
 
 #define threadIdx (emu::g_tid)
 #define blockIdx (emu::g_bid)
