@@ -2,7 +2,8 @@
 //
 // Replaces the bodies of the grainhdl phase loops (src/grainhdl.cpp:755-869, 1243-1256,
 // 1381-1394) with batched HIP launches.  Per step, with no host round trip:
-//   k_reset / k_prep   deletion of grains that vanished in the previous step, survivor count,
+//   k_reset / k_prep / k_tally (k_schedule for small networks)
+//                      deletion of grains that vanished in the previous step, survivor count,
 //                      filing of live grains into box-size buckets, allocator reset
 //   k_lists            comparison lists (computeSecondOrderNeighbours)
 //   k_conv_tiles / k_conv_strip / k_conv_fft
@@ -464,7 +465,8 @@ std::vector<std::pair<int, int>> level_groups(const ggx_ctx* ctx) {
 
 template <class T>
 int launch_compare(const ggx_ctx* ctx, hipStream_t st, LevelArgs<T>& A, int items, bool coarsen) {
-    A.blocks = ((A.nb + kRows - 1) / kRows) * ((A.nb + 63) / 64);
+    // a small network's launch holds boxes of every side: 32 waves per grain, which larger boxes loop over
+    A.blocks = std::min(32, ((A.nb + kRows - 1) / kRows) * ((A.nb + 63) / 64));
     const long long wgs = ((long long)items * A.blocks + 3) / 4;
     const int grid = (int)std::max<long long>(1, std::min<long long>(wgs, ctx->cu_count * 8));
     if (coarsen) hipLaunchKernelGGL((k_compare<T, true>), dim3(grid), dim3(256), 0, st, A);
@@ -615,13 +617,17 @@ int launch_step(ggx_ctx* ctx, bool timed, bool record = false) {
     if (timed) ev = take_events(ctx, 5);
 
     if (timed) HIPCHK(hipEventRecord(ev[0], st));
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(32), 0, st, S);
-    hipLaunchKernelGGL(k_prep, dim3((NS + 255) / 256), dim3(256), 0, st, NS, ctx->flags, ctx->box, bucket_table(ctx),
-                       ctx->blists, ctx->alist, ctx->errs, S, (const int*)ctx->perm);
-    hipLaunchKernelGGL(k_tally, dim3(1), dim3(64), 0, st, S, bucket_table(ctx));
-    hipLaunchKernelGGL(k_lists, dim3(cus * 8), dim3(256), 0, st, ctx->alist, &S->all_total, &S->cursor[kMaxBuckets],
-                       ctx->box,
-                       ctx->flags, ctx->sec_cnt, ctx->sec, ctx->cmp_cnt, ctx->cmp, ctx->errs);
+    if (NS - 1 <= kSmallNetwork) {
+        hipLaunchKernelGGL(k_schedule, dim3(1), dim3(1024), 0, st, NS, ctx->flags, ctx->box, bucket_table(ctx), ctx->blists,
+                           ctx->alist, ctx->errs, S, (const int*)ctx->perm);
+    } else {
+        hipLaunchKernelGGL(k_reset, dim3(1), dim3(32), 0, st, S);
+        hipLaunchKernelGGL(k_prep, dim3((NS + 255) / 256), dim3(256), 0, st, NS, ctx->flags, ctx->box, bucket_table(ctx),
+                           ctx->blists, ctx->alist, ctx->errs, S, (const int*)ctx->perm);
+        hipLaunchKernelGGL(k_tally, dim3(1), dim3(64), 0, st, S, bucket_table(ctx));
+    }
+    hipLaunchKernelGGL(k_lists, dim3(std::max(1, std::min(NS - 1, cus * 64))), dim3(64), 0, st, (const int*)ctx->alist,
+                       (const int*)&S->all_total, ctx->box, ctx->flags, ctx->sec_cnt, ctx->sec, ctx->cmp_cnt, ctx->cmp, ctx->errs);
     if (timed) HIPCHK(hipEventRecord(ev[1], st));
     // grid per bucket: persistent (fixed) or one workgroup per grain (counts read back)
     int counts[kMaxBuckets];
@@ -679,7 +685,12 @@ int launch_step(ggx_ctx* ctx, bool timed, bool record = false) {
         return c;
     };
     for (int phase = 0; phase < 3; ++phase) {
-        for (const auto& r : groups) {
+        for (auto r : groups) {
+            // k_compare has no size-dependent resources: a small network takes one launch of it
+            if (phase == 0 && ctx->merge_bucket >= 0) {
+                if (r.first > 0) continue;
+                r.second = ctx->nbuckets - 1;
+            }
             const int k = items(r);
             if (k == 0) continue;
             level_items(ctx, A, r.first, r.second);
@@ -776,7 +787,7 @@ int launch_step_pergrain(ggx_ctx* ctx) {
     hipLaunchKernelGGL(k_prep, dim3((NS + 255) / 256), dim3(256), 0, st, NS, ctx->flags, ctx->box, bucket_table(ctx),
                        ctx->blists, ctx->alist, ctx->errs, S, (const int*)nullptr);
     for (size_t i = 0; i < L; ++i)
-        hipLaunchKernelGGL(k_lists, dim3(1), dim3(256), 0, st, ctx->pg_list + i, ctx->pg_one + i, (int*)nullptr,
+        hipLaunchKernelGGL(k_lists, dim3(1), dim3(64), 0, st, (const int*)(ctx->pg_list + i), (const int*)(ctx->pg_one + i),
                            ctx->box, ctx->flags, ctx->sec_cnt, ctx->sec, ctx->cmp_cnt, ctx->cmp, ctx->errs);
     HIPCHK(hipEventRecord(ev[1], st));
     for (size_t i = 0; i < live.size(); ++i) {
@@ -934,7 +945,6 @@ int coarsen(ggx_ctx* ctx, int present) {
     long long cbase = 0;
     for (int b = 0; b < ctx->nbuckets; ++b) {
         hs.bucket_total[b] = (int)bl[(size_t)b].size();
-        hs.cursor[b] = 0;
         hs.contour_base[b] = cbase;
         cbase += (long long)bl[(size_t)b].size() * (long long)slot_cap(ctx, b);
         if (!bl[(size_t)b].empty())

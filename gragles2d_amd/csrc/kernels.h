@@ -63,7 +63,6 @@ constexpr int kSmallNetwork = 4096;
 constexpr int kMergeSide = 64;
 
 struct Sched {
-    int cursor[kMaxBuckets + 1];     // work cursors: level-set kernel per bucket, then the lists
     int bucket_count[kMaxBuckets];   // live grains per bucket (advanced by k_prep's atomics)
     int bucket_total[kMaxBuckets];   // the same, written by k_tally for the later kernels
     long long contour_base[kMaxBuckets];  // first contour point of each bucket's slots (k_tally)
@@ -110,7 +109,6 @@ __device__ __forceinline__ int load_counter(const int* p) {
 __global__ void k_reset(Sched* __restrict__ S) {
     int t = threadIdx.x;
     if (t < kMaxBuckets) S->bucket_count[t] = 0;
-    if (t <= kMaxBuckets) S->cursor[t] = 0;
     if (t == 0) {
         S->all_count = 0; S->present = 0; S->max_n = 0; S->any_err = 0;
         // the previous step's output layout is this step's input; its bump counters were advanced
@@ -141,9 +139,20 @@ __global__ void k_tally(Sched* __restrict__ S, Buckets B) {
     }
 }
 
-// A grain that carries an error (or a box above the largest bucket) is taken out of the step:
-// its existence flag is cleared, so no list, gather or launch touches its slots again, and it
-// is deleted at the next step like a vanished grain; the host reports the error.
+// The flags of grain g at the start of a step: deletion of a grain that vanished in the last one.  A
+// grain that carries an error (or a box above the largest bucket) is taken out of the step: its
+// existence flag is cleared, so no list, gather or launch touches its slots again, and it is deleted
+// at the next step like a vanished grain; the host reports the error.
+__device__ __forceinline__ int schedule_flags(int g, int* flags, const Box* box, int* err, const Buckets& B, bool* bad) {
+    int f = flags[g];
+    if (f & kGone) { f &= ~kGone; flags[g] = f; }
+    if ((f & kPresent) && !(f & kExists)) { f = (f & ~kPresent) | kGone; flags[g] = f; }
+    if ((f & kPresent) && (f & kExists) && !err[g] && box[g].n > B.edge[B.count - 1]) err[g] = kErrBoxCap;
+    *bad = err[g] != 0;
+    if (*bad && (f & kExists)) { f &= ~kExists; flags[g] = f; }
+    return f;
+}
+
 // perm: the grain ids in a spatial order (the work lists come out in that order), or null.
 __global__ void __launch_bounds__(256) k_prep(int nslots, int* __restrict__ flags, const Box* __restrict__ box,
                                               Buckets B, int* __restrict__ blists, int* __restrict__ alist,
@@ -160,14 +169,9 @@ __global__ void __launch_bounds__(256) k_prep(int nslots, int* __restrict__ flag
     const int g = perm ? (idx < nslots - 1 ? perm[idx] : 0) : idx;
     int bk = -1, lpos = -1, apos = -1, n = 0;
     if (g > 0 && g < nslots) {
-        int f = flags[g];
-        if (f & kGone) { f &= ~kGone; flags[g] = f; }
-        if ((f & kPresent) && !(f & kExists)) { f = (f & ~kPresent) | kGone; flags[g] = f; }
-        if ((f & kPresent) && (f & kExists) && !err[g] && box[g].n > B.edge[B.count - 1]) err[g] = kErrBoxCap;
-        if (err[g]) {
-            s_err = 1;
-            if (f & kExists) { f &= ~kExists; flags[g] = f; }
-        }
+        bool bad;
+        const int f = schedule_flags(g, flags, box, err, B, &bad);
+        if (bad) s_err = 1;
         if (f & kPresent) {
             atomicAdd(&s_present, 1);
             if (f & kExists) {
@@ -235,32 +239,70 @@ __device__ __forceinline__ int item_grain(const Items& it, int item, int* bucket
     return sload(it.lists + (size_t)b * it.stride + item);
 }
 
-// Work-list items.  Kernels whose per-item work is uniform (the convolutions: boxes of one bucket)
-// take them statically, workgroup i taking items i, i + grid, ...: a shared cursor costs one
-// same-address atomic per item, and those serialise across the chip at about 12 ns each.
-// Kernels whose per-item work varies with the grain (lists, level set) pull items from a cursor
-// when one is given (dynamic balance), else statically; with a cursor, one atomic takes a chunk
-// of `chunk` consecutive items (chunk c covers items c * chunk ... c * chunk + chunk - 1).
-__device__ __forceinline__ int take_item(int* cursor, int* s_slot, int prev, int chunk = 1) {
-    if (!cursor) return prev < 0 ? (int)blockIdx.x : prev + (int)gridDim.x;
-    if (prev >= 0 && (prev + 1) % chunk != 0) return prev + 1;
+// k_reset, k_prep and k_tally in one workgroup, for small networks: three dependent launches take
+// 15 us there, one takes 5 us.
+__global__ void __launch_bounds__(1024) k_schedule(int nslots, int* __restrict__ flags, const Box* __restrict__ box,
+                                                   Buckets B, int* __restrict__ blists, int* __restrict__ alist,
+                                                   int* __restrict__ err, Sched* __restrict__ S, const int* __restrict__ perm) {
+    __shared__ int s_cnt[kMaxBuckets];
+    __shared__ int s_all, s_present, s_err, s_maxn;
+    __shared__ unsigned long long s_upd;
+    const int t = (int)threadIdx.x;
+    if (t < kMaxBuckets) s_cnt[t] = 0;
+    if (t == 0) { s_all = 0; s_present = 0; s_err = 0; s_maxn = 0; s_upd = 0ull; }
     __syncthreads();
-    if (threadIdx.x == 0) *s_slot = atomicAdd(cursor, 1) * chunk;
+    int present = 0, maxn = 0;
+    double upd = 0.0;  // sums of n^2 are exact
+    for (int i = t; i < nslots - 1; i += (int)blockDim.x) {
+        const int g = perm[i];
+        if (g <= 0 || g >= nslots) continue;
+        bool bad;
+        const int f = schedule_flags(g, flags, box, err, B, &bad);
+        if (bad) s_err = 1;
+        if (!(f & kPresent)) continue;
+        present++;
+        if (!(f & kExists)) continue;
+        const int n = box[g].n;
+        int bk = 0;
+        while (n > B.edge[bk]) bk++;
+        blists[(size_t)bk * nslots + atomicAdd(&s_cnt[bk], 1)] = g;
+        alist[atomicAdd(&s_all, 1)] = g;
+        maxn = max(maxn, n);
+        upd += (double)n * n;
+    }
+    double p = present, m = maxn;
+    for (int d = 32; d >= 1; d >>= 1) {
+        p += __shfl_xor(p, d);
+        m = fmax(m, __shfl_xor(m, d));
+        upd += __shfl_xor(upd, d);
+    }
+    if ((t & 63) == 0) {
+        atomicAdd(&s_present, (int)p);
+        atomicMax(&s_maxn, (int)m);
+        atomicAdd(&s_upd, (unsigned long long)upd);
+    }
     __syncthreads();
-    return *s_slot;
+    if (t < kMaxBuckets) {
+        S->bucket_count[t] = s_cnt[t];
+        S->bucket_total[t] = t < B.count ? s_cnt[t] : 0;
+    }
+    if (t == 0) {
+        S->all_count = s_all; S->all_total = s_all; S->present = s_present; S->max_n = s_maxn; S->any_err = s_err;
+        // the previous step's output layout is this step's input; k_alloc's atomics advanced its counter
+        S->in_top = atomicExch(&S->tops[0], 0ull);
+        S->loop_cur = S->loop_next;
+        S->loop_next = S->loop_next + 1;
+        S->updates = s_upd;
+        S->updates_total += s_upd;
+        S->steps_total += 1ull;
+        long long base = 0;
+        for (int b = 0; b < B.count; ++b) {
+            S->contour_base[b] = base;
+            base += (long long)s_cnt[b] * (long long)B.cap[b];
+        }
+        (void)atomicExch(&S->tops[1], (unsigned long long)base);
+    }
 }
-
-// ------------------------------------------------------------------------------------------
-// Comparison lists, LSbox::computeSecondOrderNeighbours (box.cpp:1027-1068).  One 64-lane
-// workgroup per grain.  cmp = the existing entries of the previous list, then every existing
-// neighbour-of-neighbour whose input box intersects (closed intervals, checkIntersection,
-// box.cpp:881-888), first occurrence only, excluding self and the boundary grain.  The
-// first-occurrence test is an LDS hash (grain id -> smallest candidate index), so the
-// candidates are examined in parallel and compacted in their original order.
-// ------------------------------------------------------------------------------------------
-constexpr int kHash = 1024;      // LDS hash slots (grain id -> smallest candidate index)
-constexpr int kHashFill = 768;   // distinct keys allowed per grain (> 2 kCmpCap: beyond it the list overflows anyway)
-constexpr int kCandChunk = 2048; // neighbours-of-neighbours staged in LDS at a time
 
 // Block-wide exclusive scan of one int per lane; returns the exclusive prefix, *total gets the sum.
 // Shuffles within each wave, one exchange of wave totals through LDS (s_tmp: one int per wave).
@@ -285,129 +327,145 @@ __device__ __forceinline__ int block_scan(int v, int* s_tmp, int* total) {
     return base + x - v;
 }
 
+// ------------------------------------------------------------------------------------------
+// Comparison lists, LSbox::computeSecondOrderNeighbours (box.cpp:1027-1068).  cmp = the existing
+// entries of the previous list, then every existing neighbour-of-neighbour whose input box
+// intersects (closed intervals, checkIntersection, box.cpp:881-888), first occurrence only,
+// excluding self and the boundary grain.
+//
+// One wave per grain.  Bound by latency: list -> its entries' lists -> their flags and boxes, three
+// dependent reads, so the wave takes 256 candidates at a time (four reads in flight per lane) and
+// meets no workgroup barrier.  The first-occurrence test is an LDS hash (grain id -> smallest
+// candidate index): the candidates of a pass are entered together, and a candidate whose index the
+// table then holds is a first occurrence, since the later passes' indices are larger.  A 256-lane
+// workgroup per grain, pulled from a cursor with two passes over the candidates, took 1.10 ms for
+// 100k grains and 60 to 70 us for 100; this takes 0.21 ms and 10 us.
+// ------------------------------------------------------------------------------------------
+constexpr int kHash = 512;       // LDS hash slots (grain id -> smallest candidate index)
+constexpr int kHashFill = 320;   // distinct keys allowed per grain (> 2 kCmpCap: beyond it the list overflows anyway)
+static_assert(kHashFill > 2 * kCmpCap && kHashFill + 64 < kHash, "hash capacity");
+
 // Open-addressing insert (key-CAS): returns the slot holding `key`, or -1 when the table holds
-// kHashFill keys already (the caller reports an error; probing stays bounded).
+// kHashFill keys already (the caller reports an error; probing stays bounded: the lanes that pass
+// the test together enter at most one key each).
 __device__ __forceinline__ int hash_insert(int* h_key, int* fill, int key) {
-    unsigned hs = ((unsigned)key * 2654435761u) & (kHash - 1);
-    while (true) {
-        int cur = h_key[hs];
+    unsigned hs = ((unsigned)key * 2654435761u) >> 23;
+    for (int probe = 0; probe < kHash; ++probe) {
+        const int cur = h_key[hs];
         if (cur == key) return (int)hs;
         if (cur == -1) {
             if (*fill >= kHashFill) return -1;
-            int old = atomicCAS(&h_key[hs], -1, key);
+            const int old = atomicCAS(&h_key[hs], -1, key);
             if (old == -1) { atomicAdd(fill, 1); return (int)hs; }
             if (old == key) return (int)hs;
         }
         hs = (hs + 1) & (kHash - 1);
     }
+    return -1;
 }
 
-__device__ __forceinline__ int hash_find(const int* h_key, int key) {
-    unsigned hs = ((unsigned)key * 2654435761u) & (kHash - 1);
-    while (h_key[hs] != key) hs = (hs + 1) & (kHash - 1);
-    return (int)hs;
-}
-
-__global__ void __launch_bounds__(256) k_lists(const int* __restrict__ alist, const int* __restrict__ count,
-                                               int* __restrict__ cursor, const Box* __restrict__ box,
-                                               const int* __restrict__ flags, const int* __restrict__ sec_cnt,
-                                               const int* __restrict__ sec, int* __restrict__ cmp_cnt,
-                                               int* __restrict__ cmp, int* __restrict__ err) {
-    __shared__ int h_key[kHash];
-    __shared__ int h_min[kHash];
-    __shared__ int s_cand[kCandChunk];
-    __shared__ int s_sec[kCmpCap];
-    __shared__ int s_off[kCmpCap + 1];
-    __shared__ int s_tmp[256];
-    __shared__ int s_slot, s_fill, s_bad;
-    const int t = threadIdx.x;
-    const int total = *count;  // written by k_tally (or the host) before this kernel
-    constexpr int kChunk = 4;  // items per cursor atomic: the list work of a grain is light
-    for (int item = take_item(cursor, &s_slot, -1, kChunk); item < total;
-         item = take_item(cursor, &s_slot, item, kChunk)) {
-        __syncthreads();  // the previous item's shared state is free
-        const int g = alist[item];
-        const Box bg = box[g];
-        const int ns = sec_cnt[g];
+__global__ void __launch_bounds__(64) k_lists(const int* __restrict__ list, const int* __restrict__ count,
+                                              const Box* __restrict__ box, const int* __restrict__ flags,
+                                              const int* __restrict__ sec_cnt, const int* __restrict__ sec,
+                                              int* __restrict__ cmp_cnt, int* __restrict__ cmp, int* __restrict__ err) {
+    __shared__ int h_key[kHash], h_min[kHash];
+    __shared__ int s_sec[kCmpCap], s_off[kCmpCap + 1];
+    __shared__ int s_fill;
+    constexpr int kU = 4;  // candidates per lane and pass
+    const int lane = (int)threadIdx.x;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const int total = sload(count);
+    for (int item = (int)blockIdx.x; item < total; item += (int)gridDim.x) {
+        wave_lds_sync();  // the previous grain's shared state is free
+        const int g = sload(list + item);
+        const Box bg = sload_box(box + g);
+        const int ns = sload(sec_cnt + g);
         int* out = cmp + (size_t)g * kCmpCap;
-        for (int k = t; k < kHash; k += blockDim.x) { h_key[k] = -1; h_min[k] = 0x7fffffff; }
-        if (t == 0) { s_fill = 0; s_bad = 0; }
-        int ex = 0, len = 0;
-        if (t < ns) {
-            int nb = sec[(size_t)g * kCmpCap + t];
-            s_sec[t] = nb;
-            ex = (flags[nb] & kExists) ? 1 : 0;
-            len = sec_cnt[nb];
+        for (int k = lane; k < kHash; k += 64) { h_key[k] = -1; h_min[k] = 0x7fffffff; }
+        if (lane == 0) s_fill = 0;
+        wave_lds_sync();
+        // part 1: existing entries of the previous list, in order (box.cpp:1038-1041), and the offset of
+        // each entry's candidates
+        int written = 0, ntot = 0;
+        bool bad = false;
+        for (int e0 = 0; e0 < ns; e0 += 64) {
+            const int e = e0 + lane;
+            int nb = 0, len = 0;
+            bool ex = false;
+            if (e < ns) {
+                nb = sec[(size_t)g * kCmpCap + e];
+                ex = (flags[nb] & kExists) != 0;
+                len = sec_cnt[nb];
+                s_sec[e] = nb;
+            }
+            int x = len;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int y = __shfl_up(x, d);
+                if (lane >= d) x += y;
+            }
+            if (e < ns) s_off[e] = ntot + x - len;
+            ntot += __builtin_amdgcn_readlane(x, 63);
+            const unsigned long long m = __ballot(ex);
+            if (ex) {
+                out[written + __popcll(m & below)] = nb;
+                const int hs = hash_insert(h_key, &s_fill, nb);
+                if (hs >= 0) h_min[hs] = -1;  // already in the list
+                else bad = true;
+            }
+            written += __popcll(m);
         }
-        int ntot;
-        int koff = block_scan(len, s_tmp, &ntot);   // candidate offset of entry t
-        if (t < ns) s_off[t] = koff;
-        if (t == 0) s_off[ns] = ntot;
-        int n1;
-        int pos1 = block_scan(ex, s_tmp, &n1);      // rank among existing entries
-        // part 1: existing entries of the previous list, in order (box.cpp:1038-1041)
-        if (t < ns && ex) {
-            out[pos1] = s_sec[t];
-            int hs = hash_insert(h_key, &s_fill, s_sec[t]);
-            if (hs >= 0) h_min[hs] = -1;  // already in the list
-            else s_bad = 1;
-        }
-        __syncthreads();
-        // candidates, flattened in (entry, entry's entry) order (box.cpp:1042-1048), staged in
-        // chunks; pass 0 records each id's first valid index, pass 1 compacts first occurrences
-        int written = n1;
-        bool over = false;
-        for (int pass = 0; pass < 2; ++pass) {
-            for (int c0 = 0; c0 < ntot; c0 += kCandChunk) {
-                const int cl = min(kCandChunk, ntot - c0);
-                for (int a = 0; a < ns; ++a) {
-                    const int lo = max(s_off[a], c0), hi = min(s_off[a + 1], c0 + cl);
-                    const int* snb = sec + (size_t)s_sec[a] * kCmpCap - s_off[a];
-                    for (int k = lo + t; k < hi; k += blockDim.x) s_cand[k - c0] = snb[k];
+        if (lane == 0) s_off[ns] = ntot;
+        wave_lds_sync();
+        // candidates in (entry, entry's entry) order (box.cpp:1042-1048)
+        for (int c0 = 0; c0 < ntot; c0 += 64 * kU) {
+            int c[kU], hs[kU], f[kU];
+            Box bc[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const int q = c0 + 64 * u + lane;
+                c[u] = -1;
+                if (q < ntot) {
+                    int lo = 0, hi = ns;  // the entry a with s_off[a] <= q < s_off[a + 1]
+                    while (hi - lo > 1) {
+                        const int mid = (lo + hi) >> 1;
+                        if (s_off[mid] <= q) lo = mid;
+                        else hi = mid;
+                    }
+                    c[u] = sec[(size_t)s_sec[lo] * kCmpCap + (q - s_off[lo])];
                 }
-                __syncthreads();
-                for (int q = t; q < cl; q += blockDim.x) {
-                    int c = s_cand[q];
-                    bool valid = (flags[c] & kExists) && c != g && c != 0;
-                    if (valid) {
-                        Box bc = box[c];
-                        valid = !(bg.x0 > bc.x0 + bc.n || bg.x0 + bg.n < bc.x0 || bg.y0 > bc.y0 + bc.n ||
-                                  bg.y0 + bg.n < bc.y0);
-                    }
-                    if (!valid) { s_cand[q] = -1; continue; }
-                    if (pass == 0) {
-                        int hs = hash_insert(h_key, &s_fill, c);
-                        if (hs >= 0) atomicMin(&h_min[hs], c0 + q);  // stays -1 for part-1 entries
-                        else s_bad = 1;
-                    }
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                f[u] = 0;
+                bc[u] = Box{0, 0, 0, 0};
+                if (c[u] > 0 && c[u] != g) { f[u] = flags[c[u]]; bc[u] = box[c[u]]; }
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const bool valid = (f[u] & kExists) && !(bg.x0 > bc[u].x0 + bc[u].n || bg.x0 + bg.n < bc[u].x0 ||
+                                                         bg.y0 > bc[u].y0 + bc[u].n || bg.y0 + bg.n < bc[u].y0);
+                hs[u] = -1;
+                if (valid) {
+                    hs[u] = hash_insert(h_key, &s_fill, c[u]);
+                    if (hs[u] >= 0) atomicMin(&h_min[hs[u]], c0 + 64 * u + lane);  // stays -1 for part-1 entries
+                    else bad = true;
                 }
-                __syncthreads();
-                if (pass == 1 && !s_bad) {
-                    // ordered compaction of first occurrences (box.cpp:1050-1066)
-                    const int per = (cl + (int)blockDim.x - 1) / (int)blockDim.x;
-                    const int q0 = t * per, q1 = min(cl, q0 + per);
-                    int keep = 0;
-                    for (int q = q0; q < q1; ++q) {
-                        int c = s_cand[q];
-                        if (c >= 0 && h_min[hash_find(h_key, c)] == c0 + q) keep++;
-                    }
-                    int nk;
-                    int w = written + block_scan(keep, s_tmp, &nk);
-                    for (int q = q0; q < q1; ++q) {
-                        int c = s_cand[q];
-                        if (c >= 0 && h_min[hash_find(h_key, c)] == c0 + q) {
-                            if (w < kCmpCap) out[w] = c; else over = true;
-                            w++;
-                        }
-                    }
-                    written += nk;
-                }
-                __syncthreads();
+            }
+            wave_lds_sync();
+            // ordered compaction of first occurrences (box.cpp:1050-1066)
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const bool keep = hs[u] >= 0 && h_min[hs[u]] == c0 + 64 * u + lane;
+                const unsigned long long m = __ballot(keep);
+                const int at = written + __popcll(m & below);
+                if (keep && at < kCmpCap) out[at] = c[u];
+                written += __popcll(m);
             }
         }
-        if (over) err[g] = kErrCmpCap;
-        if (t == 0) {
-            if (written > kCmpCap || s_bad) err[g] = kErrCmpCap;
+        const bool over = __ballot(bad) != 0ull || written > kCmpCap;
+        if (lane == 0) {
+            if (over) err[g] = kErrCmpCap;
             cmp_cnt[g] = min(written, kCmpCap);
         }
     }

@@ -236,121 +236,122 @@ __global__ void __launch_bounds__(256) k_compare(LevelArgs<T> A) {
         const int g = item_grain(A.it, item, &bucket, &pos);
         const Box b = sload_box(A.box + g);
         const int n = b.n, W = (n + 63) >> 6, rb = (n + kRows - 1) / kRows;
-        if (blk >= rb * W) continue;
-        const int xc = blk / rb, rblk = blk - xc * rb;
-        const int r0 = rblk * kRows, rows = min(kRows, n - r0), x = xc * 64 + lane;
-        const bool on = x < n;
-        const long long o = sload(A.off + g);
-        const bool cmp_on = COARSEN ? ((sload(A.O.flags + g) & kExists) != 0) : true;
-        const int cnt = cmp_on ? sload(A.cmp_cnt + g) : 0;
-        T own[kRows], mx[kRows];
-        int id[kRows];
+        for (int block = blk; block < rb * W; block += A.blocks) {
+            const int xc = block / rb, rblk = block - xc * rb;
+            const int r0 = rblk * kRows, rows = min(kRows, n - r0), x = xc * 64 + lane;
+            const bool on = x < n;
+            const long long o = sload(A.off + g);
+            const bool cmp_on = COARSEN ? ((sload(A.O.flags + g) & kExists) != 0) : true;
+            const int cnt = cmp_on ? sload(A.cmp_cnt + g) : 0;
+            T own[kRows], mx[kRows];
+            int id[kRows];
 #pragma unroll
-        for (int r = 0; r < kRows; ++r) {
-            own[r] = (on && r < rows) ? A.tilde[o + (long long)(r0 + r) * n + x] : T(0);
-            mx[r] = T(-1.0);
-            id[r] = -1;
-        }
-        for (int e0 = 0; e0 < cnt; e0 += 64) {
-            const bool have = e0 + lane < cnt;
-            int eid = 0, ex = 0, ey = 0, en = 0;
-            long long eo = 0;
-            if (have) {
-                eid = A.cmp[(size_t)g * kCmpCap + e0 + lane];
-                const Box q = A.box[eid];
-                ex = q.x0 - b.x0;
-                ey = q.y0 - b.y0;
-                en = q.n;
-                eo = A.off[eid];
+            for (int r = 0; r < kRows; ++r) {
+                own[r] = (on && r < rows) ? A.tilde[o + (long long)(r0 + r) * n + x] : T(0);
+                mx[r] = T(-1.0);
+                id[r] = -1;
             }
-            if (blk == 0) {  // pixels of the whole box that the entry covers (a statistic)
-                const int ox = min(n, ex + en) - max(0, ex), oy = min(n, ey + en) - max(0, ey);
-                if (have && ox > 0 && oy > 0) hits += (unsigned long long)ox * (unsigned long long)oy;
-            }
-            unsigned long long todo = __ballot(have && ey < r0 + rows && ey + en > r0 && ex < xc * 64 + 64 && ex + en > xc * 64);
-            while (todo) {
-                constexpr int kK = 2;
-                T v[kK][kRows];
-                int sid[kK];
+            for (int e0 = 0; e0 < cnt; e0 += 64) {
+                const bool have = e0 + lane < cnt;
+                int eid = 0, ex = 0, ey = 0, en = 0;
+                long long eo = 0;
+                if (have) {
+                    eid = A.cmp[(size_t)g * kCmpCap + e0 + lane];
+                    const Box q = A.box[eid];
+                    ex = q.x0 - b.x0;
+                    ey = q.y0 - b.y0;
+                    en = q.n;
+                    eo = A.off[eid];
+                }
+                if (block == 0) {  // pixels of the whole box that the entry covers (a statistic)
+                    const int ox = min(n, ex + en) - max(0, ex), oy = min(n, ey + en) - max(0, ey);
+                    if (have && ox > 0 && oy > 0) hits += (unsigned long long)ox * (unsigned long long)oy;
+                }
+                unsigned long long todo = __ballot(have && ey < r0 + rows && ey + en > r0 && ex < xc * 64 + 64 && ex + en > xc * 64);
+                while (todo) {
+                    constexpr int kK = 2;
+                    T v[kK][kRows];
+                    int sid[kK];
 #pragma unroll
-                for (int u = 0; u < kK; ++u) {
+                    for (int u = 0; u < kK; ++u) {
 #pragma unroll
-                    for (int r = 0; r < kRows; ++r) v[u][r] = T(-1.0);  // no value beats the initial maximum
-                    if (u == 0 || todo) {
-                        const int k = (int)__builtin_ctzll(todo);
-                        todo &= todo - 1ull;
-                        sid[u] = __builtin_amdgcn_readlane(eid, k);
-                        const int dx = __builtin_amdgcn_readlane(ex, k), dy = __builtin_amdgcn_readlane(ey, k);
-                        const int nk = __builtin_amdgcn_readlane(en, k);
-                        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)eo, k);
-                        const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)((unsigned long long)eo >> 32), k);
-                        const T* src = A.tilde + (long long)(((unsigned long long)hi << 32) | lo);
-                        const int y0 = r0 - dy;  // the block's first row in the entry's box
-                        if (on && (unsigned)(x - dx) < (unsigned)nk) {
-                            if (y0 >= 0 && y0 + kRows <= nk) {
-                                const T* p = src + (y0 * nk + (x - dx));
+                        for (int r = 0; r < kRows; ++r) v[u][r] = T(-1.0);  // no value beats the initial maximum
+                        if (u == 0 || todo) {
+                            const int k = (int)__builtin_ctzll(todo);
+                            todo &= todo - 1ull;
+                            sid[u] = __builtin_amdgcn_readlane(eid, k);
+                            const int dx = __builtin_amdgcn_readlane(ex, k), dy = __builtin_amdgcn_readlane(ey, k);
+                            const int nk = __builtin_amdgcn_readlane(en, k);
+                            const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)eo, k);
+                            const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)((unsigned long long)eo >> 32), k);
+                            const T* src = A.tilde + (long long)(((unsigned long long)hi << 32) | lo);
+                            const int y0 = r0 - dy;  // the block's first row in the entry's box
+                            if (on && (unsigned)(x - dx) < (unsigned)nk) {
+                                if (y0 >= 0 && y0 + kRows <= nk) {
+                                    const T* p = src + (y0 * nk + (x - dx));
 #pragma unroll
-                                for (int r = 0; r < kRows; ++r) v[u][r] = p[r * nk];
-                            } else {
+                                    for (int r = 0; r < kRows; ++r) v[u][r] = p[r * nk];
+                                } else {
 #pragma unroll
-                                for (int r = 0; r < kRows; ++r)
-                                    if ((unsigned)(y0 + r) < (unsigned)nk) v[u][r] = src[(y0 + r) * nk + (x - dx)];
+                                    for (int r = 0; r < kRows; ++r)
+                                        if ((unsigned)(y0 + r) < (unsigned)nk) v[u][r] = src[(y0 + r) * nk + (x - dx)];
+                                }
                             }
+                        } else {
+                            sid[u] = 0;
                         }
-                    } else {
-                        sid[u] = 0;
                     }
+#pragma unroll
+                    for (int u = 0; u < kK; ++u)
+#pragma unroll
+                        for (int r = 0; r < kRows; ++r)
+                            if (v[u][r] > mx[r]) { mx[r] = v[u][r]; id[r] = sid[u]; }
                 }
-#pragma unroll
-                for (int u = 0; u < kK; ++u)
-#pragma unroll
-                    for (int r = 0; r < kRows; ++r)
-                        if (v[u][r] > mx[r]) { mx[r] = v[u][r]; id[r] = sid[u]; }
             }
-        }
-        // per pixel: the wall as grain 0, IDLocal, the set comparison, the sign bits
-        const bool bnd = at_wall(b, G) && cmp_on;
-        const double band = 0.7 * G.delta;
-        const int nprev = sload(A.n_prev + g);
-        const long long np = (long long)nprev * nprev;
-        const long long op = sload(A.off_prev + g);
-        unsigned long long row_ge = 0, row_gt = 0;  // of the block's row `lane`
-        unsigned col_ge = 0, col_gt = 0;            // of the lane's column, bit = row
+            // per pixel: the wall as grain 0, IDLocal, the set comparison, the sign bits
+            const bool bnd = at_wall(b, G) && cmp_on;
+            const double band = 0.7 * G.delta;
+            const int nprev = sload(A.n_prev + g);
+            const long long np = (long long)nprev * nprev;
+            const long long op = sload(A.off_prev + g);
+            unsigned long long row_ge = 0, row_gt = 0;  // of the block's row `lane`
+            unsigned col_ge = 0, col_gt = 0;            // of the lane's column, bit = row
 #pragma unroll
-        for (int r = 0; r < kRows; ++r) {
-            if (r < rows) {
-                const long long p = (long long)(r0 + r) * n + x;
-                T c = T(-1.0);
-                if (on) {
-                    T m = mx[r];
-                    int idt = id[r];
-                    if (bnd) {
-                        const double dist = wall_distance(b.y0 + r0 + r, b.x0 + x, G);
-                        if ((T)(dist * G.h) > m) { m = (T)(dist * G.h); idt = 0; }
+            for (int r = 0; r < kRows; ++r) {
+                if (r < rows) {
+                    const long long p = (long long)(r0 + r) * n + x;
+                    T c = T(-1.0);
+                    if (on) {
+                        T m = mx[r];
+                        int idt = id[r];
+                        if (bnd) {
+                            const double dist = wall_distance(b.y0 + r0 + r, b.x0 + x, G);
+                            if ((T)(dist * G.h) > m) { m = (T)(dist * G.h); idt = 0; }
+                        }
+                        const T tv = own[r];
+                        c = COARSEN ? tv : ((fabs((double)tv) < band) ? (T)(0.5 * ((double)tv - (double)m)) : tv);
+                        A.cfield[o + p] = c;
+                        A.idl_new[o + p] = (idt >= 0) ? (uint32_t)idt : ((p < np) ? A.idl_old[op + p] : 0u);
+                        if (A.rec_s) {
+                            A.rec_s[o + p] = c;
+                            A.rec_win[o + p] = idt;
+                        }
                     }
-                    const T tv = own[r];
-                    c = COARSEN ? tv : ((fabs((double)tv) < band) ? (T)(0.5 * ((double)tv - (double)m)) : tv);
-                    A.cfield[o + p] = c;
-                    A.idl_new[o + p] = (idt >= 0) ? (uint32_t)idt : ((p < np) ? A.idl_old[op + p] : 0u);
-                    if (A.rec_s) {
-                        A.rec_s[o + p] = c;
-                        A.rec_win[o + p] = idt;
-                    }
+                    const unsigned long long mge = __ballot(on && c >= T(0)), mgt = __ballot(on && c > T(0));
+                    if (lane == r) { row_ge = mge; row_gt = mgt; }
+                    col_ge |= (on && c >= T(0)) ? 1u << r : 0u;
+                    col_gt |= (on && c > T(0)) ? 1u << r : 0u;
                 }
-                const unsigned long long mge = __ballot(on && c >= T(0)), mgt = __ballot(on && c > T(0));
-                if (lane == r) { row_ge = mge; row_gt = mgt; }
-                col_ge |= (on && c >= T(0)) ? 1u << r : 0u;
-                col_gt |= (on && c > T(0)) ? 1u << r : 0u;
             }
-        }
-        unsigned long long* bits = A.bits + (o >> 3);
-        if (lane < rows) {
-            bits[kRowGe * A.plane + (long long)(r0 + lane) * W + xc] = row_ge;
-            bits[kRowGt * A.plane + (long long)(r0 + lane) * W + xc] = row_gt;
-        }
-        if (on) {
-            ((unsigned char*)(bits + kColGe * A.plane + (long long)x * W))[rblk] = (unsigned char)col_ge;
-            ((unsigned char*)(bits + kColGt * A.plane + (long long)x * W))[rblk] = (unsigned char)col_gt;
+            unsigned long long* bits = A.bits + (o >> 3);
+            if (lane < rows) {
+                bits[kRowGe * A.plane + (long long)(r0 + lane) * W + xc] = row_ge;
+                bits[kRowGt * A.plane + (long long)(r0 + lane) * W + xc] = row_gt;
+            }
+            if (on) {
+                ((unsigned char*)(bits + kColGe * A.plane + (long long)x * W))[rblk] = (unsigned char)col_ge;
+                ((unsigned char*)(bits + kColGt * A.plane + (long long)x * W))[rblk] = (unsigned char)col_gt;
+            }
         }
     }
     // one addition per wave that met a grain's first block, spread over the slots
