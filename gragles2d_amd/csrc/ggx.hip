@@ -463,12 +463,23 @@ std::vector<std::pair<int, int>> level_groups(const ggx_ctx* ctx) {
     return R;
 }
 
+// Every live grain as one launch's items, in the spatial order of the list.
+Items all_items(const ggx_ctx* ctx) {
+    Items it = bucket_items(ctx, 0, 0);
+    it.lists = ctx->alist; it.total = &ctx->sched->all_total;
+    return it;
+}
+
+// One launch over grains of every side (A.nb: the largest).  Six waves per grain, the blocks of a
+// common box; more, which leaves a wave fewer blocks to loop over, where that few would not fill
+// the chip.  Many more workgroups than fit at a time: their sizes differ, and the ones that wait
+// even them out (with 8 per CU, of which 6 fit, the last two ran alone).
 template <class T>
 int launch_compare(const ggx_ctx* ctx, hipStream_t st, LevelArgs<T>& A, int items, bool coarsen) {
-    // a small network's launch holds boxes of every side: 32 waves per grain, which larger boxes loop over
-    A.blocks = std::min(32, ((A.nb + kRows - 1) / kRows) * ((A.nb + 63) / 64));
+    const int full = ((A.nb + kRows - 1) / kRows) * ((A.nb + 63) / 64);
+    A.blocks = std::min({32, full, std::max(6, ctx->cu_count * 64 / std::max(1, items))});
     const long long wgs = ((long long)items * A.blocks + 3) / 4;
-    const int grid = (int)std::max<long long>(1, std::min<long long>(wgs, ctx->cu_count * 8));
+    const int grid = (int)std::max<long long>(1, std::min<long long>(wgs, ctx->cu_count * 128));
     if (coarsen) hipLaunchKernelGGL((k_compare<T, true>), dim3(grid), dim3(256), 0, st, A);
     else hipLaunchKernelGGL((k_compare<T, false>), dim3(grid), dim3(256), 0, st, A);
     return GGX_OK;
@@ -684,19 +695,19 @@ int launch_step(ggx_ctx* ctx, bool timed, bool record = false) {
         for (int b = r.first; b <= r.second; ++b) c += counts[b];
         return c;
     };
-    for (int phase = 0; phase < 3; ++phase) {
-        for (auto r : groups) {
-            // k_compare has no size-dependent resources: a small network takes one launch of it
-            if (phase == 0 && ctx->merge_bucket >= 0) {
-                if (r.first > 0) continue;
-                r.second = ctx->nbuckets - 1;
-            }
+    A.it = all_items(ctx);
+    A.nb = ctx->edges[ctx->nbuckets - 1];
+    if (const int k = items({0, ctx->nbuckets - 1})) {
+        const int rc = launch_compare<T>(ctx, st, A, k, false);
+        if (rc) return rc;
+    }
+    for (int phase = 1; phase < 3; ++phase) {
+        for (const auto& r : groups) {
             const int k = items(r);
             if (k == 0) continue;
             level_items(ctx, A, r.first, r.second);
             int rc = GGX_OK;
-            if (phase == 0) rc = launch_compare<T>(ctx, st, A, k, false);
-            else if (phase == 1) { rc = launch_contour<T>(ctx, st, A, k, false); all += k; }
+            if (phase == 1) { rc = launch_contour<T>(ctx, st, A, k, false); all += k; }
             else rc = launch_redist<T>(ctx, st, A, k);
             if (rc) return rc;
         }
@@ -958,14 +969,17 @@ int coarsen(ggx_ctx* ctx, int present) {
     LevelArgs<T> A = level_args<T>(ctx);
     A.cmp_cnt = ctx->sec_cnt; A.cmp = ctx->sec;  // the last step's lists
     A.cfield = (T*)ctx->P[ctx->cur];
-    for (int phase = 0; phase < 2; ++phase)
-        for (const auto& r : level_groups(ctx)) {
-            int k = 0;
-            for (int b = r.first; b <= r.second; ++b) k += (int)bl[(size_t)b].size();
-            if (k == 0) continue;
-            level_items(ctx, A, r.first, r.second);
-            if ((rc = phase == 0 ? launch_compare<T>(ctx, st, A, k, true) : launch_contour<T>(ctx, st, A, k, true))) return rc;
-        }
+    if (!list.empty()) {
+        level_items(ctx, A, 0, ctx->nbuckets - 1);
+        if ((rc = launch_compare<T>(ctx, st, A, (int)list.size(), true))) return rc;
+    }
+    for (const auto& r : level_groups(ctx)) {
+        int k = 0;
+        for (int b = r.first; b <= r.second; ++b) k += (int)bl[(size_t)b].size();
+        if (k == 0) continue;
+        level_items(ctx, A, r.first, r.second);
+        if ((rc = launch_contour<T>(ctx, st, A, k, true))) return rc;
+    }
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
     ctx->icur ^= 1;
