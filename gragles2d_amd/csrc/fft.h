@@ -1,12 +1,13 @@
-// fft.h -- batched 2-D convolution of square boxes by mixed-radix FFT (gfx950).
+// fft.h -- 2-D convolution of square boxes by transforms (gfx950): the step's by mixed-radix FFT, the
+// standalone batch's by products with the real transform matrix on the matrix cores.
 //
 // LSbox::convolutionGeneratorFFTW (box.cpp:622-695): phi~ = IDFT2( G . DFT2(phi) ) with the
 // real, even symbol G of ConvolutionMode 0 (Laplace, box.cpp:648-659), 1 (Laplace with the
 // Richardson extrapolation, 660-673) or 2 (Gaussian, 674-688).  G carries the 1/n^2 of the
 // unnormalised c2r transform and uses the global grid size R in nsq (636-637).
 //
-// One 256-lane workgroup per box, exact n (no padding to a friendly size), three phases
-// separated by workgroup barriers:
+// The step (k_conv_fft): one 256-lane workgroup per box, exact n (no padding to a friendly size),
+// three phases separated by workgroup barriers:
 //   1. rows     each wave takes a pair of rows (2p, 2p+1), transforms z = row_2p + i row_2p+1
 //               as one complex line and splits the result into the two half spectra
 //               X[k] = (Z[k] + conj Z[n-k]) / 2, Y[k] = (Z[k] - conj Z[n-k]) / 2i, k <= n/2;
@@ -60,10 +61,7 @@ __host__ __device__ inline long long fft_lds(int nb, bool spectrum_in_lds) {
 constexpr __host__ __device__ inline long long fft_slot(int nb) { return (long long)nb * (nb / 2 + 1); }
 
 // (cos 2 pi t / n, sin 2 pi t / n) for t < n, every side n of [nmin, nmax]; one workgroup per n.
-// Workgroup 0 also clears *bad when given (the error flag of a batch call).
-__global__ void __launch_bounds__(256) k_fft_twiddles(double2* __restrict__ tw, int nmin, int nmax,
-                                                      int* __restrict__ bad) {
-    if (bad && blockIdx.x == 0 && threadIdx.x == 0) *bad = 0;
+__global__ void __launch_bounds__(256) k_fft_twiddles(double2* __restrict__ tw, int nmin, int nmax) {
     const int n = nmin + (int)blockIdx.x;
     if (n > nmax) return;
     for (int t = threadIdx.x; t < n; t += blockDim.x) {
@@ -260,30 +258,208 @@ __global__ void __launch_bounds__(256) k_conv_fft(const int* __restrict__ list, 
     }
 }
 
-// The standalone batch (ggx_convolve_boxes): box b has side ns[b] and starts at offs[b] in
-// src and dst.  Workgroup i takes boxes i, i + grid, ...; this launch handles the boxes of
-// side in (nlo, nhi].
-// A box whose side is outside [1, nmax] is left alone and sets *bad (the host reports it).
-template <bool LDS>
-__global__ void __launch_bounds__(256) k_conv_fft_batch(int count, const int* __restrict__ ns,
-                                                        const int64_t* __restrict__ offs,
-                                                        const double* __restrict__ src, double* __restrict__ dst,
-                                                        const double2* __restrict__ tw, FftSymbol sy, int nb, int nlo,
-                                                        int nhi, int nmax, double2* __restrict__ work,
-                                                        int* __restrict__ bad) {
-    HIP_DYNAMIC_SHARED(unsigned char, smem)
-    double2* W = (double2*)smem;
-    double2* L = W + nb;
-    double2* H = LDS ? L + 2 * kFftWaves * nb : work + (size_t)blockIdx.x * (size_t)fft_slot(nb);
-    for (int b = (int)blockIdx.x; b < count; b += (int)gridDim.x) {
-        const int n = ns[b];
-        if (n < 1 || n > nmax) {
-            if (threadIdx.x == 0) atomicOr(bad, 1);
+// ------------------------------------------------------------------------------------------
+// The standalone batch (ggx_convolve_boxes): box b has side ns[b] and starts at offs[b] in src and
+// dst.  The symbol is real and even in both directions, so the real transform with H[j][k] =
+// cas(2 pi j k / n) = cos + sin diagonalises the convolution as the complex one does (H symmetric,
+// H H = n I; Hartley, Proc. IRE 30, 1942):  phi~ = H ( G . (H phi H) ) H.  Four products with H per box, on the matrix cores
+// in FP64 and without complex arithmetic, half spectra or a workspace:
+//   k_box_rows     dst = src H   one workgroup per 16 rows
+//   k_box_columns  dst = H (G . (H dst))   one workgroup per 16 columns
+//   k_box_rows     dst = dst H
+// each in place on its strip, which lies in LDS.  H is not stored: its elements are read from the n
+// values cas(2 pi t / n) in LDS, the index j k mod n of a lane's next element by one addition.  An
+// FP64 product of 16 x 16 x 4 keeps a SIMD's matrix core for 64 cycles, in which the LDS has room
+// for far more than the two reads it needs.  6000 boxes of side 16 to 128 take 0.45, 0.9 and 0.45 ms
+// (products with the sides rounded up to 16: 0.12 ms each; the rest is each strip's chain of load,
+// table, product and store at 16 waves per CU), 96 of side 130 to 256 take 0.36 ms.  The FFT with a
+// workgroup per box took 7.5 ms, bound by its p-term sums, and 29 ms, bound by its eight half-spectrum
+// slots.  The Richardson symbol's two 40th powers are a third of k_box_columns with pow().
+// ------------------------------------------------------------------------------------------
+struct BoxBatch {
+    int count, strips;   // boxes; strips of 16 lines of the largest side allowed
+    const int* ns;
+    const int64_t* offs;
+    int nmax;            // a box whose side is outside [1, nmax] is left alone and sets *bad
+    int* bad;
+};
+
+constexpr int kStripPitch = 17;   // doubles per line of a strip: 16 and one against bank conflicts
+
+constexpr __host__ __device__ inline int strip_lines(int n) { return (n + 3) & ~3; }
+constexpr __host__ __device__ inline long long box_rows_lds(int n) { return 8LL * (strip_lines(n) * kStripPitch + n); }
+constexpr __host__ __device__ inline long long box_columns_lds(int n) { return 8LL * (2 * strip_lines(n) * kStripPitch + 2 * n); }
+
+// K tiles of a strip product, tiles t0, t0 + 4, ...: H times the strip (ROWS: the strip, whose lines
+// are H's rows, times H).  s_in: strip_lines(n) lines of 16 values, zero beyond n.
+template <bool ROWS, int K, class Out>
+__device__ __forceinline__ void strip_tiles(int n, const double* s_cas, const double* s_in, int t0, Out out) {
+    using V = typename Mma<double>::V;
+    const int lane = (int)(threadIdx.x & 63), l = lane & 15, q = lane >> 4;
+    V sum[K];
+    int at[K], step[K];
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+        const int i = ((t0 + 4 * u) * 16 + l) % n;
+        sum[u] = V{0.0, 0.0, 0.0, 0.0};
+        at[u] = i * q % n;
+        step[u] = 4 * i % n;
+    }
+    const double* line = s_in + q * kStripPitch + l;
+    auto products = [&](V* acc, int k) {  // lines k .. k + 3
+        const double x = line[k * kStripPitch];
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            const double h = s_cas[at[u]];
+            acc[u] = ROWS ? Mma<double>::run(x, h, acc[u]) : Mma<double>::run(h, x, acc[u]);
+            at[u] += step[u];
+            if (at[u] >= n) at[u] -= n;
+        }
+    };
+    // eight lines' products are summed by themselves before they join the total: rounding errors grow
+    // with the longer of the two chains (0.8 to 0.95 of the FFT's error; one chain: up to 2.7 times it)
+    int k = 0;
+    for (; k + 8 <= n; k += 8) {
+        V acc[K];
+#pragma unroll
+        for (int u = 0; u < K; ++u) acc[u] = V{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int d = 0; d < 8; d += 4) products(acc, k + d);
+#pragma unroll
+        for (int u = 0; u < K; ++u) sum[u] += acc[u];
+    }
+    for (; k < n; k += 4) products(sum, k);
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = Mma<double>::row(q, r);
+            if (ROWS) out(row, (t0 + 4 * u) * 16 + l, sum[u][r]);
+            else out((t0 + 4 * u) * 16 + row, l, sum[u][r]);
+        }
+}
+
+// All tiles of a strip product over the workgroup's four waves; out(row, column, value) of each.
+// `turn` moves the tiles on by a wave per strip: a box of five tiles gives one wave two of them.
+template <bool ROWS, class Out>
+__device__ __forceinline__ void strip_product(int n, const double* s_cas, const double* s_in, int turn, Out out) {
+    const int tiles = (n + 15) >> 4;
+    int t0 = __builtin_amdgcn_readfirstlane((int)((threadIdx.x >> 6) + (unsigned)turn) & 3);
+    while (t0 < tiles) {
+        const int left = (tiles - t0 + 3) >> 2;
+        if (left >= 4) strip_tiles<ROWS, 4>(n, s_cas, s_in, t0, out);
+        else if (left == 3) strip_tiles<ROWS, 3>(n, s_cas, s_in, t0, out);
+        else if (left == 2) strip_tiles<ROWS, 2>(n, s_cas, s_in, t0, out);
+        else strip_tiles<ROWS, 1>(n, s_cas, s_in, t0, out);
+        t0 += 16;
+    }
+}
+
+// The box and strip of a work item; false: no such strip.
+__device__ __forceinline__ bool box_strip(const BoxBatch& B, long long item, int* n, int64_t* o, int* line0) {
+    const int b = (int)(item / B.strips);
+    *line0 = (int)(item - (long long)b * B.strips) * 16;
+    *n = sload(B.ns + b);
+    *o = sload(B.offs + b);
+    return *n >= 1 && *n <= B.nmax && *line0 < *n;
+}
+
+// x^40 by squarings with their rounding errors carried along (l: what h lacks).
+__device__ __forceinline__ double power40(double x) {
+    double h = x, l = 0.0, h8 = 0.0, l8 = 0.0;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        const double s = h * h;
+        l = fma(h, h, -s) + 2.0 * h * l;
+        h = s;
+        if (k == 2) { h8 = h; l8 = l; }
+    }
+    const double p = h * h8;
+    return p < 1e300 ? fma(h, h8, fma(h, l8, l * h8)) : p;  // not past an overflow
+}
+
+// fft_symbol with cos(2 pi t / n) from s_cos[t].
+__device__ __forceinline__ double box_symbol(int j, int i, int n, const double* s_cos, const FftSymbol& sy) {
+    const double kPi = 3.14159265358979323846;
+    const double n_nsq = (double)(n * n);
+    if (sy.mode == 2) {
+        const int i2 = min(i, n - i), j2 = min(j, n - j);
+        return exp(-sqrt(2 / kPi) * (double)(i2 * i2 + j2 * j2) * 4.0 * sy.dt * sy.nsq / n_nsq * kPi * kPi) / n_nsq;
+    }
+    const double g = 2.0 * (2.0 - s_cos[i] - s_cos[j]) * sy.nsq;
+    if (sy.mode == 0) return 1.0 / (1.0 + (sy.dt * g)) / n_nsq;
+    return (4.0 / power40(1 + 1.5 * sy.dt / 40 * g) - 1.0 / power40(1 + 3.0 * sy.dt / 40 * g)) / 3.0 / n_nsq;
+}
+
+// dst = src H by strips of 16 rows (src may be dst).  first: clears *bad.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_box_rows(BoxBatch B, const double* src, double* dst, int first) {
+    HIP_DYNAMIC_SHARED(double, s_box)
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (first && blockIdx.x == 0 && tid == 0) *B.bad = 0;
+    const long long items = (long long)B.count * B.strips;
+    for (long long item = blockIdx.x; item < items; item += gridDim.x) {
+        int n, r0;
+        int64_t o;
+        if (!box_strip(B, item, &n, &o, &r0)) continue;
+        double* s_in = s_box;
+        double* s_cas = s_box + strip_lines(n) * kStripPitch;
+        for (int t = tid; t < n; t += 256) {
+            double s, c;
+            sincospi(2.0 * (double)t / (double)n, &s, &c);
+            s_cas[t] = c + s;
+        }
+        for (int r = wave; r < 16; r += 4)
+            for (int k = lane; k < strip_lines(n); k += 64)
+                s_in[k * kStripPitch + r] = (r0 + r < n && k < n) ? src[o + (int64_t)(r0 + r) * n + k] : 0.0;
+        __syncthreads();
+        strip_product<true>(n, s_cas, s_in, (int)item, [&](int row, int col, double v) {
+            if (r0 + row < n && col < n) dst[o + (int64_t)(r0 + row) * n + col] = v;
+        });
+        __syncthreads();  // the strip is free
+    }
+}
+
+// dst = H (G . (H dst)) by strips of 16 columns.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_box_columns(BoxBatch B, double* dst, FftSymbol sy) {
+    HIP_DYNAMIC_SHARED(double, s_box)
+    const int tid = (int)threadIdx.x;
+    const long long items = (long long)B.count * B.strips;
+    for (long long item = blockIdx.x; item < items; item += gridDim.x) {
+        int n, c0;
+        int64_t o;
+        if (!box_strip(B, item, &n, &o, &c0)) {
+            if (tid == 0 && (n < 1 || n > B.nmax)) *B.bad = 1;
             continue;
         }
-        if (n <= nlo || n > nhi) continue;
-        const int64_t o = offs[b];
-        fft_conv_box<double>(n, nb, src + o, dst + o, tw + tw_offset(n), sy, W, L, H);
+        const int lines = strip_lines(n);
+        double* s_in = s_box;
+        double* s_mid = s_in + lines * kStripPitch;
+        double* s_cas = s_mid + lines * kStripPitch;
+        double* s_cos = s_cas + n;
+        for (int t = tid; t < n; t += 256) {
+            double s, c;
+            sincospi(2.0 * (double)t / (double)n, &s, &c);
+            s_cas[t] = c + s;
+            s_cos[t] = c;
+        }
+        const int lc = tid & 15, c = min(c0 + lc, n - 1);
+        for (int k = tid >> 4; k < lines; k += 16)
+            s_in[k * kStripPitch + lc] = (k < n && c0 + lc < n) ? dst[o + (int64_t)k * n + c0 + lc] : 0.0;
+        __syncthreads();
+        for (int j = tid >> 4; 2 * j <= n; j += 16) {  // the symbol, even in j
+            const double g = box_symbol(j, c, n, s_cos, sy);
+            s_mid[j * kStripPitch + lc] = g;
+            if (j > 0) s_mid[(n - j) * kStripPitch + lc] = g;
+        }
+        __syncthreads();
+        strip_product<false>(n, s_cas, s_in, (int)item, [&](int j, int col, double v) {
+            if (j < lines) s_mid[j * kStripPitch + col] = j < n ? v * s_mid[j * kStripPitch + col] : 0.0;
+        });
+        __syncthreads();
+        strip_product<false>(n, s_cas, s_mid, (int)item + 2, [&](int row, int col, double v) {
+            if (row < n && c0 + col < n) dst[o + (int64_t)row * n + c0 + col] = v;
+        });
+        __syncthreads();
     }
 }
 

@@ -307,7 +307,6 @@ int raise_lds(ggx_ctx* ctx) {
     const void* fns[] = {(const void*)k_conv_strip<double, 2>, (const void*)k_conv_strip<float, 2>,
                          (const void*)k_conv_fft<double, true>, (const void*)k_conv_fft<double, false>,
                          (const void*)k_conv_fft<float, true>, (const void*)k_conv_fft<float, false>,
-                         (const void*)k_conv_fft_batch<true>, (const void*)k_conv_fft_batch<false>,
                          (const void*)k_contour<double, false, false, 64>, (const void*)k_contour<double, false, false, 256>,
                          (const void*)k_contour<float, false, false, 64>, (const void*)k_contour<float, false, false, 256>,
                          (const void*)k_contour<double, true, false, 64>, (const void*)k_contour<double, true, false, 256>,
@@ -320,7 +319,7 @@ int raise_lds(ggx_ctx* ctx) {
                          (const void*)k_conv_strip<float, 4>, (const void*)k_conv_strip<float, 8>,
                          (const void*)k_conv_tiles<double, 2>, (const void*)k_conv_tiles<double, 3>, (const void*)k_conv_tiles<double, 4>,
                          (const void*)k_conv_tiles<float, 2>, (const void*)k_conv_tiles<float, 3>, (const void*)k_conv_tiles<float, 4>};
-    constexpr int kFns = (int)(sizeof(fns) / sizeof(fns[0])), kContour0 = 8, kRedist0 = 20, kRedist1 = 26;
+    constexpr int kFns = (int)(sizeof(fns) / sizeof(fns[0])), kContour0 = 6, kRedist0 = 18, kRedist1 = 24;
     for (const void* f : fns) {
         hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
         if (e != hipSuccess) {
@@ -1282,8 +1281,7 @@ extern "C" int ggx_load_network(ggx_ctx* ctx, const ggx_network* net) {
         // FFT engine tables: twiddles of every side up to kMaxBox (built on the device), and the
         // global half-spectrum slots when the engine may meet boxes above kFftLdsMax
         if ((rc = dalloc(ctx, ctx->tw, (size_t)tw_offset(kMaxBox + 1)))) return rc;
-        hipLaunchKernelGGL(k_fft_twiddles, dim3(kMaxBox), dim3(256), 0, ctx->stream, ctx->tw, 1, kMaxBox,
-                           (int*)nullptr);
+        hipLaunchKernelGGL(k_fft_twiddles, dim3(kMaxBox), dim3(256), 0, ctx->stream, ctx->tw, 1, kMaxBox);
         HIPCHK(hipGetLastError());
         bool any_fft = false;
         for (int b = 0; b < ctx->nbuckets; ++b) any_fft = any_fft || fft_for(ctx, ctx->edges[b]);
@@ -1980,37 +1978,6 @@ extern "C" int ggx_get_stats(ggx_ctx* ctx, ggx_stats* out) {
 // ------------------------------------------------------------------------------------------
 namespace {
 
-struct BatchDevice {
-    int cus = 0;
-    int lds_max = 0;
-    int static_lds[2] = {0, 0};  // k_conv_fft_batch<false>, <true>
-};
-
-// Device limits of the current device and the batch kernels' dynamic-LDS ceiling (no allocation).
-int batch_device(BatchDevice& B) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return fail_free(GGX_E_HIP, std::string("hipGetDevice: ") + hipGetErrorString(e));
-    hipDeviceProp_t prop;
-    e = hipGetDeviceProperties(&prop, dev);
-    if (e != hipSuccess) return fail_free(GGX_E_HIP, std::string("hipGetDeviceProperties: ") + hipGetErrorString(e));
-    B.cus = prop.multiProcessorCount;
-    int lim = std::max((int)prop.sharedMemPerBlock, (int)prop.maxSharedMemoryPerMultiProcessor);
-    const void* fns[] = {(const void*)k_conv_fft_batch<false>, (const void*)k_conv_fft_batch<true>};
-    for (int k = 0; k < 2; ++k) {
-        if (hipFuncSetAttribute(fns[k], hipFuncAttributeMaxDynamicSharedMemorySize, lim) != hipSuccess) {
-            (void)hipGetLastError();
-            lim = std::min(lim, (int)prop.sharedMemPerBlock);
-        }
-        hipFuncAttributes fa;
-        e = hipFuncGetAttributes(&fa, fns[k]);
-        if (e != hipSuccess) return fail_free(GGX_E_HIP, std::string("hipFuncGetAttributes: ") + hipGetErrorString(e));
-        B.static_lds[k] = (int)fa.sharedSizeBytes;
-    }
-    B.lds_max = lim;
-    return GGX_OK;
-}
-
 int check_batch_args(int32_t count, const int32_t* n, const int64_t* off, const double* in, const double* out,
                      int32_t max_n, int32_t mode, int32_t R) {
     if (count < 0 || mode < 0 || mode > 2 || R < 1 || max_n < 1) return GGX_E_ARG;
@@ -2019,27 +1986,29 @@ int check_batch_args(int32_t count, const int32_t* n, const int64_t* off, const 
     return GGX_OK;
 }
 
-// Twiddles into tw, then the LDS-path launch (sides up to kFftLdsMax) and, when max_n is above
-// it, the global-slot launch over `slots` workspace slots of side max_n; *bad collects sides
-// outside [1, max_n].  Everything is queued on st.
-int run_batch(const BatchDevice& B, int32_t count, const int32_t* n, const int64_t* off, const double* in,
-              double* out, int32_t max_n, const FftSymbol& sy, hipStream_t st, double2* tw, double2* work, int slots,
-              int* bad) {
-    hipLaunchKernelGGL(k_fft_twiddles, dim3(max_n), dim3(256), 0, st, tw, 1, max_n, bad);
-    const int nl = std::min(max_n, kFftLdsMax);
-    const long long lds = fft_lds<double>(nl, true);
-    if (lds + B.static_lds[1] + 256 > B.lds_max) return GGX_E_BOUNDS;
-    const int per = (int)std::max<long long>(1, std::min<long long>(8, 163840 / (lds + B.static_lds[1])));
-    const int grid = std::max(1, std::min(count, B.cus * per));
-    hipLaunchKernelGGL(k_conv_fft_batch<true>, dim3(grid), dim3(256), (size_t)lds, st, count, n, off, in, out,
-                       (const double2*)tw, sy, nl, 0, nl, max_n, (double2*)nullptr, bad);
-    if (max_n > kFftLdsMax) {
-        const long long ldsw = fft_lds<double>(max_n, false);
-        if (ldsw + B.static_lds[0] + 256 > B.lds_max) return GGX_E_BOUNDS;
-        const int gw = std::max(1, std::min(count, slots));
-        hipLaunchKernelGGL(k_conv_fft_batch<false>, dim3(gw), dim3(256), (size_t)ldsw, st, count, n, off, in, out,
-                           (const double2*)tw, sy, max_n, kFftLdsMax, max_n, max_n, work, bad);
-    }
+// The three launches of a batch, queued on st; *bad collects sides outside [1, max_n].
+int run_batch(int32_t count, const int32_t* n, const int64_t* off, const double* in, double* out, int32_t max_n,
+              const FftSymbol& sy, hipStream_t st, int* bad) {
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return fail_free(GGX_E_HIP, std::string("ggx_convolve_boxes: device: ") + hipGetErrorString(e));
+    const size_t rows = (size_t)box_rows_lds(max_n), columns = (size_t)box_columns_lds(max_n);
+    const struct { const void* f; size_t lds, most; } need[] = {
+        {(const void*)k_box_rows, rows, (size_t)box_rows_lds(kMaxBox)},
+        {(const void*)k_box_columns, columns, (size_t)box_columns_lds(kMaxBox)}};
+    for (const auto& k : need)  // above the default limit: one value for every call, so that threads agree
+        if (k.lds > 65536 && hipFuncSetAttribute(k.f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.most) != hipSuccess) {
+            (void)hipGetLastError();
+            return GGX_E_BOUNDS;
+        }
+    BoxBatch B;
+    B.count = count; B.strips = (max_n + 15) / 16;
+    B.ns = n; B.offs = off; B.nmax = max_n; B.bad = bad;
+    const dim3 grid((unsigned)std::min<long long>((long long)count * B.strips, (long long)cus * 64)), block(256);
+    hipLaunchKernelGGL(k_box_rows, grid, block, rows, st, B, in, out, 1);
+    hipLaunchKernelGGL(k_box_columns, grid, block, columns, st, B, out, sy);
+    hipLaunchKernelGGL(k_box_rows, grid, block, rows, st, B, (const double*)out, out, 0);
     if (hipGetLastError() != hipSuccess) return GGX_E_HIP;
     return GGX_OK;
 }
@@ -2059,26 +2028,10 @@ extern "C" int ggx_convolve_boxes(int32_t count, const int32_t* n, const int64_t
     int rc = check_batch_args(count, n, off, in, out, max_n, mode, R);
     if (rc != GGX_OK) return fail_free(rc, "ggx_convolve_boxes: bad arguments");
     if (count == 0) return GGX_OK;
-    BatchDevice B;
-    if ((rc = batch_device(B)) != GGX_OK) return rc;  // the reason is in ggx_last_error(NULL)
     hipStream_t st = (hipStream_t)stream;
-    double2* tw = nullptr;
-    double2* work = nullptr;
     int* bad = nullptr;
-    const int slots = kFftWideGrid;
-    auto release = [&]() {
-        if (tw) (void)hipFree(tw);
-        if (work) (void)hipFree(work);
-        if (bad) (void)hipFree(bad);
-    };
-    if (hipMalloc((void**)&tw, (size_t)tw_offset(max_n + 1) * sizeof(double2) + 16) != hipSuccess ||
-        hipMalloc((void**)&bad, sizeof(int)) != hipSuccess ||
-        (max_n > kFftLdsMax &&
-         hipMalloc((void**)&work, (size_t)slots * (size_t)fft_slot(max_n) * sizeof(double2)) != hipSuccess)) {
-        release();
-        return GGX_E_OOM;
-    }
-    rc = run_batch(B, count, n, off, in, out, max_n, batch_symbol(mode, dt, R), st, tw, work, slots, bad);
+    if (hipMalloc((void**)&bad, sizeof(int)) != hipSuccess) return GGX_E_OOM;
+    rc = run_batch(count, n, off, in, out, max_n, batch_symbol(mode, dt, R), st, bad);
     int hbad = 0;
     if (rc == GGX_OK) {
         if (hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess ||
@@ -2087,28 +2040,21 @@ extern "C" int ggx_convolve_boxes(int32_t count, const int32_t* n, const int64_t
     } else {
         (void)hipStreamSynchronize(st);
     }
-    release();
+    (void)hipFree(bad);
     if (rc == GGX_OK && hbad) return fail_free(GGX_E_BOUNDS, "ggx_convolve_boxes: a box side is outside [1, max_n]");
     if (rc != GGX_OK) return fail_free(rc, "ggx_convolve_boxes: device error");
     return rc;
 }
 
 // ------------------------------------------------------------------------------------------
-// The same batch without any allocation: its workspace is the static device array `scratch`
-// (one copy per GPU, alive until the process ends).  Layout: the bounds flag (first 256
-// bytes), the twiddle tables of sides 1..kNoAllocMaxN, then kNoAllocSlots half-spectrum slots
-// of side kNoAllocMaxN for the boxes above kFftLdsMax.  Host code never passes the array's
-// name to a kernel or a copy: it uses the device address taken once per device with
-// hipGetSymbolAddress.  Calls that overlap on one GPU share the array and race.
+// The same batch without any allocation: its bounds flag is the static device word `scratch` (one
+// copy per GPU, alive until the process ends).  Host code never passes the word's name to a kernel
+// or a copy: it uses the device address taken once per device with hipGetSymbolAddress.  Calls that
+// overlap on one GPU share the word and race.
 // ------------------------------------------------------------------------------------------
 constexpr int kNoAllocMaxN = 256;
-constexpr int kNoAllocSlots = 8;
-constexpr size_t kScratchFlag = 256;
-constexpr size_t kScratchTw = ((size_t)tw_offset(kNoAllocMaxN + 1) * sizeof(double2) + 255) & ~(size_t)255;
-constexpr size_t kScratchSlots = (size_t)kNoAllocSlots * (size_t)fft_slot(kNoAllocMaxN) * sizeof(double2);
-constexpr size_t kScratchBytes = kScratchFlag + kScratchTw + kScratchSlots;  // 4.5 MiB
 
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ int scratch;
 
 namespace {
 
@@ -2145,19 +2091,14 @@ extern "C" int ggx_convolve_boxes_noalloc(int32_t count, const int32_t* n, const
     if (rc != GGX_OK) return fail_free(rc, "ggx_convolve_boxes_noalloc: bad arguments");
     if (max_n > kNoAllocMaxN)
         return fail_free(GGX_E_BOUNDS, "ggx_convolve_boxes_noalloc: max_n " + std::to_string(max_n) +
-                                           " is above the static workspace's largest side " +
+                                           " is above the largest side " +
                                            std::to_string(kNoAllocMaxN));
     if (count == 0) return GGX_OK;
     void* base = nullptr;
     if ((rc = scratch_address(&base)) != GGX_OK) return rc;
-    BatchDevice B;
-    if ((rc = batch_device(B)) != GGX_OK) return rc;  // the reason is in ggx_last_error(NULL)
     hipStream_t st = (hipStream_t)stream;
-    unsigned char* b = (unsigned char*)base;
-    int* bad = (int*)b;                                            // cleared by the twiddle kernel
-    double2* tw = (double2*)(b + kScratchFlag);
-    double2* work = (double2*)(b + kScratchFlag + kScratchTw);
-    rc = run_batch(B, count, n, off, in, out, max_n, batch_symbol(mode, dt, R), st, tw, work, kNoAllocSlots, bad);
+    int* bad = (int*)base;
+    rc = run_batch(count, n, off, in, out, max_n, batch_symbol(mode, dt, R), st, bad);
     if (rc != GGX_OK) {
         (void)hipStreamSynchronize(st);
         return fail_free(rc, "ggx_convolve_boxes_noalloc: launch failed");

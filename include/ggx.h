@@ -324,19 +324,17 @@ int ggx_get_stats(ggx_ctx* ctx, ggx_stats* out);
  * n x n doubles (out[b] = IDFT2(G . DFT2(in[b])), G of ConvolutionMode `mode`: 0 Laplace,
  * 1 Laplace-Richardson, 2 Gaussian, with the time step dt and nsq = R^2 of the global grid,
  * box.cpp:636-691).  n, off, in and out are device pointers; in and out must not overlap.
- * `stream` is a hipStream_t (NULL: the null stream).  The call allocates its workspace (twiddle
- * tables, an error flag, half-spectrum slots for sides above 128), runs on `stream`, waits for
- * it and frees the workspace.  Returns GGX_OK, GGX_E_ARG, GGX_E_BOUNDS (max_n above 512, or a
+ * `stream` is a hipStream_t (NULL: the null stream).  The call allocates an error flag, runs on
+ * `stream` (out holds intermediate values meanwhile), waits for it and frees the flag.  Returns GGX_OK, GGX_E_ARG, GGX_E_BOUNDS (max_n above 512, or a
  * side outside [1, max_n]: that box is left unwritten), GGX_E_OOM or GGX_E_HIP. */
 int ggx_convolve_boxes(int32_t count, const int32_t* n, const int64_t* off, const double* in, double* out,
                        int32_t max_n, int32_t mode, double dt, int32_t R, void* stream);
 
 /* ggx_convolve_boxes without any allocation.  No counterpart in the reference: it is for callers
  * that cannot allocate device memory (code under hipGraph capture, tight serving loops, harnesses
- * that forbid hipMalloc).  Its workspace is a static device array of 4.5 MiB that every GPU the
- * library runs on holds until the process ends; it limits max_n to 256 (GGX_E_BOUNDS above, with
- * the reason in ggx_last_error(NULL)).  Same arguments and results as ggx_convolve_boxes.  Calls
- * that overlap on one GPU share that array and race: serialise them. */
+ * that forbid hipMalloc).  Its error flag is a static device word; max_n is limited to 256
+ * (GGX_E_BOUNDS above, with the reason in ggx_last_error(NULL)).  Same arguments and results as
+ * ggx_convolve_boxes.  Calls that overlap on one GPU share that word and race: serialise them. */
 int ggx_convolve_boxes_noalloc(int32_t count, const int32_t* n, const int64_t* off, const double* in, double* out,
                                int32_t max_n, int32_t mode, double dt, int32_t R, void* stream);
 

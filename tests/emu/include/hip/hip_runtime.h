@@ -287,6 +287,8 @@ inline hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { std::m
 inline hipError_t hipSetDevice(int) { return 0; }
 inline hipError_t hipGetDevice(int* d) { *d = 0; return 0; }
 #define HIP_SYMBOL(x) (&(x))
+enum { hipDeviceAttributeMultiprocessorCount = 1 };
+inline hipError_t hipDeviceGetAttribute(int* v, int, int) { *v = 4; return 0; }
 inline hipError_t hipGetSymbolAddress(void** p, const void* sym) { *p = const_cast<void*>(sym); return 0; }
 inline hipError_t hipStreamCreate(hipStream_t* s) { *s = new int(0); return 0; }
 inline hipError_t hipStreamDestroy(hipStream_t s) { delete s; return 0; }
