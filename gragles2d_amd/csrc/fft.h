@@ -1,12 +1,13 @@
-// fft.h -- 2-D convolution of square boxes by transforms (gfx950): the step's by mixed-radix FFT, the
-// standalone batch's by products with the real transform matrix on the matrix cores.
+// fft.h -- 2-D convolution of square boxes by transforms (gfx950): in FP64, a step's and the standalone
+// batch's, by products with the real transform matrix on the matrix cores; a step's in FP32 by
+// mixed-radix FFT, and in FP64 too where the LDS allowed to a context is too small for the strips.
 //
 // LSbox::convolutionGeneratorFFTW (box.cpp:622-695): phi~ = IDFT2( G . DFT2(phi) ) with the
 // real, even symbol G of ConvolutionMode 0 (Laplace, box.cpp:648-659), 1 (Laplace with the
 // Richardson extrapolation, 660-673) or 2 (Gaussian, 674-688).  G carries the 1/n^2 of the
 // unnormalised c2r transform and uses the global grid size R in nsq (636-637).
 //
-// The step (k_conv_fft): one 256-lane workgroup per box, exact n (no padding to a friendly size),
+// The FFT (k_conv_fft): one 256-lane workgroup per box, exact n (no padding to a friendly size),
 // three phases separated by workgroup barriers:
 //   1. rows     each wave takes a pair of rows (2p, 2p+1), transforms z = row_2p + i row_2p+1
 //               as one complex line and splits the result into the two half spectra
@@ -275,6 +276,10 @@ __global__ void __launch_bounds__(256) k_conv_fft(const int* __restrict__ list, 
 // table, product and store at 16 waves per CU), 96 of side 130 to 256 take 0.36 ms.  The FFT with a
 // workgroup per box took 7.5 ms, bound by its p-term sums, and 29 ms, bound by its eight half-spectrum
 // slots.  The Richardson symbol's two 40th powers are a third of k_box_columns with pow().
+// In a step (k_box_rows and k_box_columns of FP64 networks with the FFT engine's symbols) the boxes
+// are the grains of a launch's work items.  There the FFT took 1.2 of 2.0 ms per step of a 5000-grain
+// Laplace network, up to 0.4 ms of it for the few widest boxes, one after the other's long sums in
+// one workgroup; the strips take 0.35 ms.
 // ------------------------------------------------------------------------------------------
 struct BoxBatch {
     int count, strips;   // boxes; strips of 16 lines of the largest side allowed
@@ -282,6 +287,13 @@ struct BoxBatch {
     const int64_t* offs;
     int nmax;            // a box whose side is outside [1, nmax] is left alone and sets *bad
     int* bad;
+};
+
+struct StepBoxes {       // the same for a step's work items
+    Items it;
+    int strips, nmax;
+    const Box* box;
+    const long long* off;
 };
 
 constexpr int kStripPitch = 17;   // doubles per line of a strip: 16 and one against bank conflicts
@@ -355,12 +367,31 @@ __device__ __forceinline__ void strip_product(int n, const double* s_cas, const 
     }
 }
 
-// The box and strip of a work item; false: no such strip.
-__device__ __forceinline__ bool box_strip(const BoxBatch& B, long long item, int* n, int64_t* o, int* line0) {
-    const int b = (int)(item / B.strips);
-    *line0 = (int)(item - (long long)b * B.strips) * 16;
+__device__ __forceinline__ int box_count(const BoxBatch& B) { return B.count; }
+__device__ __forceinline__ int box_count(const StepBoxes& B) { return items_total(B.it); }
+
+__device__ __forceinline__ void box_place(const BoxBatch& B, int b, int* n, int64_t* o) {
     *n = sload(B.ns + b);
     *o = sload(B.offs + b);
+}
+__device__ __forceinline__ void box_place(const StepBoxes& B, int b, int* n, int64_t* o) {
+    int bucket, pos;
+    const int g = item_grain(B.it, b, &bucket, &pos);
+    *n = sload(&B.box[g].n);
+    *o = sload(B.off + g);
+}
+
+__device__ __forceinline__ void clear_bad(const BoxBatch& B) { *B.bad = 0; }
+__device__ __forceinline__ void clear_bad(const StepBoxes&) {}
+__device__ __forceinline__ void set_bad(const BoxBatch& B) { *B.bad = 1; }
+__device__ __forceinline__ void set_bad(const StepBoxes&) {}
+
+// The box and strip of a work item; false: no such strip.
+template <class Boxes>
+__device__ __forceinline__ bool box_strip(const Boxes& B, long long item, int* n, int64_t* o, int* line0) {
+    const int b = (int)(item / B.strips);
+    *line0 = (int)(item - (long long)b * B.strips) * 16;
+    box_place(B, b, n, o);
     return *n >= 1 && *n <= B.nmax && *line0 < *n;
 }
 
@@ -392,11 +423,12 @@ __device__ __forceinline__ double box_symbol(int j, int i, int n, const double* 
 }
 
 // dst = src H by strips of 16 rows (src may be dst).  first: clears *bad.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_box_rows(BoxBatch B, const double* src, double* dst, int first) {
+template <class Boxes>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_box_rows(Boxes B, const double* src, double* dst, int first) {
     HIP_DYNAMIC_SHARED(double, s_box)
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (first && blockIdx.x == 0 && tid == 0) *B.bad = 0;
-    const long long items = (long long)B.count * B.strips;
+    if (first && blockIdx.x == 0 && tid == 0) clear_bad(B);
+    const long long items = (long long)box_count(B) * B.strips;
     for (long long item = blockIdx.x; item < items; item += gridDim.x) {
         int n, r0;
         int64_t o;
@@ -420,15 +452,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 }
 
 // dst = H (G . (H dst)) by strips of 16 columns.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_box_columns(BoxBatch B, double* dst, FftSymbol sy) {
+template <class Boxes>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_box_columns(Boxes B, double* dst, FftSymbol sy) {
     HIP_DYNAMIC_SHARED(double, s_box)
     const int tid = (int)threadIdx.x;
-    const long long items = (long long)B.count * B.strips;
+    const long long items = (long long)box_count(B) * B.strips;
     for (long long item = blockIdx.x; item < items; item += gridDim.x) {
         int n, c0;
         int64_t o;
         if (!box_strip(B, item, &n, &o, &c0)) {
-            if (tid == 0 && (n < 1 || n > B.nmax)) *B.bad = 1;
+            if (tid == 0 && (n < 1 || n > B.nmax)) set_bad(B);
             continue;
         }
         const int lines = strip_lines(n);

@@ -351,6 +351,11 @@ int raise_lds(ggx_ctx* ctx) {
         }
     }
     ctx->lds_max = lim;
+    // the strips' launches ask for what their boxes need, within lds_max: one ceiling for every context
+    (void)hipFuncSetAttribute((const void*)k_box_rows<StepBoxes>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)box_rows_lds(kMaxBox));
+    if (hipFuncSetAttribute((const void*)k_box_columns<StepBoxes>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)box_columns_lds(kMaxBox)) != hipSuccess)
+        (void)hipGetLastError();
     // static __shared__ bytes count against the same per-workgroup limit as the dynamic request
     int* dst[] = {&ctx->static_fft[0][1], &ctx->static_fft[0][0], &ctx->static_fft[1][1], &ctx->static_fft[1][0]};
     for (int k = 0; k < kFns; ++k) {
@@ -605,6 +610,25 @@ int launch_conv_fft(ggx_ctx* ctx, hipStream_t st, const int* list, const int* co
     return GGX_OK;
 }
 
+// The three launches of strip products with the FFT engine's symbol over a launch's items, boxes up to
+// side nb (FP64).
+int launch_conv_boxes(ggx_ctx* ctx, hipStream_t st, const Items& it, int nb, int items, const double* src, double* dst) {
+    StepBoxes B;
+    B.it = it; B.strips = (nb + 15) / 16; B.nmax = nb; B.box = ctx->box; B.off = ctx->off;
+    // replayed steps launch for the grains there may be: fewer workgroups, as most find none
+    const long long cap = (long long)ctx->cu_count * (ctx->opt.persistent ? 16 : 64);
+    const dim3 grid((unsigned)std::max<long long>(1, std::min((long long)items * B.strips, cap))), block(256);
+    const size_t rows = (size_t)box_rows_lds(nb), columns = (size_t)box_columns_lds(nb);
+    hipLaunchKernelGGL(k_box_rows<StepBoxes>, grid, block, rows, st, B, src, dst, 1);
+    hipLaunchKernelGGL(k_box_columns<StepBoxes>, grid, block, columns, st, B, dst, fft_symbol_of(ctx));
+    hipLaunchKernelGGL(k_box_rows<StepBoxes>, grid, block, rows, st, B, (const double*)dst, dst, 0);
+    return GGX_OK;
+}
+
+// Whether the strips of boxes up to side nb fit the LDS this context may use.
+template <class T>
+bool boxes_for(const ggx_ctx* ctx, int nb) { return sizeof(T) == 8 && box_columns_lds(nb) + 256 <= ctx->lds_max; }
+
 // The circulant convolution of a launch's items, boxes up to side nb: the register tiles of 2, 3 or 4
 // times 16 columns, the LDS strip above 64.
 template <class T>
@@ -680,13 +704,25 @@ int launch_step(ggx_ctx* ctx, bool timed, bool record = false) {
             };
             while (e + 1 < ctx->nbuckets && !fft_for(ctx, ctx->edges[e + 1]) && tiles(e + 1) == tiles(b)) ++e;
         }
+        bool strips = false;
+        if (fft) {
+            auto limit = [&](int k) {  // strips of one launch share its LDS
+                const int side = ctx->edges[k];
+                return side <= 64 ? 64 : side <= 128 ? 128 : side <= 256 ? 256 : kMaxBox;
+            };
+            strips = boxes_for<T>(ctx, limit(b));
+            while (strips && e + 1 < ctx->nbuckets && fft_for(ctx, ctx->edges[e + 1]) && limit(e + 1) == limit(b)) ++e;
+        }
         int items = NS - 1;
         if (!ctx->opt.persistent) {
             items = 0;
             for (int k = b; k <= e; ++k) items += counts[k];
         }
         int rc = GGX_OK;
-        if (fft && (ctx->opt.persistent || items > 0))
+        if (strips) {
+            if (items > 0)
+                rc = launch_conv_boxes(ctx, st, bucket_items(ctx, b, e), ctx->edges[e], items, (const double*)P, (double*)Tt);
+        } else if (fft && (ctx->opt.persistent || items > 0))
             rc = launch_conv_fft<T>(ctx, st, ctx->blists + (size_t)b * NS, &S->bucket_total[b], ctx->edges[b],
                                     ctx->opt.persistent ? 0 : items, (const T*)P, Tt);
         else if (!fft && items > 0)
@@ -825,7 +861,9 @@ int launch_step_pergrain(ggx_ctx* ctx) {
     HIPCHK(hipEventRecord(ev[1], st));
     for (size_t i = 0; i < live.size(); ++i) {
         const int n = bx[live[i]].n;
-        int rc = fft_for(ctx, n) ? launch_conv_fft<T>(ctx, st, ctx->pg_list + i, ctx->pg_one + i, n, 1, (const T*)P, Tt)
+        int rc = fft_for(ctx, n) && boxes_for<T>(ctx, n)
+                     ? launch_conv_boxes(ctx, st, single_item(ctx->pg_list + i, ctx->pg_one + i, n), n, 1, (const double*)P, (double*)Tt)
+                 : fft_for(ctx, n) ? launch_conv_fft<T>(ctx, st, ctx->pg_list + i, ctx->pg_one + i, n, 1, (const T*)P, Tt)
                                  : launch_conv<T>(ctx, st, single_item(ctx->pg_list + i, ctx->pg_one + i, n), n, 1, (const T*)P, Tt);
         if (rc) return rc;
     }
@@ -2018,8 +2056,8 @@ int run_batch(int32_t count, const int32_t* n, const int64_t* off, const double*
     if (e != hipSuccess) return fail_free(GGX_E_HIP, std::string("ggx_convolve_boxes: device: ") + hipGetErrorString(e));
     const size_t rows = (size_t)box_rows_lds(max_n), columns = (size_t)box_columns_lds(max_n);
     const struct { const void* f; size_t lds, most; } need[] = {
-        {(const void*)k_box_rows, rows, (size_t)box_rows_lds(kMaxBox)},
-        {(const void*)k_box_columns, columns, (size_t)box_columns_lds(kMaxBox)}};
+        {(const void*)k_box_rows<BoxBatch>, rows, (size_t)box_rows_lds(kMaxBox)},
+        {(const void*)k_box_columns<BoxBatch>, columns, (size_t)box_columns_lds(kMaxBox)}};
     for (const auto& k : need)  // above the default limit: one value for every call, so that threads agree
         if (k.lds > 65536 && hipFuncSetAttribute(k.f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.most) != hipSuccess) {
             (void)hipGetLastError();
@@ -2029,9 +2067,9 @@ int run_batch(int32_t count, const int32_t* n, const int64_t* off, const double*
     B.count = count; B.strips = (max_n + 15) / 16;
     B.ns = n; B.offs = off; B.nmax = max_n; B.bad = bad;
     const dim3 grid((unsigned)std::min<long long>((long long)count * B.strips, (long long)cus * 64)), block(256);
-    hipLaunchKernelGGL(k_box_rows, grid, block, rows, st, B, in, out, 1);
-    hipLaunchKernelGGL(k_box_columns, grid, block, columns, st, B, out, sy);
-    hipLaunchKernelGGL(k_box_rows, grid, block, rows, st, B, (const double*)out, out, 0);
+    hipLaunchKernelGGL(k_box_rows<BoxBatch>, grid, block, rows, st, B, in, out, 1);
+    hipLaunchKernelGGL(k_box_columns<BoxBatch>, grid, block, columns, st, B, out, sy);
+    hipLaunchKernelGGL(k_box_rows<BoxBatch>, grid, block, rows, st, B, (const double*)out, out, 0);
     if (hipGetLastError() != hipSuccess) return GGX_E_HIP;
     return GGX_OK;
 }
