@@ -16,7 +16,7 @@
 // field is not read again in the step) and its signs as bit planes: per grain, rows and columns
 // of the tests C >= 0 and C > 0.  The contour's topology and the sweeps' signs come from the
 // bits; C itself is read at the zero crossings only.  On the 100k-grain lognormal network in FP64
-// (1.61e8 box points) the four take 2.8, 1.9, 0.01 and 2.2 ms per step; one kernel that did all of
+// (1.61e8 box points) the four take 2.2, 1.8, 0.01 and 2.1 ms per step; one kernel that did all of
 // it per grain, 256 lanes wide with C and the new field in LDS, took 11.8 ms: its serial phases
 // left three of four waves idle and its LDS tiles held four or five grains per CU.
 #pragma once
@@ -401,9 +401,26 @@ __global__ void __launch_bounds__(256) k_compare(LevelArgs<T> A) {
 // arrays hold, are walked by wave 0 over the bit rows.  Both record the same moves.
 // The ordered sums (area, perimeter, energy, lengths per neighbour) keep the contour's order: 64
 // terms at a time go through LDS and one wave adds them, so every sum sees the reference's
-// rounding.  One wave per grain up to side 64 (no barrier), four above.
+// rounding; the terms are loaded eight ahead (a 100-grain network 49 -> 36 us per step, 30k grains in
+// FP32 0.82 -> 0.74 ms: a load per addition waited for the LDS each time).  One wave per grain up to
+// side 64 (no barrier), four above.  What is left is one grain's latency, phase after phase.
 // ------------------------------------------------------------------------------------------
 constexpr int kNodeEnd = 0xffff;
+
+// use(k, load(k)) for k = 0 .. m - 1 in order, U loads ahead of their uses: an ordered sum over LDS
+// then waits for the LDS once in U terms.
+template <int U, class Load, class Use>
+__device__ __forceinline__ void in_order(int m, Load load, Use use) {
+    int k = 0;
+    for (; k + U <= m; k += U) {
+        decltype(load(0)) v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = load(k + u);
+#pragma unroll
+        for (int u = 0; u < U; ++u) use(k + u, v[u]);
+    }
+    for (; k < m; ++k) use(k, load(k));
+}
 
 // nearest_vertex by a whole wave: the smallest squared distance below 1e6, the first vertex that
 // has it; 1e9 where there is none.  pt(i) reads contour point i.
@@ -738,11 +755,10 @@ __global__ void __launch_bounds__(NT) k_contour(LevelArgs<T> A) {
                     __syncthreads();
                     if (tid < 64) {
                         const int m = min(NT, L1 - c0);
-                        for (int k = 0; k < m; ++k) {
-                            const double2 v = s_stage[k];
+                        in_order<8>(m, [&](int k) { return s_stage[k]; }, [&](int, const double2& v) {
                             vs += v.x;
                             per = fma(v.y, G.h, per);
-                        }
+                        });
                     }
                     __syncthreads();
                 }
@@ -1073,15 +1089,18 @@ __global__ void __launch_bounds__(NT) k_contour(LevelArgs<T> A) {
                     s_stage[lane] = make_double2(lv, ANISO ? lv * ev : 0.0);
                     wave_lds_sync();
                     const int m = min(64, L1 - c0), ms = min(m, stop - c0);
-                    for (int k = 0; k < ms; ++k) {
-                        const double2 v = s_stage[k];
-                        if (s_cand[c0 + k] == lane) my_len = fma(v.x, h, my_len);
-                        if constexpr (ANISO) e = fma(v.y, h, e);
-                    }
+                    struct Term { double2 v; int slot; };
+                    in_order<8>(ms, [&](int k) { return Term{s_stage[k], s_cand[c0 + k]}; }, [&](int, const Term& q) {
+                        const double longer = fma(q.v.x, h, my_len);
+                        my_len = q.slot == lane ? longer : my_len;
+                        if constexpr (ANISO) e = fma(q.v.y, h, e);
+                    });
                     if constexpr (ANISO) {
-                        for (int k = max(ms, 0); k < m; ++k) e = fma(s_stage[k].y, h, e);
+                        const int from = max(ms, 0);
+                        in_order<8>(m - from, [&](int k) { return s_stage[from + k].y; }, [&](int, double v) { e = fma(v, h, e); });
                     } else if (!whole) {
-                        for (int k = 0; k < m; ++k) e = fma(c0 + k >= stop ? -s_stage[k].x : s_stage[k].x, h, e);
+                        in_order<8>(m, [&](int k) { return s_stage[k].x; },
+                                    [&](int k, double v) { e = fma(c0 + k >= stop ? -v : v, h, e); });
                     }
                     wave_lds_sync();
                 }
