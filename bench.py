@@ -8,9 +8,9 @@ between two device synchronisations.  Prints one JSON line.
   value           grid-point updates/s of the hipGraph-replayed step (the production launch mode)
   phases / roofline
                   the same network stepped with stream launches and HIP events around each phase
-                  (on the library's stream): the k_level launches of a step run back to back
-                  between two events, so their summed duration and algorithmic bytes give the
-                  achieved HBM rate of the dominant kernel
+                  (on the library's stream): the level-set launches of a step (k_compare,
+                  k_contour, k_alloc, k_redist) run back to back between two events, so their
+                  summed duration and algorithmic bytes give the achieved HBM rate of the phase
   pergrain_value  the same kernels with one launch per grain (the reference's per-LSbox calls)
   cpu_baseline    the oracle (C++/OpenMP restatement of the reference's CPU path) on a bounded
                   sample of the same workload, on this host's cores
@@ -181,6 +181,9 @@ def adjoint_timing(iters, warm=16):
             "fwd_adj_s_per_step": (fwd + adj) / iters}
 
 
+LEVEL_KERNELS = ("k_compare", "k_contour", "k_alloc", "k_redist")
+
+
 def phase_split(G, N, s, net, prec, w, a):
     """Per-phase device time of stream-launched steps (HIP events on the library's stream) and
     the roofline of the dominant HBM-bound kernel from them."""
@@ -197,11 +200,12 @@ def phase_split(G, N, s, net, prec, w, a):
     aniso = not w.isotropic
     if aniso or phases["level_ms"] >= phases["convolution_ms"]:
         # anisotropic networks: the convolution phase also holds the velocity corrector (k_aniso,
-        # bound by its per-pixel projection, not by HBM), so the roofline line is k_level's
-        kern, byts, ms = "k_level", level_b, phases["level_ms"]
+        # bound by its per-pixel projection, not by HBM), so the roofline line is the level-set phase's
+        kern, byts, ms = LEVEL_KERNELS, level_b, phases["level_ms"]
     else:
         fft = a.conv == "fft" or s.convolution_mode != 2
-        kern, byts, ms = ("k_conv_fft" if fft else "k_conv_tiles"), conv_b, phases["convolution_ms"]
+        strips = fft and prec == N.PREC_FP64
+        kern, byts, ms = (("k_box_rows", "k_box_columns") if strips else ("k_conv_fft",) if fft else ("k_conv_tiles",)), conv_b, phases["convolution_ms"]
     achieved = byts / (ms * 1e-3)
     precision = "fp64" if prec == N.PREC_FP64 else "fp32"
     if aniso:
@@ -210,14 +214,14 @@ def phase_split(G, N, s, net, prec, w, a):
         "phases_ms_per_step": phases,
         "stream_ms_per_step": 1e3 * sec / k,
         "algorithmic_bytes_per_step": {"convolution": conv_b, "level": level_b},
-        "roofline": {"kernel": kern, "bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9,
+        "roofline": {"kernel": " + ".join(kern), "bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK,
                      "traffic": measured_traffic(w.name, precision, kern)},
     }
 
 
-def measured_traffic(workload, precision, kernel):
-    """HBM bytes per step of the kernel's launches from the committed rocprofv3 --pmc summary
+def measured_traffic(workload, precision, kernels):
+    """HBM bytes per step of the kernels' launches from the committed rocprofv3 --pmc summary
     (FETCH_SIZE and WRITE_SIZE, scaled by what the counters read for a copy of known size);
     None when no summary exists for this workload and precision."""
     path = os.path.join(ROOT, "profiles", f"traffic_{workload.replace('-', '')}_{precision}.json")
@@ -225,8 +229,8 @@ def measured_traffic(workload, precision, kernel):
         return None
     with open(path) as f:
         t = json.load(f)
-    prefix = f"ggx::{kernel}<{'double' if precision == 'fp64' else 'float'}"
-    hits = [e["hbm_bytes"] for name, e in t.get("per_step", {}).items() if name.startswith(prefix)]
+    prefixes = tuple(f"ggx::{k}" for k in kernels)
+    hits = [e["hbm_bytes"] for name, e in t.get("per_step", {}).items() if name.startswith(prefixes)]
     return sum(hits) if hits else None
 
 

@@ -210,7 +210,7 @@ __device__ __forceinline__ int block_flag_scan(bool f, int* s_wt, int* total) {
 // next entry's were issued.  The lanes hold the list's boxes (readlane hands them out), so the waves
 // of a grain share nothing and meet no barrier.  Only the entries that meet the block are walked, in
 // list order (strict >, first wins).  One launch takes all sides in spatial order, a contiguous part
-// per die: 8 launches, one per side, read most of a neighbour's pixels from beyond the die's cache.
+// per die: 8 launches, one per side, fetched 8.9 GB in place of 4.7 from beyond the dies' caches.
 // 100k-grain network in FP64 2.65 -> 2.2 ms per step, 30k in FP32 0.62 -> 0.51, 2000 grains 0.39 -> 0.23.
 //
 // COARSEN: the pass after a grid coarsening (grainhdl.cpp:1464-1476): the comparison of the grains
