@@ -630,13 +630,13 @@ template <class T>
 bool boxes_for(const ggx_ctx* ctx, int nb) { return sizeof(T) == 8 && box_columns_lds(nb) + 256 <= ctx->lds_max; }
 
 // The circulant convolution of a launch's items, boxes up to side nb: the register tiles of 2, 3 or 4
-// times 16 columns, the LDS strip above 64.
+// times 16 columns, the LDS strip above 64 and where the tiles are above the context's lds_budget.
 template <class T>
 int launch_conv(ggx_ctx* ctx, hipStream_t st, const Items& it, int nb, int items, const T* src, T* dst) {
     const int nt = (nb + 15) / 16;
     const T* kern = (const T*)ctx->kern;
-    if (nb <= 64) {
-        const int tiles = std::max(2, nt);
+    const int tiles = std::max(2, nt);
+    if (nb <= 64 && conv_tiles_lds<T>(tiles) + 256 <= ctx->lds_max) {
         const size_t lds = (size_t)conv_tiles_lds<T>(tiles);
         const dim3 grid(std::max(1, std::min(items, ctx->cu_count * 64))), block(64 * tiles);
         if (tiles == 2)

@@ -656,13 +656,15 @@ __global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT
 }
 
 // Larger boxes, up to side 64 TU: four waves share 16 columns, each takes every fourth 16-row tile;
-// B in LDS, the field through LDS 16 columns at a time (the next 16 on their way meanwhile).
+// B in LDS, the field through LDS 16 columns at a time (the next 16 on their way meanwhile).  Takes a
+// box of any side n at about 160 n bytes of LDS, so where the lds_budget is too small for the tiles of
+// a smaller box it is convolved here, with the same bits.
 constexpr int kStripCols = 16;
 
 template <class T>
 __host__ __device__ inline long long conv_strip_lds(int nb) {
     const int rows = (nb + 15) & ~15;
-    return ((long long)rows * 16 + (long long)rows * tile_pitch<T>(kStripCols) + ktab_len(nb)) * (long long)sizeof(T);
+    return ((long long)rows * tile_pitch<T>(kStripCols) + ktab_len(nb)) * (long long)sizeof(T);
 }
 
 // Calls f with the tile count as a constant: 1 .. N.
@@ -700,8 +702,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
         if (xt >= nt) continue;
         const long long o = sload(off + g);
         const T* s = src + o;
-        T* strip = (T*)smem;                      // B: row i, 16 columns
-        T* chunk = strip + 16 * nt * 16;          // the field's columns k0 .. k0 + 15, all rows
+        T* chunk = (T*)smem;                      // the field's columns k0 .. k0 + 15, all rows
+        T* strip = chunk;                         // then B: row i, 16 columns (no chunk is read any more)
         T* table = chunk + 16 * nt * pitch;
         const T* kg = kern + sload(kern_off + n);
         const T* kt = table + n + kKPad;

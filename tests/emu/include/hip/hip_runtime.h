@@ -62,6 +62,7 @@ inline int g_cur = 0;
 inline dim3 g_tid, g_bid, g_bdim, g_gdim;
 inline std::function<void()>* g_body = nullptr;
 inline unsigned char* g_dyn = nullptr;
+inline size_t g_lds_most = 0;  // largest dynamic LDS of any launch so far
 constexpr size_t kStack = 256 * 1024;
 
 // Barriers: a workgroup barrier waits until every live lane of the block has arrived; a wave
@@ -131,6 +132,7 @@ inline void launch(dim3 grid, dim3 block, size_t shmem, std::function<void()> bo
 
 inline void run_launch(dim3 grid, dim3 block, size_t shmem, std::function<void()> body) {
     unsigned nt = block.x * block.y * block.z;
+    g_lds_most = std::max(g_lds_most, shmem);
     if (std::getenv("EMU_TRACE")) std::fprintf(stderr, "[emu] launch grid %u block %u lds %zu\n", grid.x, nt, shmem);
     while (g_stacks.size() < nt) g_stacks.push_back((char*)std::malloc(kStack));
     g_fibers.assign(nt, Fiber{});
