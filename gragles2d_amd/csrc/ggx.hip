@@ -2066,7 +2066,9 @@ int run_batch(int32_t count, const int32_t* n, const int64_t* off, const double*
     BoxBatch B;
     B.count = count; B.strips = (max_n + 15) / 16;
     B.ns = n; B.offs = off; B.nmax = max_n; B.bad = bad;
-    const dim3 grid((unsigned)std::min<long long>((long long)count * B.strips, (long long)cus * 64)), block(256);
+    // an odd stride, so that a workgroup's items differ in their strip (50000 boxes of side 4 to 8 with
+    // max_n 128: 1.69 ms with cus * 64, 0.78)
+    const dim3 grid((unsigned)std::min<long long>((long long)count * B.strips, (long long)cus * 64 - 1)), block(256);
     hipLaunchKernelGGL(k_box_rows<BoxBatch>, grid, block, rows, st, B, in, out, 1);
     hipLaunchKernelGGL(k_box_columns<BoxBatch>, grid, block, columns, st, B, out, sy);
     hipLaunchKernelGGL(k_box_rows<BoxBatch>, grid, block, rows, st, B, (const double*)out, out, 0);

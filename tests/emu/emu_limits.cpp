@@ -4,6 +4,9 @@
 //     one-grain launches under lds_budget against the same run without one: same bits, no launch above
 //     the budget.  Without a budget given: the LDS that a grain's contour points (36 bytes each), its
 //     squares (one byte each up to side 128) and 480 bytes take, for the network's neediest grain.
+//   emu_limits batch <count> <lowest side> <highest side> <max_n> <mode>
+//     ggx_convolve_boxes against the oracle, with the work spread over the dies: none has less than half
+//     of the average (workgroup barriers, which only a workgroup with a strip meets).
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -98,10 +101,46 @@ static int budget_check(int argc, char** argv) {
     return bad ? 1 : 0;
 }
 
+static int batch_check(int argc, char** argv) {
+    auto arg = [&](int k, int d) { return argc > k ? atoi(argv[k]) : d; };
+    const int count = arg(2, 64), lo = arg(3, 3), hi = arg(4, 16), max_n = arg(5, 128), mode = arg(6, 2), R = 200;
+    const double dt = 2.2e-5;
+    std::vector<int32_t> n;
+    std::vector<int64_t> off;
+    int64_t total = 0;
+    for (int b = 0; b < count; ++b) {
+        n.push_back(lo + (7 * b) % (hi - lo + 1));
+        off.push_back(total);
+        total += (int64_t)n[b] * n[b];
+    }
+    std::vector<double> in((size_t)total), out((size_t)total, 0.0), ref;
+    unsigned long long x = 12345;
+    for (auto& v : in) {
+        x = x * 6364136223846793005ULL + 1442695040888963407ULL;
+        v = ((double)(x >> 11) / 9007199254740992.0 - 0.5) * 0.1;
+    }
+    std::fill(emu::g_die_barriers, emu::g_die_barriers + 8, 0ull);
+    const int rc = ggx_convolve_boxes(count, n.data(), off.data(), in.data(), out.data(), max_n, mode, dt, R, nullptr);
+    int bad = rc != GGX_OK;
+    double worst = 0.0;
+    for (int b = 0; b < count && !bad; ++b) {
+        ref.assign((size_t)n[b] * n[b], 0.0);
+        ggxo_convolve(n[b], mode, dt, R, in.data() + off[b], ref.data());
+        for (size_t k = 0; k < ref.size(); ++k) worst = std::max(worst, fabs(out[(size_t)off[b] + k] - ref[k]));
+    }
+    unsigned long long sum = 0, least = ~0ull;
+    for (unsigned long long v : emu::g_die_barriers) { sum += v; least = std::min(least, v); }
+    printf("rc %d, max|diff| %.3e, barriers %llu, of the idlest die %llu\n", rc, worst, sum, least);
+    if (!(worst <= 1e-12) || 16 * least < sum) bad++;
+    printf(bad ? "LIMITS FAILED\n" : "LIMITS OK\n");
+    return bad ? 1 : 0;
+}
+
 int main(int argc, char** argv) {
     setvbuf(stdout, nullptr, _IOLBF, 0);
     const char* what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "budget")) return budget_check(argc, argv);
+    if (!strcmp(what, "batch")) return batch_check(argc, argv);
     printf("unknown check %s\n", what);
     return 2;
 }

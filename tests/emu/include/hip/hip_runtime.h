@@ -63,6 +63,7 @@ inline dim3 g_tid, g_bid, g_bdim, g_gdim;
 inline std::function<void()>* g_body = nullptr;
 inline unsigned char* g_dyn = nullptr;
 inline size_t g_lds_most = 0;  // largest dynamic LDS of any launch so far
+inline unsigned long long g_die_barriers[8];  // workgroup barriers passed so far, by workgroup mod 8 (its die)
 constexpr size_t kStack = 256 * 1024;
 
 // Barriers: a workgroup barrier waits until every live lane of the block has arrived; a wave
@@ -147,6 +148,7 @@ inline void run_launch(dim3 grid, dim3 block, size_t shmem, std::function<void()
         std::memset(g_dyn, 0xCD, shmem ? shmem : 1);
         g_done = 0;
         g_bar_count = 0;
+        const unsigned gen = g_bar_gen;
         for (unsigned w = 0; w < 16; ++w) g_wave_count[w] = 0;
         for (unsigned t = 0; t < nt; ++t) {
             getcontext(&g_fibers[t].ctx);
@@ -167,6 +169,7 @@ inline void run_launch(dim3 grid, dim3 block, size_t shmem, std::function<void()
                 if (!g_fibers[t].done) any = true;
             }
         }
+        g_die_barriers[b & 7u] += g_bar_gen - gen;
     }
     g_body = nullptr;
 }

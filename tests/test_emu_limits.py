@@ -31,3 +31,12 @@ def limits():
 ])
 def test_lds_budget_is_kept_and_nothing_it_allowed_is_refused(limits, args):
     limits("budget " + args)
+
+
+@pytest.mark.parametrize("args", [
+    "64 3 16 128 2",    # one strip of eight there, more work items than workgroups
+    "100 1 40 64 0",
+    "20 5 16 256 1",    # one strip of sixteen, a workgroup per work item
+])
+def test_batch_spreads_over_the_dies_whatever_max_n(limits, args):
+    limits("batch " + args)
