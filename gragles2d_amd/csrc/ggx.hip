@@ -587,15 +587,43 @@ FftSymbol fft_symbol_of(const ggx_ctx* ctx) {
 // Workgroups of an FFT launch whose half spectra live in global slots (boxes above kFftLdsMax).
 constexpr int kFftWideGrid = 64;
 
+// Whether the half spectra of an FFT launch for boxes up to side nb stay in LDS.
+template <class T>
+bool fft_in_lds(const ggx_ctx* ctx, int nb) {
+    return nb <= kFftLdsMax && fft_lds<T>(nb, true) + ctx->static_fft[sizeof(T) == 8 ? 0 : 1][1] + 256 <= ctx->lds_max;
+}
+
+// Whether the strips of boxes up to side nb fit the LDS this context may use.
+template <class T>
+bool boxes_for(const ggx_ctx* ctx, int nb) { return sizeof(T) == 8 && box_columns_lds(nb) + 256 <= ctx->lds_max; }
+
+// Largest side of the buckets that share a launch of strips with a bucket of this edge.
+int strips_limit(int side) { return side <= 64 ? 64 : side <= 128 ? 128 : side <= 256 ? 256 : kMaxBox; }
+
+// Whether any launch of this context's steps runs the FFT (k_conv_fft), and with global slots.
+template <class T>
+void fft_needs(const ggx_ctx* ctx, bool* engine, bool* slots) {
+    *engine = *slots = false;
+    auto meet = [&](int nb, int strips_nb) {
+        if (!fft_for(ctx, nb) || boxes_for<T>(ctx, strips_nb)) return;
+        *engine = true;
+        if (!fft_in_lds<T>(ctx, nb)) *slots = true;
+    };
+    if (ctx->opt.batching == GGX_BATCH_PERGRAIN)
+        for (int n = 1; n <= kMaxBox; ++n) meet(n, n);
+    else
+        for (int b = 0; b < ctx->nbuckets; ++b) meet(ctx->edges[b], strips_limit(ctx->edges[b]));
+}
+
 template <class T>
 int launch_conv_fft(ggx_ctx* ctx, hipStream_t st, const int* list, const int* count, int nb, int grid,
                     const T* src, T* dst) {
     const int ti = sizeof(T) == 8 ? 0 : 1;
-    const bool in_lds = nb <= kFftLdsMax && fft_lds<T>(nb, true) + ctx->static_fft[ti][1] + 256 <= ctx->lds_max;
+    const bool in_lds = fft_in_lds<T>(ctx, nb);
     const long long lds = fft_lds<T>(nb, in_lds);
     if (lds + ctx->static_fft[ti][in_lds ? 1 : 0] + 256 > ctx->lds_max)
         return fail(ctx, GGX_E_BOUNDS, "box too large for the FFT line buffers: side " + std::to_string(nb));
-    if (!ctx->fft_work && !in_lds) return fail(ctx, GGX_E_STATE, "FFT workspace missing");
+    if (!ctx->tw || (!ctx->fft_work && !in_lds)) return fail(ctx, GGX_E_STATE, "FFT workspace missing");
     using C = typename Cplx<T>::type;
     if (in_lds) {
         if (grid <= 0) grid = ctx->cu_count * per_cu(ctx, lds + ctx->static_fft[ti][1]);
@@ -624,10 +652,6 @@ int launch_conv_boxes(ggx_ctx* ctx, hipStream_t st, const Items& it, int nb, int
     hipLaunchKernelGGL(k_box_rows<StepBoxes>, grid, block, rows, st, B, (const double*)dst, dst, 0);
     return GGX_OK;
 }
-
-// Whether the strips of boxes up to side nb fit the LDS this context may use.
-template <class T>
-bool boxes_for(const ggx_ctx* ctx, int nb) { return sizeof(T) == 8 && box_columns_lds(nb) + 256 <= ctx->lds_max; }
 
 // The circulant convolution of a launch's items, boxes up to side nb: the register tiles of 2, 3 or 4
 // times 16 columns, the LDS strip above 64 and where the tiles are above the context's lds_budget.
@@ -706,10 +730,7 @@ int launch_step(ggx_ctx* ctx, bool timed, bool record = false) {
         }
         bool strips = false;
         if (fft) {
-            auto limit = [&](int k) {  // strips of one launch share its LDS
-                const int side = ctx->edges[k];
-                return side <= 64 ? 64 : side <= 128 ? 128 : side <= 256 ? 256 : kMaxBox;
-            };
+            auto limit = [&](int k) { return strips_limit(ctx->edges[k]); };  // strips of one launch share its LDS
             strips = boxes_for<T>(ctx, limit(b));
             while (strips && e + 1 < ctx->nbuckets && fft_for(ctx, ctx->edges[e + 1]) && limit(e + 1) == limit(b)) ++e;
         }
@@ -1339,14 +1360,17 @@ extern "C" int ggx_load_network(ggx_ctx* ctx, const ggx_network* net) {
     }
     if ((rc = build_kernels(ctx))) return rc;
     {
-        // FFT engine tables: twiddles of every side up to kMaxBox (built on the device), and the
-        // global half-spectrum slots when the engine may meet boxes above kFftLdsMax
-        if ((rc = dalloc(ctx, ctx->tw, (size_t)tw_offset(kMaxBox + 1)))) return rc;
-        hipLaunchKernelGGL(k_fft_twiddles, dim3(kMaxBox), dim3(256), 0, ctx->stream, ctx->tw, 1, kMaxBox);
-        HIPCHK(hipGetLastError());
-        bool any_fft = false;
-        for (int b = 0; b < ctx->nbuckets; ++b) any_fft = any_fft || fft_for(ctx, ctx->edges[b]);
-        if (any_fft) {
+        // what the FFT engine reads, where a launch of this context runs it: twiddles of every side up
+        // to kMaxBox (built on the device), and the global half-spectrum slots
+        bool engine, slots;
+        if (es == 8) fft_needs<double>(ctx, &engine, &slots);
+        else fft_needs<float>(ctx, &engine, &slots);
+        if (engine) {
+            if ((rc = dalloc(ctx, ctx->tw, (size_t)tw_offset(kMaxBox + 1)))) return rc;
+            hipLaunchKernelGGL(k_fft_twiddles, dim3(kMaxBox), dim3(256), 0, ctx->stream, ctx->tw, 1, kMaxBox);
+            HIPCHK(hipGetLastError());
+        }
+        if (slots) {
             HIPCHK(hipMalloc(&p, (size_t)kFftWideGrid * (size_t)fft_slot(kMaxBox) * 2 * es + 256));
             ctx->fft_work = p;
         }

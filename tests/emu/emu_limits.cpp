@@ -1,9 +1,14 @@
 // The library's limits and its transform engine on the CPU (the fiber stand-in for the HIP runtime).
 // Test infrastructure.
-//   emu_limits budget <grains> <steps> <seed> <gb> <ppg> <fp32> <aniso> [lds_budget]
+//   emu_limits budget <grains> <steps> <seed> <gb> <ppg> <fp32> <aniso> [lds_budget] [ConvolutionMode]
 //     one-grain launches under lds_budget against the same run without one: same bits, no launch above
 //     the budget.  Without a budget given: the LDS that a grain's contour points (36 bytes each), its
-//     squares (one byte each up to side 128) and 480 bytes take, for the network's neediest grain.
+//     squares (one byte each up to side 128) and 480 bytes take, for the network's neediest grain.  With a
+//     Laplace mode, whose engine the budget decides, the fields may differ by rounding (1e-10).
+//   emu_limits engine
+//     k_conv_fft, every form, against the oracle's convolution.
+//   emu_limits workspace
+//     device memory of Laplace contexts against Gaussian ones: more only where the FFT runs.
 //   emu_limits batch <count> <lowest side> <highest side> <max_n> <mode>
 //     ggx_convolve_boxes against the oracle, with the work spread over the dies: none has less than half
 //     of the average (workgroup barriers, which only a workgroup with a strip meets).
@@ -19,6 +24,10 @@
 
 #include "ggx.h"
 #include "ggx_oracle.h"
+
+#define ggx ggx_engine  // the kernels once more, in a namespace of their own
+#include "fft.h"
+#undef ggx
 
 static ggx_ctx* make_run(ggx_network* net, int gb, int ppg, int fp32, int aniso, int cmode, int engine, int budget) {
     ggx_settings s;
@@ -53,12 +62,12 @@ static ggx_ctx* make_run(ggx_network* net, int gb, int ppg, int fp32, int aniso,
 
 static int budget_check(int argc, char** argv) {
     auto arg = [&](int k, int d) { return argc > k ? atoi(argv[k]) : d; };
-    const int N = arg(2, 6), steps = arg(3, 2), seed = arg(4, 1001), gb = arg(5, 7), ppg = arg(6, 20), fp32 = arg(7, 0), aniso = arg(8, 0);
+    const int N = arg(2, 6), steps = arg(3, 2), seed = arg(4, 1001), gb = arg(5, 7), ppg = arg(6, 20), fp32 = arg(7, 0), aniso = arg(8, 0), cmode = arg(10, 2);
     int budget = arg(9, 0);
     ggx_network* net = nullptr;
     if (ggx_network_generate(N, (unsigned long long)seed, 0.0, &net)) return 2;
     const int ng = ggx_network_count(net);
-    ggx_ctx* a = make_run(net, gb, ppg, fp32, aniso, 2, GGX_CONV_AUTO, 0);
+    ggx_ctx* a = make_run(net, gb, ppg, fp32, aniso, cmode, GGX_CONV_AUTO, 0);
     std::vector<std::vector<double>> phi;   // every grain's field after every step
     std::set<int> sides;
     std::vector<double> buf(1 << 20);
@@ -77,7 +86,7 @@ static int budget_check(int argc, char** argv) {
     if (budget == 0)
         for (int n : sides) budget = std::max(budget, (8 * n + 64) * 36 + (n <= 128 ? (n + 1) * (n + 1) : 0) + 480);
     printf("sides %d .. %d, budget %d\n", *sides.begin(), *sides.rbegin(), budget);
-    ggx_ctx* b = make_run(net, gb, ppg, fp32, aniso, 2, GGX_CONV_AUTO, budget);
+    ggx_ctx* b = make_run(net, gb, ppg, fp32, aniso, cmode, GGX_CONV_AUTO, budget);
     emu::g_lds_most = 0;
     int bad = 0;
     size_t at = 0;
@@ -86,7 +95,10 @@ static int budget_check(int argc, char** argv) {
         for (int g = 1; g <= ng; ++g, ++at) {
             const int c = ggx_get_phi(b, g, buf.data(), (int)buf.size());
             const std::vector<double>& want = phi[at];
-            if ((size_t)std::max(0, c) != want.size() || (c > 0 && memcmp(buf.data(), want.data(), want.size() * 8))) {
+            bool same = (size_t)std::max(0, c) == want.size();
+            for (size_t k = 0; same && k < want.size(); ++k)
+                same = cmode == 2 ? buf[k] == want[k] : fabs(buf[k] - want[k]) <= 1e-10;
+            if (!same) {
                 printf("step %d grain %d differs\n", t, g);
                 bad++;
             }
@@ -99,6 +111,98 @@ static int budget_check(int argc, char** argv) {
     ggx_network_free(net);
     printf(bad ? "LIMITS FAILED\n" : "LIMITS OK\n");
     return bad ? 1 : 0;
+}
+
+// One form of k_conv_fft over boxes of the given sides, random fields, every mode.  The bound: a stage of
+// prime p sums p products in a row, which leaves about sqrt(p) / 2 units of relative rounding in the mean
+// square, so four transforms leave 2 sqrt(sum of n's primes) of them; the table, the symbol and the two
+// stored halves add 4 primes' worth, eight standard deviations cover the largest of 10^5 values, and the
+// oracle's own rounding in FP64 doubles it.
+template <class T, bool LDS>
+static int engine_form(const char* name, const std::vector<int>& sides) {
+    using C = typename ggx_engine::Cplx<T>::type;
+    int nb = 1;
+    std::vector<int> list;
+    std::vector<ggx_engine::Box> box;
+    std::vector<long long> off;
+    long long total = 0;
+    for (int n : sides) {
+        list.push_back((int)list.size());
+        box.push_back(ggx_engine::Box{0, 0, n, 0});
+        off.push_back(total);
+        total += (long long)n * n;
+        nb = std::max(nb, n);
+    }
+    const int count = (int)sides.size(), grid = 3, R = 200;
+    const double dt = 2.2e-5, unit = sizeof(T) == 8 ? 2 * 0x1p-53 : 0x1p-24;
+    std::vector<T> src((size_t)total), dst((size_t)total);
+    unsigned long long x = 99;
+    for (auto& v : src) {
+        x = x * 6364136223846793005ULL + 1442695040888963407ULL;
+        v = (T)(((double)(x >> 11) / 9007199254740992.0 - 0.5) * 0.1);
+    }
+    std::vector<double2> tw((size_t)ggx_engine::tw_offset(nb + 1));
+    hipLaunchKernelGGL(ggx_engine::k_fft_twiddles, dim3(nb), dim3(256), 0, nullptr, tw.data(), 1, nb);
+    std::vector<C> work((size_t)grid * (size_t)ggx_engine::fft_slot(nb));
+    int bad = 0;
+    for (int mode = 0; mode <= 2; ++mode) {
+        ggx_engine::FftSymbol sy;
+        sy.mode = mode;
+        sy.dt = dt;
+        sy.nsq = (double)R * R;
+        std::fill(dst.begin(), dst.end(), (T)NAN);
+        hipLaunchKernelGGL((ggx_engine::k_conv_fft<T, LDS>), dim3(grid), dim3(256), (size_t)ggx_engine::fft_lds<T>(nb, LDS), nullptr,
+                           (const int*)list.data(), &count, (const ggx_engine::Box*)box.data(), (const long long*)off.data(),
+                           (const T*)src.data(), dst.data(), (const double2*)tw.data(), sy, nb, work.data());
+        for (int b = 0; b < count; ++b) {
+            const int n = sides[(size_t)b];
+            std::vector<double> in((size_t)n * n), ref((size_t)n * n);
+            double sq = 0, worst = 0;
+            for (size_t k = 0; k < in.size(); ++k) {
+                in[k] = (double)src[(size_t)off[(size_t)b] + k];
+                sq += in[k] * in[k];
+            }
+            ggxo_convolve(n, mode, dt, R, in.data(), ref.data());
+            bool finite = true;
+            for (size_t k = 0; k < in.size(); ++k) {
+                const double v = (double)dst[(size_t)off[(size_t)b] + k];
+                finite = finite && std::isfinite(v);
+                worst = std::max(worst, fabs(v - ref[k]));
+            }
+            int primes = 4;
+            for (int m = n, p = 2; m > 1; ++p)
+                while (m % p == 0) { primes += p; m /= p; }
+            const double bound = 8 * unit * 2 * sqrt((double)primes) * sqrt(sq / (double)in.size());
+            printf("%s mode %d n %d: max|diff| %.3e of %.3e\n", name, mode, n, worst, bound);
+            if (!finite || !(worst <= bound)) bad++;
+        }
+    }
+    return bad;
+}
+
+static int engine_check() {
+    const std::vector<int> lds = {1, 2, 3, 5, 16, 17, 31, 40, 64, 97, 127, 128}, wide = {3, 61, 129, 130, 200, 256};
+    int bad = engine_form<float, true>("FP32, LDS", lds) + engine_form<float, false>("FP32, slots", wide) +
+              engine_form<double, true>("FP64, LDS", lds) + engine_form<double, false>("FP64, slots", wide);
+    printf(bad ? "LIMITS FAILED\n" : "LIMITS OK\n");
+    return bad ? 1 : 0;
+}
+
+static int workspace_check() {
+    ggx_network* net = nullptr;
+    if (ggx_network_generate(6, 1001, 0.0, &net)) return 2;
+    auto bytes = [&](int fp32, int cmode, int engine) {
+        const size_t from = g_device_bytes;
+        ggx_destroy(make_run(net, 7, 20, fp32, 0, cmode, engine, 0));
+        return (long long)(g_device_bytes - from);
+    };
+    const long long plain64 = bytes(0, 2, GGX_CONV_AUTO), plain32 = bytes(1, 2, GGX_CONV_AUTO);
+    const long long more[] = {bytes(0, 0, GGX_CONV_AUTO) - plain64, bytes(0, 2, GGX_CONV_FFT) - plain64, bytes(1, 0, GGX_CONV_AUTO) - plain32};
+    printf("beyond the Gaussian's: FP64 Laplace %lld, FP64 forced %lld, FP32 Laplace %lld\n", more[0], more[1], more[2]);
+    const bool ok = more[0] == 0 && more[1] == 0 && more[2] > 0;
+    ggx_network_free(net);
+    printf(ok ? "LIMITS OK\n" : "LIMITS FAILED\n");
+    return ok ? 0 : 1;
 }
 
 static int batch_check(int argc, char** argv) {
@@ -140,6 +244,8 @@ int main(int argc, char** argv) {
     setvbuf(stdout, nullptr, _IOLBF, 0);
     const char* what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "budget")) return budget_check(argc, argv);
+    if (!strcmp(what, "engine")) return engine_check();
+    if (!strcmp(what, "workspace")) return workspace_check();
     if (!strcmp(what, "batch")) return batch_check(argc, argv);
     printf("unknown check %s\n", what);
     return 2;

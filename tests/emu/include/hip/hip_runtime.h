@@ -273,7 +273,9 @@ struct hipDeviceProp_t {
 inline const char* hipGetErrorString(hipError_t) { return "emu error"; }
 // device and pinned allocations come back filled with a junk pattern (as reused device memory
 // does), so a read of memory no kernel or copy has written shows up as a difference
+inline size_t g_device_bytes = 0;  // allocated by hipMalloc so far
 inline hipError_t hipMalloc(void** p, size_t n) {
+    g_device_bytes += n;
     *p = std::malloc(n ? n : 1);
     if (*p) std::memset(*p, 0xA5, n ? n : 1);
     return *p ? 0 : 2;

@@ -40,3 +40,7 @@ def test_lds_budget_is_kept_and_nothing_it_allowed_is_refused(limits, args):
 ])
 def test_batch_spreads_over_the_dies_whatever_max_n(limits, args):
     limits("batch " + args)
+
+
+def test_fft_workspace_is_there_only_where_the_fft_runs(limits):
+    limits("workspace")
