@@ -5,6 +5,9 @@
 //     the budget.  Without a budget given: the LDS that a grain's contour points (36 bytes each), its
 //     squares (one byte each up to side 128) and 480 bytes take, for the network's neediest grain.  With a
 //     Laplace mode, whose engine the budget decides, the fields may differ by rounding (1e-10).
+//   emu_limits corrector <grains> <steps> <seed> <gb> <ppg> <sigma> <model> <pergrain>
+//     an anisotropic run against the oracle (existence, boxes, fields to 1e-10) in which corrected grains
+//     had contours longer than the corrector stages in LDS.
 //   emu_limits engine
 //     k_conv_fft, every form, against the oracle's convolution.
 //   emu_limits workspace
@@ -26,6 +29,7 @@
 #include "ggx_oracle.h"
 
 #define ggx ggx_engine  // the kernels once more, in a namespace of their own
+#include "aniso.h"
 #include "fft.h"
 #undef ggx
 
@@ -108,6 +112,100 @@ static int budget_check(int argc, char** argv) {
     if (emu::g_lds_most > (size_t)budget) { printf("a launch is above the budget\n"); bad++; }
     ggx_destroy(a);
     ggx_destroy(b);
+    ggx_network_free(net);
+    printf(bad ? "LIMITS FAILED\n" : "LIMITS OK\n");
+    return bad ? 1 : 0;
+}
+
+static int corrector_check(int argc, char** argv) {
+    auto arg = [&](int k, double d) { return argc > k ? atof(argv[k]) : d; };
+    const int N = (int)arg(2, 6), steps = (int)arg(3, 3), gb = (int)arg(5, 9), ppg = (int)arg(6, 80), model = (int)arg(8, 1);
+    ggx_network* net = nullptr;
+    if (ggx_network_generate(N, (unsigned long long)arg(4, 15), arg(7, 0.0), &net)) return 2;
+    const int ng = ggx_network_count(net);
+    ggx_settings s;
+    ggx_settings_default(&s);
+    s.number_of_particles = ng;
+    s.number_of_points_per_grain = ppg;
+    s.number_of_timesteps = steps;
+    s.analysis_timestep = 1;
+    s.domain_border_size = gb;
+    s.microstructure_gen_mode = 0;
+    s.convolution_mode = 2;
+    s.is_isotropic_network = 0;
+    s.breakup_number = 0;
+    s.research_mode = 0;
+    s.use_mobility_model = model;
+    s.triple_point_drag = 0.5;
+    s.constant_sector_radius = 3;
+    s.interpolating_sector_radius = 2;
+    ggx_derived d;
+    ggx_settings_derive(&s, &d);
+    ggx_options o;
+    ggx_options_default(&o);
+    o.batching = arg(9, 0) != 0 ? GGX_BATCH_PERGRAIN : GGX_BATCH_FUSED;
+    double bins[16];
+    for (int b = 0; b < 16; ++b) bins[b] = 0.2 + 0.05 * b;
+    ggx_ctx* ctx = nullptr;
+    if (ggx_create(&s, &o, &ctx) || (model == 4 && ggx_set_mobility_bins(ctx, bins)) || ggx_load_network(ctx, net)) return 2;
+    ggxo_params p;
+    memset(&p, 0, sizeof p);
+    p.real_domain_size = d.real_domain_size;
+    p.grid_blowup = gb;
+    p.convolution_mode = 2;
+    p.dt = d.dt;
+    p.analysis_timestep = 1;
+    p.nthreads = 1;
+    p.number_of_particles = ng;
+    p.mobility_model = model;
+    p.triple_point_drag = 0.5;
+    p.constant_sector_radius = 3;
+    p.interpolating_sector_radius = 2;
+    for (int b = 0; b < 16; ++b) p.mobility_bins[b] = bins[b];
+    void* oc = nullptr;
+    ggxo_create(&p, ng, &oc);
+    for (int i = 0; i < ng; ++i) {
+        int id, nv;
+        const double *xy, *q;
+        ggx_network_grain(net, i, &id, &nv, &xy, &q);
+        ggxo_add_grain(oc, id, nv, xy, q);
+    }
+    ggxo_init(oc);
+    int bad = 0, longer = 0, shorter = 0;
+    std::vector<double> a(1 << 18), b(1 << 18);
+    for (int t = 0; t < steps; ++t) {
+        if (t > 0)  // the contours this step's corrector reads
+            for (int g = 1; g <= ng; ++g) {
+                ggx_grain_info i;
+                ggx_get_info(ctx, g, &i);
+                if (i.present && i.exists && i.motion_regular) (i.contour_len > ggx_engine::kAnisoContourLds ? longer : shorter)++;
+            }
+        if (ggx_step(ctx, 1) || ggx_sync(ctx)) { printf("step failed: %s\n", ggx_last_error(ctx)); return 3; }
+        ggxo_step(oc, t);
+        double worst = 0.0;
+        for (int g = 1; g <= ng; ++g) {
+            ggx_grain_info gi;
+            ggxo_grain_info oi;
+            ggx_get_info(ctx, g, &gi);
+            ggxo_get_info(oc, g, &oi);
+            const bool ge = gi.present && gi.exists, oe = oi.present && oi.exists;
+            if (ge != oe || (oe && (gi.xmin != oi.xmin || gi.xmax != oi.xmax || gi.ymin != oi.ymin || gi.ymax != oi.ymax))) {
+                printf("step %d grain %d: existence or box\n", t, g);
+                bad++;
+                continue;
+            }
+            if (!oe) continue;
+            const int c = ggx_get_phi(ctx, g, a.data(), (int)a.size());
+            if (c != ggxo_grain_phi(oc, g, b.data())) { bad++; continue; }
+            for (int k = 0; k < c; ++k) worst = std::max(worst, fabs(a[(size_t)k] - b[(size_t)k]));
+        }
+        printf("step %d: max|dphi| %.3e\n", t, worst);
+        if (!(worst <= 1e-10)) bad++;
+    }
+    printf("corrected grains: %d with longer contours, %d with shorter ones\n", longer, shorter);
+    if (!longer) bad++;
+    ggx_destroy(ctx);
+    ggxo_destroy(oc);
     ggx_network_free(net);
     printf(bad ? "LIMITS FAILED\n" : "LIMITS OK\n");
     return bad ? 1 : 0;
@@ -244,6 +342,7 @@ int main(int argc, char** argv) {
     setvbuf(stdout, nullptr, _IOLBF, 0);
     const char* what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "budget")) return budget_check(argc, argv);
+    if (!strcmp(what, "corrector")) return corrector_check(argc, argv);
     if (!strcmp(what, "engine")) return engine_check();
     if (!strcmp(what, "workspace")) return workspace_check();
     if (!strcmp(what, "batch")) return batch_check(argc, argv);
