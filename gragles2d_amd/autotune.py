@@ -1,5 +1,5 @@
 """Autotuner of the batched timestep: box-size bucket edges and, per bucket, the convolution
-engine (circulant or FFT), picked by timing the real step on the device.
+engine (circulant or GGX_CONV_FFT, which takes the strip products in FP64), picked by timing the real step on the device.
 
     python -m gragles2d_amd.autotune --workload batch-100k [--precision fp64] [--steps 5]
 

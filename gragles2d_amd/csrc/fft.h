@@ -271,15 +271,15 @@ __global__ void __launch_bounds__(256) k_conv_fft(const int* __restrict__ list, 
 // each in place on its strip, which lies in LDS.  H is not stored: its elements are read from the n
 // values cas(2 pi t / n) in LDS, the index j k mod n of a lane's next element by one addition.  An
 // FP64 product of 16 x 16 x 4 keeps a SIMD's matrix core for 64 cycles, in which the LDS has room
-// for far more than the two reads it needs.  6000 boxes of side 16 to 128 take 0.45, 0.9 and 0.45 ms
+// for far more than the two reads it needs.  6000 boxes of side 16 to 128 take 0.36, 0.74 and 0.37 ms
 // (products with the sides rounded up to 16: 0.12 ms each; the rest is each strip's chain of load,
-// table, product and store at 16 waves per CU), 96 of side 130 to 256 take 0.36 ms.  The FFT with a
-// workgroup per box took 7.5 ms, bound by its p-term sums, and 29 ms, bound by its eight half-spectrum
+// table, product and store at 16 waves per CU), 96 of side 130 to 256 take 0.33 ms.  The FFT with a
+// workgroup per box took 8.6 ms, bound by its p-term sums, and 25 ms, bound by its eight half-spectrum
 // slots.  The Richardson symbol's two 40th powers are a third of k_box_columns with pow().
 // In a step (k_box_rows and k_box_columns of FP64 networks with the FFT engine's symbols) the boxes
 // are the grains of a launch's work items.  There the FFT took 1.2 of 2.0 ms per step of a 5000-grain
 // Laplace network, up to 0.4 ms of it for the few widest boxes, one after the other's long sums in
-// one workgroup; the strips take 0.35 ms.
+// one workgroup; the strips take 0.42 ms, 0.06 of it in launches for sides that the network has few of.
 // ------------------------------------------------------------------------------------------
 struct BoxBatch {
     int count, strips;   // boxes; strips of 16 lines of the largest side allowed
@@ -329,7 +329,7 @@ __device__ __forceinline__ void strip_tiles(int n, const double* s_cas, const do
         }
     };
     // eight lines' products are summed by themselves before they join the total: rounding errors grow
-    // with the longer of the two chains (0.8 to 0.95 of the FFT's error; one chain: up to 2.7 times it)
+    // with the longer of the two chains (0.7 to 0.95 of the FFT's error; one chain: up to 2.7 times it)
     int k = 0;
     for (; k + 8 <= n; k += 8) {
         V acc[K];

@@ -57,8 +57,10 @@ __device__ __forceinline__ void wave_lds_sync() {
 // ------------------------------------------------------------------------------------------
 constexpr int kMaxBuckets = 16;
 // Networks up to this many grain ids are launch-latency bound (a launch lasts about as long as its
-// slowest grain): the corrector runs as one launch, and the level-set kernel as one launch for
-// every grain up to kMergeSide, the larger buckets keeping their own.
+// slowest grain): the scheduling runs in one workgroup, and the circulant convolution, contour and
+// redistancing as one launch for every grain up to kMergeSide, the larger buckets keeping their own.
+// Set below the break-even: a lognormal network takes 0.61 ms per step with 4000 grains and, launched
+// per bucket, 0.83 with 4200.
 constexpr int kSmallNetwork = 4096;
 constexpr int kMergeSide = 64;
 
@@ -494,13 +496,14 @@ __host__ __device__ inline long long ktab_len(int n) { return 2LL * n + 2 * kKPa
 // (read from global memory instead, a product's 16 row pieces take as long as the product), and the
 // coefficients of a step are 19 consecutive table entries.  Both kernels ask for two waves per SIMD or
 // more: within 256 registers the compiler keeps the accumulators in vector registers, else it moves
-// them to and from accumulation registers around every product (three times the time).
+// them to and from accumulation registers around every product (three times the time).  The strips of
+// sides above 256 hold too many for that in FP64: 496 bytes per lane lie in scratch there.
 //
 // On the 100k-grain network in FP64 (4 n flops and 16 bytes per point: floor 0.6 ms, the products at
 // the 77 TFLOP/s the matrix cores reach) this takes 1.2 ms per step, where register-blocked VALU
 // products with both tiles in LDS took 1.85 ms (five output blocks on four waves, 40 of 64 lanes
-// active).  The boxes of 130 to 190 points among 200 fine grains, whose tiles did not fit LDS before,
-// go from 1.7 to 0.05 ms.  What is left is the latency of reading and writing each box.
+// active).  Boxes of 70 to 300 points among 200 fine grains, most of whose tiles did not fit LDS before,
+// go from 1.7 to 0.1 ms.  What is left is the latency of reading and writing each box.
 // ------------------------------------------------------------------------------------------
 template <class T> struct Mma;
 template <> struct Mma<double> {
@@ -804,9 +807,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 // LSbox::extractContour (box.cpp:1089-1153) with MarchingSquaresAlgorithm::generateContour
 // (marchingSquares.cpp:28-188), isMotionRegular (box.cpp:1155-1190), clearContourGrainArea
 // (1883-1904), then computeVolumeAndEnergy (1201-1228) -> buildDirectNeighbours
-// (grainBoundary.cpp:85-199).  One workgroup per grain: the inside/outside test of the box is
-// kept as a bitmask in LDS so lane 0's trace never waits on memory for its direction; the
-// neighbour probes run on all lanes.
+// (grainBoundary.cpp:85-199).  What k_contour and k_alloc (level.h) leave per grain, and the cases and
+// directions of the marching squares.
 // ------------------------------------------------------------------------------------------
 struct ContourOut {
     double2* pts;             // contour arena

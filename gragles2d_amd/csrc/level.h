@@ -12,9 +12,9 @@
 //              (grainBoundary.cpp:85-199); one wave per grain up to side 64, four above
 //   k_alloc    room in the next field arena for every new box (one atomic per 256 grains)
 //   k_redist   LSbox::executeRedistancing (1259-1399); one line per lane, the new field in LDS
-// The kernels hand each other the compared field C (in the grain's slot of the input arena, whose
-// field is not read again in the step) and its signs as bit planes: per grain, rows and columns
-// of the tests C >= 0 and C > 0.  The contour's topology and the sweeps' signs come from the
+// The kernels hand each other the compared field C (in an arena of its own at the step's offsets: a
+// frame's copy may still be reading the input fields) and its signs as bit planes: per grain, rows and
+// columns of the tests C >= 0 and C > 0.  The contour's topology and the sweeps' signs come from the
 // bits; C itself is read at the zero crossings only.  On the 100k-grain lognormal network in FP64
 // (1.61e8 box points) the four take 2.2, 1.8, 0.01 and 2.1 ms per step; one kernel that did all of
 // it per grain, 256 lanes wide with C and the new field in LDS, took 11.8 ms: its serial phases
@@ -43,7 +43,7 @@ struct LevelArgs {
     const int* cmp_cnt;
     const int* cmp;
     const T* tilde;            // convolved fields (all grains)
-    T* cfield;                 // phi arena of this step: takes the compared fields
+    T* cfield;                 // takes the compared fields: an arena of their own (after a coarsening, the phi arena)
     unsigned long long* bits;  // sign planes, `plane` words each
     long long plane;
     const uint32_t* idl_old;
@@ -62,7 +62,7 @@ struct LevelArgs {
     unsigned long long* out_total;     // running sum of the new boxes' areas
     int nb;                    // largest box side of the launch
     int cap;                   // largest contour capacity of the launch
-    int blocks;                // k_compare: waves per grain, ceil(nb / 8) * ceil(nb / 64)
+    int blocks;                // k_compare: waves per grain; each loops over blocks of 8 rows x 64 columns
     int tile;                  // k_redist: largest new box side the LDS tile holds (0: no tile)
     AnisoConst K;              // anisotropic boundaries (K.on = 0: isotropic network)
     AnisoState AS;
@@ -1249,9 +1249,9 @@ __device__ __forceinline__ void sweep_line(OL oload, OS ostore, CL cload, int L,
     }
 }
 
-// LSbox::executeRedistancing (box.cpp:1259-1399) of one grain: Ob is the output tile (LDS with
-// an odd pitch, or the global slot itself), C the compared field on the old box b (row pitch
-// cp), bo the new box.  Lanes own columns (y sweeps) or rows (x sweeps); the value carried
+// LSbox::executeRedistancing (box.cpp:1259-1399) of one grain in place in the output arena, for what
+// does not fit k_redist's tile: Ob is the grain's slot (row pitch `pitch`), C the compared field on the
+// old box b (row pitch cp), bo the new box.  Lanes own columns (y sweeps) or rows (x sweeps); the value carried
 // along a sweep stays in a register and the next line's inputs are loaded one step ahead (a
 // sweep step only writes its own two lines, so the early loads see final values).
 template <class T>

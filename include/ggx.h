@@ -135,9 +135,10 @@ typedef struct ggx_ctx ggx_ctx;
 #define GGX_BATCH_FUSED    0  /* all grains per launch (the batched step) */
 #define GGX_BATCH_PERGRAIN 1  /* one launch per grain per kernel (the per-grain baseline) */
 
-#define GGX_CONV_AUTO      0  /* the engine chosen per box size (the FFT for ConvolutionMode 0 and 1) */
+#define GGX_CONV_AUTO      0  /* the engine chosen per box size (GGX_CONV_FFT for ConvolutionMode 0 and 1) */
 #define GGX_CONV_CIRCULANT 1  /* exact dense circulant, K_n phi K_n (real space; the separable Gaussian only) */
-#define GGX_CONV_FFT       2  /* batched mixed-radix FFT, any n, every ConvolutionMode */
+#define GGX_CONV_FFT       2  /* by transforms, any n, every ConvolutionMode: products with the real transform
+                                 matrix (FP64), mixed-radix FFT (FP32, or a small lds_budget) */
 
 typedef struct ggx_options {
     int32_t precision;        /* GGX_PREC_* */
@@ -314,7 +315,7 @@ typedef struct ggx_stats {
 int ggx_get_stats(ggx_ctx* ctx, ggx_stats* out);
 
 /* ---------------------------------------------------------------------------------------
- * Batched convolution without a context (the FFT engine on caller-owned device buffers).
+ * Batched convolution without a context, on caller-owned device buffers.
  * ------------------------------------------------------------------------------------- */
 
 /* Replaces LSbox::convolutionGeneratorFFTW (src/box.cpp:622-695) -- the FFTW r2c plan, the
@@ -323,10 +324,13 @@ int ggx_get_stats(ggx_ctx* ctx, ggx_stats* out);
  * (1 <= n[b] <= max_n <= 512) and is read from in + off[b] and written to out + off[b], row-major
  * n x n doubles (out[b] = IDFT2(G . DFT2(in[b])), G of ConvolutionMode `mode`: 0 Laplace,
  * 1 Laplace-Richardson, 2 Gaussian, with the time step dt and nsq = R^2 of the global grid,
- * box.cpp:636-691).  n, off, in and out are device pointers; in and out must not overlap.
+ * box.cpp:636-691).  n, off, in and out are device pointers; in and out must not overlap,
+ * and no two boxes of a batch may share elements of out (a box listed twice is not computed twice but
+ * spoiled: the passes work in place on out).
  * `stream` is a hipStream_t (NULL: the null stream).  The call allocates an error flag, runs on
- * `stream` (out holds intermediate values meanwhile), waits for it and frees the flag.  Returns GGX_OK, GGX_E_ARG, GGX_E_BOUNDS (max_n above 512, or a
- * side outside [1, max_n]: that box is left unwritten), GGX_E_OOM or GGX_E_HIP. */
+ * `stream` (out holds intermediate values meanwhile), waits for it and frees the flag.  Returns
+ * GGX_OK, GGX_E_ARG, GGX_E_BOUNDS (max_n above 512, or a side outside [1, max_n]: that box is left
+ * unwritten), GGX_E_OOM or GGX_E_HIP. */
 int ggx_convolve_boxes(int32_t count, const int32_t* n, const int64_t* off, const double* in, double* out,
                        int32_t max_n, int32_t mode, double dt, int32_t R, void* stream);
 
