@@ -387,7 +387,7 @@ __device__ __forceinline__ void set_bad(const BoxBatch& B) { *B.bad = 1; }
 __device__ __forceinline__ void set_bad(const StepBoxes&) {}
 
 // The box and strip of a work item; false: no such strip.  Box b's items take its strips from strip b on,
-// round and round: workgroup i runs on die i mod 8, so with strip = item mod strips the strips of one
+// wrapping at the last: workgroup i runs on die i mod 8, so with strip = item mod strips the strips of one
 // place in a box, and the empty ones beyond it where max_n is far above the sides, all fell to the same
 // dies.  6000 boxes of side 16 to 32 called with max_n 512: 5.2 -> 1.04 ms (two of eight dies had the work;
 // the rest is one workgroup of 147 KB per CU); 96 of side 130 to 256 0.355 -> 0.331.
