@@ -5,6 +5,6 @@ import pytest
 from .test_emu_limits import limits  # noqa: F401
 
 
-@pytest.mark.parametrize("args", ["4 2 11 9 110 0 1 0", "6 2 15 9 80 0.3 1 0", "5 2 14 9 90 0 4 1"])
+@pytest.mark.parametrize("args", ["6 2 15 9 80 0.3 1 0", "5 2 14 9 90 0 4 1"])
 def test_corrector_on_long_contours(limits, args):  # noqa: F811
     limits("corrector " + args)

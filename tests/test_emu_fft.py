@@ -19,11 +19,11 @@ def test_fp64_steps_whose_strips_are_above_the_budget(limits, cmode):  # noqa: F
     limits(f"budget 6 2 1001 7 20 0 0 16000 {cmode}")
 
 
-@pytest.mark.parametrize("net,engine,cmode", [
-    ("6 2 1001 7 20", 0, 0), ("6 2 1001 7 20", 0, 1), ("6 2 1001 7 20", 2, 2),  # half spectra in LDS
-    ("6 2 3 40 60", 0, 0),                                                       # sides 150-226: global slots
+@pytest.mark.parametrize("net,engine,cmode,pergrain", [
+    ("6 2 1001 7 20", 0, 0, 0), ("6 2 1001 7 20", 0, 1, 0), ("6 2 1001 7 20", 2, 2, 0),  # half spectra in LDS
+    ("6 2 1001 7 20", 0, 0, 1), ("6 2 1001 7 20", 2, 2, 1),
+    ("6 2 3 40 60", 0, 0, 0),                                                             # sides 150-226: global slots
 ])
-@pytest.mark.parametrize("pergrain", [0, 1])
 def test_fp32_steps(limits, net, engine, cmode, pergrain):  # noqa: F811
     # everything discrete that the FP32 run is held to, and the areas: within 1e-5 of the oracle's
     r = subprocess.run([os.path.join(EMU, "emu_parity")] + f"{net} 0.0 1 {pergrain} 0.0 1 {engine} {cmode}".split(),

@@ -27,7 +27,7 @@ def limits():
     "6 2 1001 7 20 1",        # FP32
     "6 2 1001 7 20 1 0 20000",
     "6 2 1001 7 20 0 1",      # anisotropic
-    "3 1 1024 20 128 0",      # sides above 128: the strips
+    "2 1 7 9 90 0",           # sides 142 and 145 under 44.5 KB: the strips
 ])
 def test_lds_budget_is_kept_and_nothing_it_allowed_is_refused(limits, args):
     limits("budget " + args)
